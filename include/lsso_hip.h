@@ -404,6 +404,33 @@ int lsso_hip_layer_forward_train(const lsso_hip_mixer_shape* shape,
                                  size_t workspace_bytes,
                                  void* stream);
 
+/* Types of the position ids of lsso_hip_center_positions. */
+#define LSSO_HIP_IDS_NONE 0 /* 0 .. length - 1 */
+#define LSSO_HIP_IDS_I32 1
+#define LSSO_HIP_IDS_I64 2
+#define LSSO_HIP_IDS_F32 3
+#define LSSO_HIP_IDS_F64 4
+
+/* Longest row lsso_hip_center_positions takes (one workgroup walks it). */
+#define LSSO_HIP_CENTER_MAX_LENGTH 65536
+
+/* Centred positions and valid counts of the mixer, in one launch.
+ * valid_mask: uint8 [rows, length] contiguous or NULL (all valid).
+ * position_ids: device array of position_type read at row *
+ * position_batch_stride + token * position_token_stride (elements), or NULL
+ * with LSSO_HIP_IDS_NONE.  centered_positions: float32 [rows, length] =
+ * id - (first valid id) - mean over the valid tokens, 0 at excluded tokens;
+ * differences are taken in the ids' own type, the mean and its subtraction in
+ * FP64 for FP64 ids, else in FP32 from an FP64 sum.  valid_counts: float32
+ * [rows], the valid tokens of each row and at least 1 (required with
+ * valid_mask, else unused).
+ * Replaces: LSSO._center_positions and the valid counts
+ * (lsso/ball/model.py:163-243, 364-370). */
+int lsso_hip_center_positions(const uint8_t* valid_mask, const void* position_ids,
+                              int position_type, int64_t position_batch_stride,
+                              int64_t position_token_stride, int64_t rows, int64_t length,
+                              float* centered_positions, float* valid_counts, void* stream);
+
 /* Device scratch bytes needed by lsso_hip_linear. */
 int lsso_hip_linear_workspace_bytes(int64_t rows, int64_t in_features,
                                     int64_t out_features, size_t* bytes);

@@ -34,12 +34,15 @@ _BF16 = 2
 _POSITIONS_DEFAULT = 0
 _POSITIONS_SHARED = 1
 _POSITIONS_BATCHED = 2
+_CENTER_MAX_LENGTH = 65536
+_ID_TYPES = {torch.int32: 1, torch.int64: 2, torch.float32: 3, torch.float64: 4}
 
 _SYMBOLS = (
     "lsso_hip_contract_version",
     "lsso_hip_target",
     "lsso_hip_last_error",
     "lsso_hip_mixer_validate",
+    "lsso_hip_center_positions",
     "lsso_hip_mixer_workspace_bytes",
     "lsso_hip_mixer_tape_floats",
     "lsso_hip_mixer_forward",
@@ -89,6 +92,10 @@ def _declare(library: ctypes.CDLL) -> None:
     library.lsso_hip_last_error.argtypes = []
     library.lsso_hip_mixer_validate.restype = ctypes.c_int
     library.lsso_hip_mixer_validate.argtypes = [shape_p, ctypes.c_int]
+    library.lsso_hip_center_positions.restype = ctypes.c_int
+    library.lsso_hip_center_positions.argtypes = [
+        vp, vp, ctypes.c_int, i64, i64, i64, i64, vp, vp, vp,
+    ]  # valid_mask, position_ids, type, batch stride, token stride, rows, length, centered, counts, stream
     library.lsso_hip_mixer_workspace_bytes.restype = ctypes.c_int
     library.lsso_hip_mixer_workspace_bytes.argtypes = [shape_p, ctypes.c_int, size_p]
     library.lsso_hip_mixer_tape_floats.restype = ctypes.c_int
@@ -425,6 +432,55 @@ def _validate_core(
         if valid_counts.dim() != 1 or valid_counts.shape[0] != batch:
             raise RuntimeError(f"valid_counts must have shape [B], got {tuple(valid_counts.shape)}")
     return MixerShape(batch, length, heads, rank, head_dim), mode
+
+
+def center_positions(
+    position_ids: torch.Tensor | None,
+    valid_mask: torch.Tensor | None,
+    batch: int,
+    length: int,
+    device: torch.device,
+) -> tuple[torch.Tensor, torch.Tensor | None] | None:
+    """(centered positions, valid counts) of a masked or explicitly positioned
+    batch in one native launch: float32 [N] for ids shared by all samples
+    without a mask, else [B, N]; counts float32 [B] with a mask, else None.
+    The values of LSSO._center_positions (reference model.py:163-243), the
+    mean from an FP64 sum.
+
+    None where the kernel does not apply: rows longer than
+    ``_CENTER_MAX_LENGTH`` (one workgroup walks a row), and ids of another
+    type, shape or device, which the tensor path converts or rejects."""
+
+    if length > _CENTER_MAX_LENGTH or (position_ids is None and valid_mask is None):
+        return None
+    rows, kind, ids, batch_stride, token_stride = batch, 0, None, 0, 0
+    if position_ids is not None:
+        kind = _ID_TYPES.get(position_ids.dtype, 0)
+        if kind == 0 or position_ids.device != device:
+            return None
+        if position_ids.dim() == 1 and position_ids.shape[0] == length:
+            token_stride = position_ids.stride(0)
+            rows = 1 if valid_mask is None else batch
+        elif position_ids.dim() == 2 and position_ids.shape == (batch, length):
+            batch_stride, token_stride = position_ids.stride()
+        else:
+            return None
+        ids = position_ids.data_ptr()
+    counts = mask_ptr = None
+    if valid_mask is not None:
+        valid_mask = valid_mask.contiguous()
+        mask_ptr = valid_mask.data_ptr()
+        counts = torch.empty(batch, dtype=torch.float32, device=device)
+    shared = rows == 1 and valid_mask is None and position_ids.dim() == 1
+    centered = torch.empty((length,) if shared else (batch, length), dtype=torch.float32, device=device)
+    library = _library()
+    with torch.cuda.device(device):
+        status = library.lsso_hip_center_positions(
+            mask_ptr, ids, kind, batch_stride, token_stride, rows, length, centered.data_ptr(),
+            None if counts is None else counts.data_ptr(), _stream(device),
+        )
+    _check(status, library)
+    return centered, counts
 
 
 def _mixer_forward(
@@ -1477,6 +1533,7 @@ def linear(
 
 __all__ = [
     "backward",
+    "center_positions",
     "fast_mix",
     "forward_inference",
     "forward_train",

@@ -390,21 +390,25 @@ class LSSO(nn.Module):
             if all_valid
             else self._validate_mask(valid_mask, batch=batch, length=length, device=x.device)
         )
-        centered_positions = None
-        if valid_mask is not None or position_ids is not None:
-            centered = self._center_positions(
-                position_ids,
-                mask,
-                dtype=torch.float32,
-                all_valid=all_valid,
-                batch=batch,
-                length=length,
-                device=x.device,
-            )
-            if position_ids is None or position_ids.ndim == 1:
-                centered_positions = centered[0].contiguous() if all_valid else centered.contiguous()
-            else:
-                centered_positions = centered.contiguous()
+        if valid_mask is None and position_ids is None:
+            return None, None, None
+
+        from . import hip
+
+        native = hip.center_positions(position_ids, mask, batch, length, x.device)
+        if native is not None:
+            return (*native, mask)
+        centered = self._center_positions(
+            position_ids,
+            mask,
+            dtype=torch.float32,
+            all_valid=all_valid,
+            batch=batch,
+            length=length,
+            device=x.device,
+        )
+        shared = all_valid and position_ids.ndim == 1
+        centered_positions = (centered[0] if shared else centered).contiguous()
         valid_counts = (
             None
             if all_valid

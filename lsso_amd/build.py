@@ -26,6 +26,7 @@ OFFLOAD_ARCH = "gfx950"
 LIBRARY_NAME = f"liblsso_hip_{OFFLOAD_ARCH}.so"
 SOURCES = (
     "lsso_capi.hip",
+    "lsso_geometry.hip",
     "lsso_mixer.hip",
     "lsso_linear.hip",
     "lsso_linear_grad.hip",

@@ -203,6 +203,40 @@ int lsso_hip_mixer_tape_floats(const lsso_hip_mixer_shape* shape, size_t* floats
     return LSSO_HIP_OK;
 }
 
+int lsso_hip_center_positions(const uint8_t* valid_mask, const void* position_ids,
+                              int position_type, int64_t position_batch_stride,
+                              int64_t position_token_stride, int64_t rows, int64_t length,
+                              float* centered_positions, float* valid_counts, void* stream) {
+    if (rows <= 0 || length <= 0) {
+        return fail(LSSO_HIP_EINVAL, "rows and length must be positive");
+    }
+    if (length > LSSO_HIP_CENTER_MAX_LENGTH || rows > INT32_MAX) {
+        return fail(LSSO_HIP_EUNSUPPORTED, "center_positions takes rows of up to " +
+                                               std::to_string(LSSO_HIP_CENTER_MAX_LENGTH) + " tokens");
+    }
+    if (position_type < LSSO_HIP_IDS_NONE || position_type > LSSO_HIP_IDS_F64) {
+        return fail(LSSO_HIP_EINVAL, "position_type must be one of LSSO_HIP_IDS_*");
+    }
+    if ((position_ids == nullptr) != (position_type == LSSO_HIP_IDS_NONE)) {
+        return fail(LSSO_HIP_EINVAL, "position_ids must be NULL exactly with LSSO_HIP_IDS_NONE");
+    }
+    if (centered_positions == nullptr || (valid_mask != nullptr && valid_counts == nullptr)) {
+        return fail(LSSO_HIP_EINVAL, "centered_positions (and valid_counts with a mask) must not be NULL");
+    }
+    lsso_hip::GeometryArgs args{};
+    args.mask = valid_mask;
+    args.positions = position_ids;
+    args.position_batch_stride = position_batch_stride;
+    args.position_token_stride = position_token_stride;
+    args.rows = rows;
+    args.length = length;
+    args.centered = centered_positions;
+    args.counts = valid_counts;
+    const hipError_t error =
+        lsso_hip::launch_geometry(args, position_type, static_cast<hipStream_t>(stream));
+    return error == hipSuccess ? LSSO_HIP_OK : hip_failure(error, "geometry_kernel launch");
+}
+
 }  // extern "C"
 
 namespace {

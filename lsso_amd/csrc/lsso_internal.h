@@ -43,6 +43,18 @@ struct PhaseArgs {
     float inverse_frequency[kMaxPairs];
 };
 
+// Centred positions and valid counts from a mask and position ids.
+struct GeometryArgs {
+    const uint8_t* mask;        // [rows, length] or nullptr
+    const void* positions;      // ids, or nullptr (0 .. length - 1)
+    int64_t position_batch_stride;
+    int64_t position_token_stride;
+    int64_t rows;               // samples, or 1 (one grid shared by all samples)
+    int64_t length;
+    float* centered;            // [rows, length]
+    float* counts;              // [rows] (written when mask is set)
+};
+
 struct ReduceArgs {
     const uint16_t* projected;  // BF16 [B, N, width] (relation columns)
     const uint16_t* content;    // BF16 rows whose head-h columns are contracted with A
@@ -268,6 +280,7 @@ struct WeightGradArgs {
 };
 
 hipError_t launch_phase(const PhaseArgs& a, hipStream_t stream);
+hipError_t launch_geometry(const GeometryArgs& a, int position_type, hipStream_t stream);
 hipError_t launch_reduce(int rank, const ReduceArgs& a, int cpw, bool vec, hipStream_t stream);
 // Heads per workgroup of the staged reduce for this geometry, or 0 where it
 // does not apply (the one-wave-per-item reduce_kernel runs instead).
