@@ -1217,8 +1217,6 @@ int lsso_hip_linear_weight_grad(const void* g, int g_dtype, int64_t g_row_stride
     args.bias_partials = grad_bias != nullptr ? bias_partials : nullptr;
     args.rows_per_split = plan.rows_per_split;
     args.splits = plan.splits;
-    args.tiles_n = ceil_div(out_features, lsso_hip::weight_grad_tile());
-    args.tiles_k = ceil_div(in_features, lsso_hip::weight_grad_tile());
     args.vec = (out_features % 8 == 0 && in_features % 8 == 0 && g_row_stride % 8 == 0 &&
                 x_row_stride % 8 == 0 && aligned(g, 16) && aligned(x, 16)) ? 1 : 0;
     hipError_t error = lsso_hip::launch_weight_grad(args, g_dtype, x_dtype, stream);

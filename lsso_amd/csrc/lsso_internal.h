@@ -274,9 +274,11 @@ struct WeightGradArgs {
     float* bias_partials;       // [splits, out_features] or nullptr
     int64_t rows_per_split;     // multiple of 32
     int64_t splits;
-    int64_t tiles_n;
+    int64_t tiles_n;            // output tiles (set by the launcher)
     int64_t tiles_k;
     int vec;                    // 16-byte loads of g and x are legal
+    int dealt;                  // row splits are dealt to the XCDs (set by the launcher)
+    int large;                  // 256 x 256 output tiles, else 128 x 128 (set by the launcher)
 };
 
 hipError_t launch_phase(const PhaseArgs& a, hipStream_t stream);
@@ -331,7 +333,6 @@ hipError_t launch_grad_columns(const GradColumnsArgs& a, int g_dtype, bool vec, 
                                int64_t slabs, float* column_sums, hipStream_t stream);
 void plan_weight_grad(int64_t rows, int64_t in_features, int64_t out_features, int64_t* splits,
                       int64_t* rows_per_split);
-int weight_grad_tile();
 hipError_t launch_weight_grad(const WeightGradArgs& a, int g_dtype, int x_dtype, hipStream_t stream);
 int linear_tile_rows(int k_steps);
 int linear_columns_per_group(int k_steps);

@@ -130,53 +130,105 @@ __global__ __launch_bounds__(kGradThreads) void grad_columns_kernel(GradColumnsA
     }
 }
 
-// out[c] = sum over splits s of partials[s][c]: 32 columns x 8 split lanes
-// per workgroup; split lane l adds splits l, l + 8, ... in order (sixteen
-// loads in flight), then the lanes are added in lane order.  One launch can
-// serve two such sums over the same splits (a weight gradient and its bias):
-// the first `blocks` workgroups take the first, the rest the second.
-__global__ __launch_bounds__(kGradThreads) void column_sum_kernel(const float* partials, int64_t splits,
-                                                                  int64_t cols, float* out,
-                                                                  const float* partials2, int64_t cols2,
-                                                                  float* out2, int64_t blocks) {
-    constexpr int kLanes = kGradThreads / 32;
-    constexpr int kLoads = 16;
-    const int c = threadIdx.x & 31;
-    const int lane = threadIdx.x >> 5;
+// out[c] = sum over splits s of partials[s][c], in a fixed order: a thread
+// takes one piece (four columns, one 16-byte load; one column where the rows
+// are not whole pieces) of every `lanes`-th split with eight loads in flight,
+// then the lanes of a piece are added in lane order.  The lanes per piece (a
+// power of two up to 32) are the fewest that give the device its threads:
+// few columns over many splits need many lanes, and a wide weight over eight
+// splits needs one (with eight fixed lanes of sixteen loads each, 1,344 x
+// 768 columns over 8 splits ran at 1 TB/s).  One launch can serve two such
+// sums over the same splits (a weight gradient and its bias): the first
+// `blocks` workgroups take the first, the rest the second.
+constexpr int kSumLoads = 8;
+constexpr int kSumMaxLanes = 32;
+constexpr int64_t kSumThreads = 256 * 512;   // threads that keep the memory busy: two per SIMD lane
+
+struct ColumnSum {
+    const float* partials;
+    int64_t cols;
+    float* out;
+    int lanes;
+};
+
+template <int V>
+struct SumPiece {
+    float v[V];
+};
+template <int V>
+__device__ __forceinline__ SumPiece<V> load_sum_piece(const float* at) {
+    SumPiece<V> p;
+    if constexpr (V == 4) {
+        const f32x4 raw = *reinterpret_cast<const f32x4*>(at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            p.v[e] = raw[e];
+        }
+    } else {
+        p.v[0] = *at;
+    }
+    return p;
+}
+
+template <int V>
+__global__ __launch_bounds__(kGradThreads) void column_sum_kernel(ColumnSum first, ColumnSum second, int64_t splits,
+                                                                  int64_t blocks) {
+    __shared__ float s_acc[kGradThreads][V];
     int64_t block = blockIdx.x;
+    ColumnSum a = first;
     if (block >= blocks) {   // uniform over the workgroup
         block -= blocks;
-        partials = partials2;
-        cols = cols2;
-        out = out2;
+        a = second;
     }
-    const int64_t column = block * 32 + c;
-    const int64_t safe_column = column < cols ? column : 0;
-    float acc = 0.0f;
-    for (int64_t s0 = lane; s0 < splits; s0 += kLanes * kLoads) {
-        float v[kLoads];
+    const int pieces = kGradThreads / a.lanes;   // of this workgroup
+    const int piece = threadIdx.x % pieces;
+    const int lane = threadIdx.x / pieces;
+    const int64_t column = (block * pieces + piece) * V;
+    const bool live = column < a.cols;
+    const float* base = a.partials + (live ? column : 0);
+    float acc[V];
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u) {
-            const int64_t s = s0 + static_cast<int64_t>(u) * kLanes;
-            v[u] = partials[(s < splits ? s : 0) * cols + safe_column];
+    for (int e = 0; e < V; ++e) {
+        acc[e] = 0.0f;
+    }
+    for (int64_t s0 = lane; s0 < splits; s0 += a.lanes * kSumLoads) {
+        SumPiece<V> v[kSumLoads];
+#pragma unroll
+        for (int u = 0; u < kSumLoads; ++u) {
+            const int64_t s = s0 + u * a.lanes;
+            v[u] = load_sum_piece<V>(base + (s < splits ? s : s0) * a.cols);
         }
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u) {
-            if (s0 + static_cast<int64_t>(u) * kLanes < splits) {
-                acc += v[u];
+        for (int u = 0; u < kSumLoads; ++u) {
+            if (s0 + u * a.lanes < splits) {
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    acc[e] += v[u].v[e];
+                }
             }
         }
     }
-    __shared__ float s_acc[kLanes][32];
-    s_acc[lane][c] = acc;
-    __syncthreads();
-    if (lane == 0 && column < cols) {
-        float total = 0.0f;
+    if (a.lanes > 1) {   // uniform
 #pragma unroll
-        for (int l = 0; l < kLanes; ++l) {
-            total += s_acc[l][c];
+        for (int e = 0; e < V; ++e) {
+            s_acc[threadIdx.x][e] = acc[e];
         }
-        out[column] = total;
+        __syncthreads();
+        if (lane != 0) {
+            return;
+        }
+        for (int l = 1; l < a.lanes; ++l) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                acc[e] += s_acc[l * pieces + piece][e];
+            }
+        }
+    }
+    if (live) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            a.out[column + e] = acc[e];
+        }
     }
 }
 
@@ -187,11 +239,30 @@ hipError_t launch_column_sum(const float* partials, int64_t splits, int64_t cols
 
 hipError_t launch_column_sums(const float* partials, int64_t cols, float* out, const float* partials2,
                               int64_t cols2, float* out2, int64_t splits, hipStream_t stream) {
-    const int64_t blocks = (cols + 31) / 32;
-    const int64_t blocks2 = (cols2 + 31) / 32;
+    const auto whole = [](const float* base, int64_t n) {
+        return n % 4 == 0 && reinterpret_cast<uintptr_t>(base) % 16 == 0;
+    };
+    const int v = whole(partials, cols) && (cols2 == 0 || whole(partials2, cols2)) ? 4 : 1;
+    const auto plan = [&](const float* base, int64_t n, float* to, int64_t* blocks) {
+        const int64_t pieces = (n + v - 1) / v;
+        int lanes = 1;
+        while (lanes < kSumMaxLanes && lanes < splits && pieces * lanes < kSumThreads) {
+            lanes *= 2;
+        }
+        const int64_t per_block = kGradThreads / lanes;
+        *blocks = (pieces + per_block - 1) / per_block;
+        return ColumnSum{base, n, to, lanes};
+    };
+    int64_t blocks = 0;
+    int64_t blocks2 = 0;
+    const ColumnSum first = plan(partials, cols, out, &blocks);
+    const ColumnSum second = plan(partials2, cols2, out2, &blocks2);
     const dim3 grid(static_cast<unsigned>(blocks + blocks2));
-    column_sum_kernel<<<grid, kGradThreads, 0, stream>>>(partials, splits, cols, out, partials2, cols2, out2,
-                                                         blocks);
+    if (v == 4) {
+        column_sum_kernel<4><<<grid, kGradThreads, 0, stream>>>(first, second, splits, blocks);
+    } else {
+        column_sum_kernel<1><<<grid, kGradThreads, 0, stream>>>(first, second, splits, blocks);
+    }
     return hipGetLastError();
 }
 

@@ -5,46 +5,81 @@
 // with rows that the row mask excludes counting as zero.
 //
 // The contraction runs over rows, the strided dimension of both row-major
-// operands, while an MFMA fragment needs 8 consecutive rows of one column.
-// Each workgroup (four waves) owns a 128 (n) x 128 (k) output tile and a
-// split of consecutive rows, taken in 64-row stages.  Per stage, each thread
-// loads one 8-row x 8-column block of g (waves 0-1) or x (waves 2-3) as eight
-// 16-byte row pieces, one stage ahead of its use; rounds it to BF16 (the
-// reference's operands); transposes it in registers (byte permutes); and
-// writes its 8 columns to LDS column-major, so that every MFMA fragment
-// (v_mfma_f32_32x32x16_bf16, A = g^T, B = x, K = rows) is one 16-byte LDS
-// read.  Each wave accumulates a 64 x 64 quarter of the tile.  A split writes
-// FP32 partials [split][n][k]; column_sum_kernel adds the splits in order, so
-// the result is deterministic.  The bias sums are taken from the g blocks (in
-// g's own precision, as the reference sums g) by the k-tile-0 workgroups.
-// The workgroups of one row split are dealt to one XCD, so that the re-reads
-// of g and x by the neighbouring tiles hit that XCD's L2.
+// operands, while an MFMA fragment needs 8 rows of one column.  The operands
+// stay row-major in LDS, as they come from HBM, and ds_read_b64_tr_b16 turns
+// them on the way into registers: 16 lanes read 4 rows x 16 columns and lane
+// i receives its column's 4 rows, so two such reads are one fragment of
+// v_mfma_f32_32x32x16_bf16 (A = g^T, B = x, K = rows).
+//
+// Bound: HBM (g and x once) plus the FP32 partials; at 262,144 x (512, 256)
+// that is 403 MB and 2 x 67 MB.  What sets the form is how often the operands
+// pass from L2 to the CUs, how many loads are in flight, and how much of the
+// conversion work hides under the MFMAs:
+// - A workgroup of eight waves owns a 256 (n) x 256 (k) output tile (128
+//   accumulation registers per wave) of a large product, so g is read K / 256
+//   times and x N / 256 times; a small product takes 128 x 128 tiles.
+// - 32-row stages, each thread moving 16-byte pieces; two stages of loads are
+//   in flight in registers while a third is multiplied from LDS (two
+//   buffers).  FP16 operands are rounded to BF16 (the reference's operands)
+//   between the registers and LDS.
+// - A stage is one basic block in which the next stage's conversions and LDS
+//   writes are scheduled between the MFMAs: the two waves of a SIMD run in
+//   step, so work not interleaved within a wave does not overlap at all
+//   (126 us with the conversions before the products, 101 between them).
+// - The LDS pitch of 32 bf16 past the tile puts the 4 rows that a half wave
+//   reads on disjoint quarters of the 64 banks.
+// The former kernel (128 x 128 tiles of four waves, 8 x 8 blocks transposed in
+// registers with byte permutes, one stage in flight) took, with the column
+// sums, 181 us at 262,144 x (512, 256), 96 at 262,144 x (256, 256), 112 at
+// 131,072 x (640, 256) and 98 at 8,192 x (1,344, 768); this one 116, 73, 85
+// and 44 (4.6-5.7 TB/s of operands and partials at the first two).
+//
+// A split writes FP32 partials [split][n][k]; column_sum_kernel adds the
+// splits in a fixed order, so the result is deterministic.  The bias sums are
+// taken from the g pieces (in g's own precision, as the reference sums g) by
+// the k-tile-0 workgroups.  The workgroups of one row split are dealt to one
+// XCD, so that the re-reads of g and x by the neighbouring tiles hit that
+// XCD's L2.
 
 #include "lsso_device.h"
 #include "lsso_internal.h"
 #include "lsso_hip.h"
 
+#include <algorithm>
+#include <cmath>
+
 namespace lsso_hip {
 
 namespace {
 
-constexpr int kWgTile = 128;            // output tile edge (n and k)
-constexpr int kWgRows = 64;             // rows per stage (four MFMA K steps)
-constexpr int kWgThreads = 256;
-constexpr int kWgPitch = kWgRows + 8;   // column-major LDS pitch (bf16)
+constexpr int kWgRows = 32;             // rows per stage (two MFMA K steps)
+constexpr int kWgSteps = kWgRows / 16;
+constexpr int kWgThreads = 512;         // eight waves: four along n, two along k
 
-// LDS offset (bf16) of rows 8 g .. 8 g + 7 of a stage column.  The 8-row
-// group index is XOR-swizzled by bits 4-6 of the column, so that both the
-// transposed block writes (16 lanes: 16 columns 8 apart, one row group) and
-// the fragment reads (consecutive columns, one row group) spread over all
-// LDS banks; with the plain layout, columns 8 apart land on two bank groups.
-__device__ __forceinline__ int stage_offset(int column, int group) {
-    return column * kWgPitch + 8 * (group ^ ((column >> 4) & 7));
-}
+// Output tile of a workgroup: NB x KB blocks of 32 x 32 per wave.
+template <int NB>
+struct WgTile {
+    static constexpr int kNB = NB;
+    static constexpr int kKB = 2 * NB;
+    static constexpr int kEdge = 4 * 32 * NB;            // n and k
+    static constexpr int kPitch = kEdge + 32;            // row-major LDS pitch (bf16): 64 bytes past a multiple of 256
+    static constexpr int kPieces = kEdge / 8;            // 16-byte pieces per row
+    static constexpr int kRowLanes = kWgThreads / kPieces;
+    static constexpr int kPasses = kWgRows / kRowLanes;  // pieces per thread, operand and stage
+    static constexpr int kSlotsPerXcd = 32 * (NB == 1 ? 2 : 1);   // resident workgroups (by registers), 32 CUs
+};
+using WgLarge = WgTile<2>;   // 256 x 256
+using WgSmall = WgTile<1>;   // 128 x 128
 constexpr int kWgXcds = 8;
-// Resident workgroups per XCD on MI355X: 32 CUs x 2 (the two stage buffers
-// take 76 KB of a CU's 160 KB of LDS).
-constexpr int kWgSlotsPerXcd = 64;
+
+// Instruction classes of __builtin_amdgcn_sched_group_barrier.
+constexpr int kSchedValu = 0x2;
+constexpr int kSchedMfma = 0x8;
+constexpr int kSchedDsRead = 0x100;
+constexpr int kSchedDsWrite = 0x200;
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 LdsS16x4;
 
 template <int T>
 __device__ __forceinline__ float bits_to_float(uint32_t bits) {
@@ -52,26 +87,6 @@ __device__ __forceinline__ float bits_to_float(uint32_t bits) {
         return bf16_bits_to_float(static_cast<uint16_t>(bits));
     } else {
         return f16_bits_to_float(static_cast<uint16_t>(bits));
-    }
-}
-
-// 8 elements of one row (columns c .. c + 7 of a [rows, cols] matrix), zero
-// past the columns and for a dead row; VEC: one 16-byte load (cols and the
-// row stride multiples of 8).
-template <bool VEC>
-__device__ __forceinline__ u32x4 load_piece(const uint16_t* base, int64_t row, int64_t stride,
-                                            int64_t c, int64_t cols, bool live) {
-    if constexpr (VEC) {
-        return (live && c < cols) ? *reinterpret_cast<const u32x4*>(base + row * stride + c) : u32x4{};
-    } else {
-        u32x4 v;
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const uint32_t lo = (live && c + 2 * p < cols) ? base[row * stride + c + 2 * p] : 0u;
-            const uint32_t hi = (live && c + 2 * p + 1 < cols) ? base[row * stride + c + 2 * p + 1] : 0u;
-            v[p] = lo | (hi << 16);
-        }
-        return v;
     }
 }
 
@@ -89,40 +104,65 @@ __device__ __forceinline__ u32x4 to_bf16_piece(const u32x4& raw) {
     }
 }
 
-// Column c of an 8 x 8 block of 16-bit values given as 8 rows of 8: the
-// block's rows 2p and 2p + 1 of that column form dword p.
-__device__ __forceinline__ u32x4 block_column(const u32x4 (&rows)[8], int c) {
-    const int q = c >> 1;
-    u32x4 out;
+// One operand's pieces of a stage: columns c .. c + 7 of rows row_lane +
+// kWgRowLanes * i, zero past the rows (end) and the columns.  VEC: raw-buffer
+// loads whose buffer ends with the split's last row (cols, the row stride and
+// the base multiples of 16 bytes); else element loads under conditions.
+template <typename Tile, bool VEC>
+__device__ __forceinline__ void load_pieces(u32x4 (&out)[Tile::kPasses], const uint16_t* base, int64_t row,
+                                            int64_t end, int64_t stride, int64_t c, int64_t cols, int row_lane) {
+    if constexpr (VEC) {
+        const BufferRsrc buffer = make_buffer(base + row * stride, (end - row) * stride * 2);
+        const uint32_t offset = c < cols ? static_cast<uint32_t>((row_lane * stride + c) * 2) : kOutOfRange;
+        const uint32_t step = c < cols ? static_cast<uint32_t>(Tile::kRowLanes * stride * 2) : 0u;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const uint32_t a = rows[2 * p][q];
-        const uint32_t b = rows[2 * p + 1][q];
-        // Byte selectors of v_perm_b32 over {b : a}: low halves or high halves.
-        out[p] = __builtin_amdgcn_perm(b, a, (c & 1) ? 0x07060302u : 0x05040100u);
+        for (int i = 0; i < Tile::kPasses; ++i) {
+            out[i] = buffer_load16(buffer, offset + i * step);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < Tile::kPasses; ++i) {
+            const int64_t m = row + row_lane + Tile::kRowLanes * i;
+            u32x4 v;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const uint32_t lo = (m < end && c + 2 * p < cols) ? base[m * stride + c + 2 * p] : 0u;
+                const uint32_t hi = (m < end && c + 2 * p + 1 < cols) ? base[m * stride + c + 2 * p + 1] : 0u;
+                v[p] = lo | (hi << 16);
+            }
+            out[i] = v;
+        }
     }
-    return out;
 }
+
+template <typename Tile>
+struct WgStage {
+    u32x4 g[Tile::kPasses];
+    u32x4 x[Tile::kPasses];
+    uint32_t keep[Tile::kPasses];
+};
 
 }  // namespace
 
-template <int GT, int XT, bool VEC>
+// MASK: a.row_mask is set; SUMS: a.bias_partials is set.  Both are template
+// choices so that a stage is one basic block: the conversions, LDS writes and
+// loads of the next stages are then scheduled between the MFMAs of this one.
+template <typename Tile, int GT, int XT, bool VEC, bool MASK, bool SUMS>
 __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs a) {
-    // Column-major stage buffers: s_t[buf][operand][column * kWgPitch + row].
-    __shared__ __attribute__((aligned(16))) uint16_t s_t[2][2][kWgTile * kWgPitch];
-    __shared__ float s_sum[kWgRows / 8][kWgTile];
+    // Row-major stage buffers: s_t[buf][operand][row * Tile::kPitch + column].
+    __shared__ __attribute__((aligned(16))) uint16_t s_t[2][2][kWgRows * Tile::kPitch];
+    __shared__ float s_sum[Tile::kRowLanes][Tile::kEdge];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5;
     const int64_t tiles = a.tiles_n * a.tiles_k;
-    int64_t tile = blockIdx.x;
-    int64_t split = 0;
-    if (a.splits > 1) {
+    int64_t tile;
+    int64_t split;
+    if (a.dealt) {
         // Row splits dealt round-robin over the XCDs, each XCD walking all
-        // output tiles of its splits.  With one split the grid holds one
-        // workgroup per output tile.
+        // output tiles of its splits.
         const int64_t xcd = blockIdx.x % kWgXcds;
         const int64_t slot = blockIdx.x / kWgXcds;
         tile = slot % tiles;
@@ -130,159 +170,192 @@ __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs 
         if (split >= a.splits) {
             return;
         }
+    } else {
+        tile = blockIdx.x % tiles;
+        split = blockIdx.x / tiles;
     }
     const int64_t nt = tile / a.tiles_k;
     const int64_t kt = tile - nt * a.tiles_k;
-    const int64_t n0 = nt * kWgTile;
-    const int64_t k0 = kt * kWgTile;
+    const int64_t n0 = nt * Tile::kEdge;
+    const int64_t k0 = kt * Tile::kEdge;
     const int64_t N = a.out_features;
     const int64_t K = a.in_features;
     const int64_t r0 = split * a.rows_per_split;
     const int64_t r1 = r0 + a.rows_per_split < a.rows ? r0 + a.rows_per_split : a.rows;
 
-    // This thread's 8 x 8 block of each stage: operand (waves 0-1: g, 2-3: x),
-    // rows 8 rb .. + 7 and columns 8 cb .. + 7 of the stage's 64 x 128 tile.
-    const int operand = wave >> 1;                  // wave-uniform
-    const int block = tid & 127;
-    const int rb = block >> 4;
-    const int cb = block & 15;
-    const bool is_g = operand == 0;
-    const uint16_t* src = static_cast<const uint16_t*>(is_g ? a.g : a.x);
-    const int64_t stride = is_g ? a.g_stride : a.x_stride;
-    const int64_t cols = is_g ? N : K;
-    const int64_t c0 = (is_g ? n0 : k0) + 8 * cb;
-    const bool sums = is_g && a.bias_partials != nullptr && kt == 0;
+    const int row_lane = tid / Tile::kPieces;
+    const int piece = tid % Tile::kPieces;
+    const uint16_t* g = static_cast<const uint16_t*>(a.g);
+    const uint16_t* x = static_cast<const uint16_t*>(a.x);
 
-    u32x4 raw[8];
     float colsum[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         colsum[e] = 0.0f;
     }
-    auto load = [&](int64_t base) {
+    auto load = [&](WgStage<Tile>& stage, int64_t row) {
+        load_pieces<Tile, VEC>(stage.g, g, row, r1, a.g_stride, n0 + 8 * piece, N, row_lane);
+        load_pieces<Tile, VEC>(stage.x, x, row, r1, a.x_stride, k0 + 8 * piece, K, row_lane);
+        if constexpr (MASK) {
+            const BufferRsrc mask = make_buffer(a.row_mask + row, r1 - row);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int64_t m = base + 8 * rb + r;
-            bool keep = m < r1;
-            if (keep && a.row_mask != nullptr) {
-                keep = a.row_mask[m] != 0;
+            for (int i = 0; i < Tile::kPasses; ++i) {
+                stage.keep[i] = buffer_load_byte(mask, row_lane + Tile::kRowLanes * i);
             }
-            raw[r] = load_piece<VEC>(src, keep ? m : r0, stride, c0, cols, keep);
         }
     };
-    auto store = [&](int buf) {
-        u32x4 rows[8];
-        if (is_g) {
+    auto commit = [&](WgStage<Tile>& stage, int buf) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                rows[r] = to_bf16_piece<GT>(raw[r]);
-                if (sums) {
-                    // Excluded rows were loaded as zeros; the sums take g in its own precision.
+        for (int i = 0; i < Tile::kPasses; ++i) {
+            if constexpr (MASK) {
 #pragma unroll
-                    for (int p = 0; p < 4; ++p) {
-                        colsum[2 * p] += bits_to_float<GT>(raw[r][p] & 0xffffu);
-                        colsum[2 * p + 1] += bits_to_float<GT>(raw[r][p] >> 16);
-                    }
+                for (int p = 0; p < 4; ++p) {
+                    stage.g[i][p] = stage.keep[i] != 0 ? stage.g[i][p] : 0u;
+                    stage.x[i][p] = stage.keep[i] != 0 ? stage.x[i][p] : 0u;
                 }
             }
-        } else {
+            if constexpr (SUMS) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                rows[r] = to_bf16_piece<XT>(raw[r]);
+                for (int p = 0; p < 4; ++p) {
+                    colsum[2 * p] += bits_to_float<GT>(stage.g[i][p] & 0xffffu);
+                    colsum[2 * p + 1] += bits_to_float<GT>(stage.g[i][p] >> 16);
+                }
             }
-        }
-        uint16_t* dst = s_t[buf][operand];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            *reinterpret_cast<u32x4*>(dst + stage_offset(8 * cb + c, rb)) = block_column(rows, c);
+            const int at = (row_lane + Tile::kRowLanes * i) * Tile::kPitch + 8 * piece;
+            *reinterpret_cast<u32x4*>(s_t[buf][0] + at) = to_bf16_piece<GT>(stage.g[i]);
+            *reinterpret_cast<u32x4*>(s_t[buf][1] + at) = to_bf16_piece<XT>(stage.x[i]);
         }
     };
 
-    const int wn = wave & 1;    // 64-row (n) half of the output tile
-    const int wk = wave >> 1;   // 64-column (k) half of the output tile
-    f32x16 acc[2][2];
+    constexpr int NB = Tile::kNB;
+    constexpr int KB = Tile::kKB;
+    const int wn = 32 * NB * (wave & 3);    // this wave's quarter (n) and half (k) of the output tile
+    const int wk = 32 * KB * (wave >> 2);
+    f32x16 acc[NB][KB];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
+        for (int kb = 0; kb < KB; ++kb) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 acc[nb][kb][e] = 0.0f;
             }
         }
     }
-    auto compute = [&](int buf) {
-        const uint16_t* gt = s_t[buf][0];
-        const uint16_t* xt = s_t[buf][1];
+    // This lane's 8 bytes of a transposed read: row (lane % 16) / 4 of the 4
+    // rows (8 rows further for the upper half wave: the K order of the
+    // fragments), 4 columns of its 16-column group.
+    const int fragment = ((lane & 15) / 4 + 8 * half) * Tile::kPitch + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    auto read_fragment = [&](const uint16_t* base) {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4*)(base));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4*)(base + 4 * Tile::kPitch));
+        const u32x2 l = __builtin_bit_cast(u32x2, lo);
+        const u32x2 h = __builtin_bit_cast(u32x2, hi);
+        return (u32x4){l[0], l[1], h[0], h[1]};
+    };
+    // One stage: the products of LDS buffer `buf`, and between them the next
+    // stage's pieces (`stage`, loaded two steps ago) into the other buffer and
+    // the loads of the stage three ahead into the registers they leave.
+    // Waves whose block lies past N or K multiply zeros (LDS holds zeros past
+    // the columns) rather than branch.
+    auto step = [&](int buf, WgStage<Tile>& stage, int64_t next_row) {
+        const uint16_t* gt = s_t[buf][0] + fragment + wn;
+        const uint16_t* xt = s_t[buf][1] + fragment + wk;
+        u32x4 af[kWgSteps][NB];
+        u32x4 bf[kWgSteps][KB];
 #pragma unroll
-        for (int kk = 0; kk < kWgRows / 16; ++kk) {
-            const int group = 2 * kk + half;
-            u32x4 af[2];
-            u32x4 bf[2];
+        for (int kk = 0; kk < kWgSteps; ++kk) {
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                af[b] = *reinterpret_cast<const u32x4*>(gt + stage_offset(wn * 64 + b * 32 + (lane & 31), group));
-                bf[b] = *reinterpret_cast<const u32x4*>(xt + stage_offset(wk * 64 + b * 32 + (lane & 31), group));
+            for (int b = 0; b < NB; ++b) {
+                af[kk][b] = read_fragment(gt + 16 * kk * Tile::kPitch + 32 * b);
             }
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
+            for (int b = 0; b < KB; ++b) {
+                bf[kk][b] = read_fragment(xt + 16 * kk * Tile::kPitch + 32 * b);
+            }
+        }
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb) {
-                    acc[nb][kb] = mfma32x32x16(af[nb], bf[kb], acc[nb][kb]);
+        for (int kk = 0; kk < kWgSteps; ++kk) {
+            if (kk == kWgSteps - 1) {
+                commit(stage, buf ^ 1);
+                load(stage, next_row);
+            }
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    acc[nb][kb] = mfma32x32x16(af[kk][nb], bf[kk][kb], acc[nb][kb]);
                 }
             }
         }
-    };
-    // One stage ahead: the loads of stage s + 1 are issued before stage s is
-    // multiplied, and written to the other LDS buffer after it.
-    int buf = 0;
-    if (r0 < r1) {
-        load(r0);
-        store(0);
-    }
-    __syncthreads();
-    for (int64_t base = r0; base < r1; base += kWgRows) {
-        const bool more = base + kWgRows < r1;
-        if (more) {
-            load(base + kWgRows);
+        // The order of the block: the first K step's fragments, its MFMAs with
+        // the second's fragment reads between them, then the second's MFMAs
+        // with the next stage's conversions and LDS writes between them.
+        constexpr int kReads = 2 * (NB + KB);
+        constexpr int kProducts = NB * KB;
+        constexpr int kPerProduct = kReads / kProducts + (kReads % kProducts != 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, kReads, 0);
+#pragma unroll
+        for (int i = 0; i < kProducts; ++i) {
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedDsRead, kPerProduct, 0);
         }
-        compute(buf);
-        if (more) {
-            store(buf ^ 1);
+#pragma unroll
+        for (int i = 0; i < kProducts; ++i) {
+            __builtin_amdgcn_sched_group_barrier(kSchedValu, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedDsWrite, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
         }
         __syncthreads();
-        buf ^= 1;
+    };
+    // Stages past the split load zeros without an access; an odd last one is
+    // multiplied all the same (a branch around it would make the loop carry
+    // copies of the registers in flight, and wait for them).
+    WgStage<Tile> even;
+    WgStage<Tile> odd;
+    load(even, r0);
+    load(odd, r0 + kWgRows);
+    commit(even, 0);
+    load(even, r0 + 2 * kWgRows);
+    __syncthreads();
+    for (int64_t row = r0; row < r1; row += 2 * kWgRows) {
+        step(0, odd, row + 3 * kWgRows);
+        step(1, even, row + 4 * kWgRows);
     }
 
     // Partials: lane (half, j) of block (nb, kb) holds column k = j and rows
     // n = 8 q + 4 half + e of the block, for accumulator entry 4 q + e.
     float* out = a.partials + split * N * K;
+    {
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            const int64_t k = k0 + wk * 64 + kb * 32 + (lane & 31);
+            for (int kb = 0; kb < KB; ++kb) {
+                const int64_t nb0 = n0 + wn + 32 * nb;
+                const int64_t kb0 = k0 + wk + 32 * kb;
+                const bool whole = nb0 + 32 <= N && kb0 + 32 <= K;   // uniform
+                const int64_t k = kb0 + (lane & 31);
+                float* block = out + (nb0 + 4 * half) * K + k;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int64_t n = n0 + wn * 64 + nb * 32 + 8 * (e / 4) + 4 * half + (e % 4);
-                if (n < N && k < K) {
-                    out[n * K + k] = acc[nb][kb][e];
+                for (int e = 0; e < 16; ++e) {
+                    const int64_t n = 8 * (e / 4) + (e % 4);
+                    if (whole || (nb0 + 4 * half + n < N && k < K)) {
+                        block[n * K] = acc[nb][kb][e];
+                    }
                 }
             }
         }
     }
-    if (a.bias_partials != nullptr && kt == 0) {
-        if (sums) {
+    if (SUMS && kt == 0) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                s_sum[rb][8 * cb + e] = colsum[e];
-            }
+        for (int e = 0; e < 8; ++e) {
+            s_sum[row_lane][8 * piece + e] = colsum[e];
         }
         __syncthreads();
-        if (tid < kWgTile) {
+        if (tid < Tile::kEdge) {
             float total = 0.0f;
 #pragma unroll
-            for (int r = 0; r < kWgRows / 8; ++r) {
+            for (int r = 0; r < Tile::kRowLanes; ++r) {
                 total += s_sum[r][tid];
             }
             if (n0 + tid < N) {
@@ -292,19 +365,44 @@ __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs 
     }
 }
 
+// The output tile.  The large tile moves half the operand bytes between L2 and
+// the CUs per product but writes four times the partials per workgroup and
+// leaves short row ranges with fewer, longer chains.  Measured with the column
+// sums, large against small (us): 131,072 rows x (640, 256) 79 / 80, x (768,
+// 384) 127 / 144, x (768, 768) 191 / 298, 65,536 x (512, 256) 45 / 46, 16,000 x
+// (768, 768) 46 / 53; but 65,536 x (256, 256) 37 / 31, 16,000 x (768, 384)
+// 39 / 37, 8,192 x (1,344, 768) 48 / 45, 2,048 x (512, 256) 24 / 19: the line
+// lies near 2^33 multiply-adds.
+bool weight_grad_large(int64_t rows, int64_t in_features, int64_t out_features) {
+    return static_cast<double>(rows) * in_features * out_features >= 8.5e9;
+}
+
+// Row splits.  More splits put more CUs on the product (its time falls as 1 /
+// splits) but write and read again splits x N x K floats: with a workgroup's
+// matrix rate p and the memory rate m the sum of 2 M N K / (splits tiles p)
+// and 8 splits N K / m is least at splits = sqrt(M m / (4 tiles p)); m = 5
+// TB/s, p = 2 TFLOP/s (a workgroup of a short problem is latency-bound).  Up
+// to one XCD's resident workgroups in output tiles, the splits are a multiple
+// of the eight XCDs, at least 16 (two 32-row stages already take longer than
+// their sum saves), bounded so that all workgroups of an XCD (its splits x the
+// output tiles) are resident at once: one more, nearly empty round would take
+// as long as the first.  Beyond, as many splits as keep the device's CUs busy
+// in one round, not dealt to the XCDs.
 void plan_weight_grad(int64_t rows, int64_t in_features, int64_t out_features, int64_t* splits,
                       int64_t* rows_per_split) {
-    const int64_t tiles = ((out_features + kWgTile - 1) / kWgTile) * ((in_features + kWgTile - 1) / kWgTile);
+    const bool large = weight_grad_large(rows, in_features, out_features);
+    const int64_t edge = large ? WgLarge::kEdge : WgSmall::kEdge;
+    const int64_t slots = large ? WgLarge::kSlotsPerXcd : WgSmall::kSlotsPerXcd;
+    const int64_t tiles = ((out_features + edge - 1) / edge) * ((in_features + edge - 1) / edge);
     const int64_t stages = (rows + kWgRows - 1) / kWgRows;
-    // As many row splits per XCD as let all of that XCD's workgroups (its
-    // splits x the output tiles) be resident at once: one more, nearly empty
-    // round of workgroups would take as long as the first.  When the output
-    // tiles alone fill every resident slot of the device, splitting the rows
-    // gains no occupancy and only multiplies the FP32 partials (splits x N x
-    // K floats, written and summed again), so the rows stay in one split.
-    int64_t per_xcd = kWgSlotsPerXcd / tiles;
-    if (per_xcd < 1) per_xcd = 1;
-    int64_t want = tiles >= kWgXcds * kWgSlotsPerXcd ? 1 : kWgXcds * per_xcd;
+    int64_t want;
+    if (tiles <= slots) {
+        const double best = std::sqrt(static_cast<double>(rows) * 5.0 / (4.0 * 2.0 * static_cast<double>(tiles)));
+        const int64_t per_xcd = std::max<int64_t>(2, static_cast<int64_t>(best / kWgXcds + 0.5));
+        want = kWgXcds * std::min(per_xcd, slots / tiles);
+    } else {
+        want = std::max<int64_t>(1, kWgXcds * slots / tiles);
+    }
     if (want > stages) want = stages;
     if (want < 1) want = 1;
     const int64_t per = (rows + want - 1) / want;
@@ -312,22 +410,46 @@ void plan_weight_grad(int64_t rows, int64_t in_features, int64_t out_features, i
     *splits = rows == 0 ? 0 : (rows + *rows_per_split - 1) / *rows_per_split;
 }
 
-template <int GT, int XT>
+template <typename Tile, int GT, int XT, bool VEC>
 static void launch_wg(const WeightGradArgs& a, dim3 grid, hipStream_t stream) {
-    if (a.vec) {
-        weight_grad_kernel<GT, XT, true><<<grid, kWgThreads, 0, stream>>>(a);
+    const auto run = [&](auto kernel) { kernel<<<grid, kWgThreads, 0, stream>>>(a); };
+    if (a.row_mask != nullptr) {
+        a.bias_partials != nullptr ? run(weight_grad_kernel<Tile, GT, XT, VEC, true, true>)
+                                   : run(weight_grad_kernel<Tile, GT, XT, VEC, true, false>);
     } else {
-        weight_grad_kernel<GT, XT, false><<<grid, kWgThreads, 0, stream>>>(a);
+        a.bias_partials != nullptr ? run(weight_grad_kernel<Tile, GT, XT, VEC, false, true>)
+                                   : run(weight_grad_kernel<Tile, GT, XT, VEC, false, false>);
     }
 }
 
-hipError_t launch_weight_grad(const WeightGradArgs& a, int g_dtype, int x_dtype, hipStream_t stream) {
-    if (a.splits == 0) {
+template <int GT, int XT>
+static void launch_wg(const WeightGradArgs& a, dim3 grid, hipStream_t stream) {
+    if (!a.vec) {
+        launch_wg<WgSmall, GT, XT, false>(a, grid, stream);
+    } else if (a.large) {
+        launch_wg<WgLarge, GT, XT, true>(a, grid, stream);
+    } else {
+        launch_wg<WgSmall, GT, XT, true>(a, grid, stream);
+    }
+}
+
+hipError_t launch_weight_grad(const WeightGradArgs& args, int g_dtype, int x_dtype, hipStream_t stream) {
+    if (args.splits == 0) {
         return hipSuccess;
     }
+    WeightGradArgs a = args;
+    // The raw buffers' 32-bit offsets reach one stage's rows.  Element loads
+    // (rows that are not whole 16-byte pieces) take the small tile, whose
+    // registers have room for them; the splits are the plan's either way.
+    a.vec = a.vec && a.g_stride < (1 << 24) && a.x_stride < (1 << 24);
+    a.large = a.vec && weight_grad_large(a.rows, a.in_features, a.out_features);
+    const int64_t edge = a.large ? WgLarge::kEdge : WgSmall::kEdge;
+    a.tiles_n = (a.out_features + edge - 1) / edge;
+    a.tiles_k = (a.in_features + edge - 1) / edge;
     const int64_t tiles = a.tiles_n * a.tiles_k;
+    a.dealt = a.splits > 1 && tiles <= (a.large ? WgLarge::kSlotsPerXcd : WgSmall::kSlotsPerXcd);
     const int64_t rounds = (a.splits + kWgXcds - 1) / kWgXcds;
-    const dim3 grid(static_cast<unsigned>(a.splits == 1 ? tiles : rounds * kWgXcds * tiles));
+    const dim3 grid(static_cast<unsigned>(a.dealt ? rounds * kWgXcds * tiles : a.splits * tiles));
     if (g_dtype == LSSO_HIP_F16) {
         if (x_dtype == LSSO_HIP_F16) {
             launch_wg<LSSO_HIP_F16, LSSO_HIP_F16>(a, grid, stream);
@@ -343,7 +465,5 @@ hipError_t launch_weight_grad(const WeightGradArgs& a, int g_dtype, int x_dtype,
     }
     return hipGetLastError();
 }
-
-int weight_grad_tile() { return kWgTile; }
 
 }  // namespace lsso_hip

@@ -1,0 +1,73 @@
+"""The weight-gradient kernel at the edges of its tiles and plans (GPU): both
+output tiles (256 x 256 from about 2^33 multiply-adds on, else 128 x 128), column
+remainders, a last stage of one row, rows that are not whole 16-byte pieces,
+masks and the variants without bias sums, against FP64 of the same BF16
+operands.
+
+Bound: an output is a chain of at most `rows` FP32 additions of products that
+are exact in FP32; for independent zero-mean terms the rounding errors add like
+a random walk, so the relative L2 error is at most about 2^-24 sqrt(rows)."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize(
+    ("rows", "in_features", "out_features", "g_dtype", "x_dtype", "masked", "pad", "bias"),
+    [
+        (65537, 264, 520, torch.bfloat16, torch.float16, False, 0, True),     # large tile, remainders, odd last stage
+        (65537, 264, 520, torch.float16, torch.bfloat16, True, 8, False),
+        (131072, 256, 264, torch.float16, torch.float16, True, 0, True),
+        (33, 128, 128, torch.bfloat16, torch.bfloat16, False, 0, True),       # one whole small tile, a row past a stage
+        (1, 136, 120, torch.float16, torch.bfloat16, False, 0, False),
+        (2000, 768, 1344, torch.bfloat16, torch.bfloat16, True, 0, True),     # more tiles than an XCD's workgroups
+        (517, 131, 257, torch.bfloat16, torch.float16, False, 0, True),       # element loads
+        (4100, 72, 56, torch.float16, torch.float16, True, 3, False),         # a row stride that is not whole pieces
+    ],
+)
+def test_weight_gradient_tiles_match_fp64(
+    native, rows, in_features, out_features, g_dtype, x_dtype, masked, pad, bias
+) -> None:
+    generator = torch.Generator(device="cuda").manual_seed(rows + in_features)
+
+    def matrix(cols, dtype):
+        storage = torch.randn(rows, cols + pad, device="cuda", generator=generator)
+        return storage.to(dtype)[:, :cols]
+
+    g, x = matrix(out_features, g_dtype), matrix(in_features, x_dtype)
+    mask = None
+    if masked:
+        mask = torch.rand(rows, device="cuda", generator=generator) > 0.3
+        g[~mask] = float("nan")
+        x[~mask] = float("inf")
+    grad_weight, grad_bias = native._weight_gradient(g, x, mask, bias)
+    if masked:
+        g, x = torch.where(mask[:, None], g, 0), torch.where(mask[:, None], x, 0)
+    expected = g.bfloat16().double().t().contiguous() @ x.bfloat16().double()
+    limit = 2.0 ** -24 * max(2.0, math.sqrt(rows))
+    assert float((grad_weight.double() - expected).norm() / expected.norm()) <= limit
+    again, _ = native._weight_gradient(g, x, None, bias)
+    assert torch.equal(again, grad_weight)              # zeros in place of the excluded rows: the same sums
+    if bias:
+        scale = g.double().abs().sum(0)
+        assert torch.all((grad_bias.double() - g.double().sum(0)).abs() <= limit * scale)
+    else:
+        assert grad_bias is None
+
+
+@pytest.mark.parametrize(("splits", "cols"), ((1, 5), (2, 4), (7, 132), (64, 8), (600, 1024), (33, 1003)))
+def test_column_sums_of_few_and_many_splits(native, splits, cols) -> None:
+    """The split sums' lane plans (one lane per piece to 32, whole and odd
+    pieces) through the one-pass column sums, whose splits follow the rows."""
+
+    rows = splits * 16
+    g = torch.randn(rows, cols, device="cuda").bfloat16()
+    _, sums = native._grad_columns(g, None, False, True)
+    scale = g.double().abs().sum(0)
+    assert torch.all((sums.double() - g.double().sum(0)).abs() <= 2.0 ** -24 * math.sqrt(rows) * scale)
