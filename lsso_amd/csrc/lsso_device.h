@@ -243,40 +243,96 @@ __device__ __forceinline__ void load_weight_row(u32x4 (&wreg)[KSTEPS], const flo
     }
 }
 
-// load_weight_row for K a multiple of 8, through one raw buffer over the
-// whole [N, K] weight (wave-uniform descriptor, per-lane offsets; a row
-// n < 0 and columns past K read as zeros): no per-element fallback, so
-// loading several rows keeps no address registers alive.
-template <int KSTEPS>
-__device__ __forceinline__ void load_weight_row_k8(u32x4 (&wreg)[KSTEPS], const float* weight,
-                                                   int64_t n, int64_t N, int64_t K, int lane) {
-    const int half = lane >> 5;
-    const BufferRsrc buffer = make_buffer(weight, 4 * N * K);
-    const uint32_t row = n >= 0 ? static_cast<uint32_t>(4 * n * K) : kOutOfRange;
+// load_weight_row of NB x 32 rows for K a multiple of 4, coalesced: 8 lanes
+// read one row's 32 columns (one 128-byte line) per 16-byte load, the BF16
+// values pass through `scratch` (kWeightScratch bf16 of LDS of this wave's
+// own, so no barrier) and come back in the lane layout.  row_offset(nb, r) is
+// the byte offset of row r of block nb in the raw buffer, or kOutOfRange;
+// columns past K read as zeros.  A persistent kernel cannot start its first
+// tile before its weights are in registers.  Read by the lanes that keep them
+// (row n at 16 bytes per lane, one K step at a time, as load_weight_row does),
+// every load touches 32 lines for a quarter of their bytes and waits for the
+// one before; with eight steps in flight instead, the lines of all waves no
+// longer fit the L1 and are fetched four times (the training step at 262,144
+// tokens 4% slower).  Four 2-step pieces are in flight here; the scheduling
+// barriers keep the FP32 staging of the whole slice from being live at once.
+// With it the layer call at 64 x 1,024 x 256 (rank 32) takes 84 us instead of
+// 92, at 64 x 4,096 212 instead of 221; and the fused kernels, which spilled 12
+// to 36 registers around the per-lane addresses, spill none.
+constexpr int kWeightPitch = 40;                      // bf16 per row of 32: 16 rows' 16-byte reads cover all banks
+constexpr int kWeightScratch = 32 * kWeightPitch;     // bf16 per wave
+constexpr int kWeightRing = 4;
+template <int NB, int KSTEPS, typename RowOffset>
+__device__ __forceinline__ void load_weight_rows(u32x4 (&wreg)[NB][KSTEPS], BufferRsrc buffer, RowOffset row_offset,
+                                                 int64_t K, int lane, uint16_t* scratch) {
+    static_assert(KSTEPS % 2 == 0, "a piece is two K steps");
+    constexpr int kPieces = KSTEPS / 2;
+    constexpr int kTotal = NB * kPieces;
+    constexpr int kRing = kTotal < kWeightRing ? kTotal : kWeightRing;
+    const int row8 = lane >> 3;
+    const uint32_t k_lane = 4 * (lane & 7);
+    const uint32_t k_end = static_cast<uint32_t>(K);
+    uint32_t offset[NB][4];
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-        const uint32_t k0 = 16 * ks + 8 * half;
-        const bool live = n >= 0 && k0 < K;
-        const f32x4 lo = __builtin_bit_cast(f32x4, buffer_load16(buffer, live ? row + 4 * k0 : kOutOfRange));
-        const f32x4 hi = __builtin_bit_cast(f32x4, buffer_load16(buffer, live ? row + 4 * k0 + 16 : kOutOfRange));
-        wreg[ks][0] = pack_bf16(lo[0], lo[1]);
-        wreg[ks][1] = pack_bf16(lo[2], lo[3]);
-        wreg[ks][2] = pack_bf16(hi[0], hi[1]);
-        wreg[ks][3] = pack_bf16(hi[2], hi[3]);
-        // One K step at a time, so the FP32 staging of the whole row is never
-        // live at once.
+    for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            offset[nb][j] = row_offset(nb, 8 * j + row8);
+        }
+    }
+    u32x4 raw[kRing][4];
+    auto issue = [&](int i) {
+        const uint32_t k0 = 32 * (i % kPieces) + k_lane;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t row = offset[i / kPieces][j];
+            raw[i % kRing][j] = buffer_load16(buffer, k0 < k_end && row != kOutOfRange ? row + 4 * k0 : kOutOfRange);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < kRing; ++i) {
+        issue(i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kTotal; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const f32x4 v = __builtin_bit_cast(f32x4, raw[i % kRing][j]);
+            const u32x2 packed = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+            *reinterpret_cast<u32x2*>(scratch + (8 * j + row8) * kWeightPitch + k_lane) = packed;
+        }
+        if (i + kRing < kTotal) {
+            issue(i + kRing);
+        }
+        // LDS operations of one wave execute in order: these reads see the
+        // writes above, and the next piece's writes follow them.
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            wreg[i / kPieces][2 * (i % kPieces) + s] = *reinterpret_cast<const u32x4*>(
+                scratch + (lane & 31) * kWeightPitch + 16 * s + 8 * (lane >> 5));
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
 }
 
 // Resident slice of rows n0 .. n0 + 31 (one row per lane % 32), columns
-// k_base .. k_base + 16 KSTEPS.
+// k_base .. k_base + 16 KSTEPS; vector: K is a multiple of 4 and the weight
+// 16-byte aligned.
 template <int KSTEPS>
-__device__ __forceinline__ void load_weight_slice(u32x4 (&wreg)[KSTEPS], const float* weight,
-                                                  int64_t N, int64_t K, int64_t n0, int lane,
-                                                  int64_t k_base = 0) {
-    const int64_t n = n0 + (lane & 31);
-    load_weight_row<KSTEPS>(wreg, weight, n < N ? n : -1, K, lane, k_base);
+__device__ __forceinline__ void load_weight_slice(u32x4 (&wreg)[1][KSTEPS], const float* weight,
+                                                  int64_t N, int64_t K, int64_t n0, int lane, bool vector,
+                                                  uint16_t* scratch, int64_t k_base = 0) {
+    if (vector) {   // uniform
+        const int64_t rows = N - n0 < 32 ? N - n0 : 32;
+        const int64_t skip = (n0 < N ? n0 : 0) * K + k_base;
+        const auto row_offset = [&](int, int r) { return static_cast<uint32_t>(4 * r * K); };
+        load_weight_rows<1, KSTEPS>(wreg, make_buffer(weight + skip, 4 * (rows * K - k_base)), row_offset,
+                                    K - k_base, lane, scratch);
+    } else {
+        const int64_t n = n0 + (lane & 31);
+        load_weight_row<KSTEPS>(wreg[0], weight, n < N ? n : -1, K, lane, k_base);
+    }
 }
 
 }  // namespace lsso_hip

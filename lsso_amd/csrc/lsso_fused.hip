@@ -115,11 +115,14 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
         const int half = lane >> 5;
         const int ksteps = (Di + 15) / 16;
         u32x4 wreg[2][kMixKSteps];
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            const int n = n0 + 32 * nb + lane_c;
-            load_weight_row_k8<kMixKSteps>(wreg[nb], a.weight, n < Di ? n : -1, D, D, lane);
-        }
+        static_assert(kMixRows * kMixStPitch >= kWeightScratch, "the output stage holds the weight scratch");
+        load_weight_rows<2, kMixKSteps>(
+            wreg, make_buffer(a.weight, 4 * D * D),
+            [&](int nb, int r) {
+                const int n = n0 + 32 * nb + r;
+                return n < Di ? 4u * static_cast<uint32_t>(n * Di) : kOutOfRange;
+            },
+            D, lane, s_st[wave]);
         // Output pieces of this lane: row p / 8, features n0 + 8 (p % 8) ..,
         // for p = lane + 64 i (16 bytes each).
         uint16_t* stage = s_st[wave];

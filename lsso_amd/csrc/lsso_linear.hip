@@ -188,8 +188,13 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
     const int64_t K = a.in_features;
     const int64_t N = a.out_features;
 
-    u32x4 wreg[KW];
-    load_weight_slice<KW>(wreg, a.weight, N, K, n0, lane, int64_t{16} * kofs);
+    u32x4 wreg[1][KW];
+    // The output stage (or, where it is too small, the second x tile) is not
+    // written before the first tile's products.
+    constexpr bool kStageHolds = kTileRows * YP >= kWaves * kWeightScratch;
+    static_assert(kStageHolds || kTileRows * KP >= kWaves * kWeightScratch, "weight scratch");
+    load_weight_slice<KW>(wreg, a.weight, N, K, n0, lane, a.w_vector != 0,
+                          (kStageHolds ? s_y : s_x[1]) + wave * kWeightScratch, int64_t{16} * kofs);
     for (int c = tid; c < kGroupColumns; c += kThreads) {
         const int64_t n = cg * kGroupColumns + c;
         s_bias[c] = (a.bias != nullptr && n < N) ? a.bias[n] : 0.0f;
@@ -296,7 +301,7 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
                 for (int ks = 0; ks < kGroup; ++ks) {
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb) {
-                        acc[mb] = mfma32x32x16(wreg[k2 + ks], xb[slot][ks][mb], acc[mb]);
+                        acc[mb] = mfma32x32x16(wreg[0][k2 + ks], xb[slot][ks][mb], acc[mb]);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);

@@ -191,10 +191,15 @@ __global__ __launch_bounds__(pr_waves<KSTEPS>() * 64) void project_reduce_kernel
         // Projection waves.
         const int lane_c = lane & 31;
         u32x4 wreg[2][KSTEPS];
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            load_weight_row_k8<KSTEPS>(wreg[nb], a.weight, packed_column(wave * 64 + nb * 32 + lane_c), a.width, D, lane);
-        }
+        // The packed tiles are not written before the first projection.
+        static_assert(sizeof(s_y) >= kProj * kWeightScratch * sizeof(uint16_t), "the packed tiles hold the weight scratch");
+        load_weight_rows<2, KSTEPS>(
+            wreg, make_buffer(a.weight, 4 * a.width * D),
+            [&](int nb, int r) {
+                const int64_t column = packed_column(wave * 64 + nb * 32 + r);
+                return column >= 0 ? static_cast<uint32_t>(4 * column * D) : kOutOfRange;
+            },
+            D, lane, &s_y[0][0] + wave * kWeightScratch);
         __syncthreads();   // s_bias, s_col and tile 0 are in LDS
         // The packed tile k - 1 (in s_y[(k - 1) & 1]) goes out during tile
         // k's MFMAs, as 16-byte pieces of the group's two column runs: this
