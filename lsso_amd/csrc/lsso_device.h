@@ -204,41 +204,29 @@ struct ApplyLayout {
 
 // Resident BF16 row of an FP32 weight [N, K] for y^T = W x^T on
 // v_mfma_f32_32x32x16_bf16: the lane holds row n (zeros when n < 0) at
-// columns 16 ks + 8 (lane / 32) + 0..7, RNE-rounded, zero past K.  Rows are
-// read as float4 pairs when K is a multiple of 4.
+// columns 16 ks + 8 (lane / 32) + 0..7, RNE-rounded, zero past K.  Element
+// loads, for weights that load_weight_rows does not take (K not a multiple of
+// 4, or a base that is not 16-byte aligned).
 template <int KSTEPS>
 __device__ __forceinline__ void load_weight_row(u32x4 (&wreg)[KSTEPS], const float* weight,
-                                                int64_t n, int64_t K, int lane, int64_t k_base = 0) {
-    const int half = lane >> 5;
-    const bool nv = n >= 0;
-    const float* wrow = weight + (nv ? n : 0) * K;
-    const bool vector_rows = (K % 4) == 0;
+                                                int64_t n, int64_t K, int lane) {
+    const float* wrow = weight + (n >= 0 ? n : 0) * K;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
-        const int64_t k0 = k_base + 16 * ks + 8 * half;
+        const int k0 = 16 * ks + 8 * (lane >> 5);
         float v[8];
-        if (vector_rows && nv && k0 + 8 <= K) {
-            const f32x4 lo = *reinterpret_cast<const f32x4*>(wrow + k0);
-            const f32x4 hi = *reinterpret_cast<const f32x4*>(wrow + k0 + 4);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                v[i] = lo[i];
-                v[4 + i] = hi[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const bool live = nv && k0 + i < K;
-                const float value = wrow[live ? k0 + i : 0];
-                v[i] = live ? value : 0.0f;
-            }
+        for (int i = 0; i < 8; ++i) {
+            const bool live = n >= 0 && k0 + i < K;
+            const float value = wrow[live ? k0 + i : 0];
+            v[i] = live ? value : 0.0f;
         }
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             wreg[ks][p] = pack_bf16(v[2 * p], v[2 * p + 1]);
         }
-        // Convert one K step at a time: keeps the FP32 staging of W from
-        // being hoisted next to the whole BF16 slice.
+        // One K step at a time: keeps the FP32 staging of W from being
+        // hoisted next to the whole BF16 slice.
         __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -316,22 +304,20 @@ __device__ __forceinline__ void load_weight_rows(u32x4 (&wreg)[NB][KSTEPS], Buff
     }
 }
 
-// Resident slice of rows n0 .. n0 + 31 (one row per lane % 32), columns
-// k_base .. k_base + 16 KSTEPS; vector: K is a multiple of 4 and the weight
-// 16-byte aligned.
+// Resident slice of rows n0 .. n0 + 31 (one row per lane % 32); vector: K is
+// a multiple of 4 and the weight 16-byte aligned; n0 is wave-uniform.
 template <int KSTEPS>
 __device__ __forceinline__ void load_weight_slice(u32x4 (&wreg)[1][KSTEPS], const float* weight,
                                                   int64_t N, int64_t K, int64_t n0, int lane, bool vector,
-                                                  uint16_t* scratch, int64_t k_base = 0) {
+                                                  uint16_t* scratch) {
     if (vector) {   // uniform
         const int64_t rows = N - n0 < 32 ? N - n0 : 32;
-        const int64_t skip = (n0 < N ? n0 : 0) * K + k_base;
         const auto row_offset = [&](int, int r) { return static_cast<uint32_t>(4 * r * K); };
-        load_weight_rows<1, KSTEPS>(wreg, make_buffer(weight + skip, 4 * (rows * K - k_base)), row_offset,
-                                    K - k_base, lane, scratch);
+        load_weight_rows<1, KSTEPS>(wreg, make_buffer(weight + (n0 < N ? n0 : 0) * K, 4 * rows * K), row_offset,
+                                    K, lane, scratch);
     } else {
         const int64_t n = n0 + (lane & 31);
-        load_weight_row<KSTEPS>(wreg[0], weight, n < N ? n : -1, K, lane, k_base);
+        load_weight_row<KSTEPS>(wreg[0], weight, n < N ? n : -1, K, lane);
     }
 }
 

@@ -7,15 +7,25 @@
 //
 // Schedule: persistent workgroups of 8 waves.  Each wave keeps a 32-column
 // slice of W (BF16, K padded to 16) in registers for the whole launch, so the
-// weights are read once per workgroup; past K = 384 two waves share a slice,
-// one per half of K.  64-row x tiles (32-row once
-// K > 384, so that two of them and the split's partials fit LDS) are staged
-// through a double-buffered LDS tile (converted to BF16 once) and shared by
-// the workgroup's waves.
+// weights are read once per workgroup.  64-row x tiles (32-row once K > 384,
+// where W takes 128 or 160 of a wave's 256 registers) are staged through a
+// double-buffered LDS tile (converted to BF16 once) and shared by the
+// workgroup's waves.
 // The MFMA computes y^T = W x^T on v_mfma_f32_32x32x16_bf16; in that form a
 // lane's accumulators are 4 runs of 4 consecutive output features of one
 // row.  The rounded tile is staged in LDS and written back in 16-byte pieces
 // of whole row segments (scattered 8-byte writes cost half the store rate).
+//
+// Bound: HBM, by the latency of the tile loads.  A tile's products take about
+// 1 us, a load under traffic 2 to 4, so one tile in flight (32 KB per CU) ran
+// the loop at the latency's pace.  Two tiles are in flight in registers (one at
+// K > 512) while a third is multiplied, and a piece is converted and its
+// registers reloaded between two MFMAs, so the conversions hide under them.
+// Up to K = 640 a wave holds all of K: at K > 384 the former form shared a
+// 32-column slice between two waves, half of K each, and read x twice for
+// 256 outputs.  Before and now (us): 262,144 x 256 -> 256 68 / 57, x 512 -> 256
+// 142 / 98, 131,072 x 640 -> 256 79 / 55, x 256 -> 640 84 / 68, x 384 -> 768
+// 111 / 97.
 
 #include "lsso_device.h"
 #include "lsso_internal.h"
@@ -31,22 +41,19 @@ constexpr int kStreamColsHost = 128;
 template <int KSTEPS>
 constexpr int linear_tile_rows_k() { return KSTEPS <= 24 ? 64 : 32; }
 
-// Waves per workgroup: eight, two per SIMD at up to 256 registers each.  Up
-// to K = 384 each wave holds its whole 32-column slice (96 VGPRs at K = 384;
-// with four waves, one per SIMD, the K = 384 tier took 175 us instead of
-// 131 us for 32 x 4096 rows of 384 -> 768) and the K order is a single
-// chain, the one the fused projection kernels reproduce bit for bit.  Past
-// K = 384 two waves share each 32-column slice, one per half of K, and add
-// their accumulators through LDS.
-template <int KSTEPS>
-constexpr int linear_waves() { return 8; }
-template <int KSTEPS>
-constexpr int linear_ksplit() { return KSTEPS >= 32 ? 2 : 1; }
+// Waves per workgroup: eight, two per SIMD at up to 256 registers each, of
+// which a wave's 32-column W slice takes 4 per K step (160 at K = 640).
+constexpr int kLinearWaves = 8;
+
+// Instruction classes of __builtin_amdgcn_sched_group_barrier.
+constexpr int kSchedValu = 0x2;
+constexpr int kSchedMfma = 0x8;
+constexpr int kSchedDsRead = 0x100;
 
 // Tier 0 is the K-streaming kernel (any in_features above 640).
 int linear_tile_rows(int k_steps) { return k_steps == 0 ? kStreamRowsHost : (k_steps <= 24 ? 64 : 32); }
 int linear_columns_per_group(int k_steps) {
-    return k_steps == 0 ? kStreamColsHost : (k_steps <= 24 ? 8 : 4) * 32;
+    return k_steps == 0 ? kStreamColsHost : kLinearWaves * 32;
 }
 
 int linear_k_tier(int64_t in_features) {
@@ -60,14 +67,33 @@ int linear_k_tier(int64_t in_features) {
     return 0;   // K-streaming tier
 }
 
-// Load 8 consecutive x elements as BF16 one element at a time (rows whose
-// length or stride rules out 16-byte loads).  Out-of-range rows and columns
+// BF16 bits of a 16-byte piece of x as loaded.
+template <int XT>
+__device__ __forceinline__ u32x4 to_bf16_piece(const u32x4& raw) {
+    u32x4 out = raw;
+    if constexpr (XT == LSSO_HIP_F16) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            out[p] = pack_bf16(f16_lo(raw[p]), f16_hi(raw[p]));
+        }
+    }
+    return out;
+}
+
+// Load 8 consecutive x elements as BF16, for shapes outside the vector form
+// of the kernel: one 16-byte piece where x allows it (only y does not), else
+// one element at a time.  Out-of-range rows and columns
 // read a clamped in-bounds address and are zeroed by select.  Masked rows are
 // loaded like any other: the output rows they feed are zeroed in the epilogue.
 template <int XT>
-__device__ __forceinline__ u32x4 load_x_chunk_scalar(const LinearArgs& a, int64_t row, int64_t k0) {
+__device__ __forceinline__ u32x4 load_x_chunk(const LinearArgs& a, int64_t row, int64_t k0) {
     const int64_t safe_row = row < a.rows ? row : a.rows - 1;
     const uint16_t* x = static_cast<const uint16_t*>(a.x) + safe_row * a.x_stride;
+    if (a.x_vector) {
+        const bool live = row < a.rows && k0 < a.in_features;
+        const u32x4 raw = *reinterpret_cast<const u32x4*>(x + (live ? k0 : 0));
+        return live ? to_bf16_piece<XT>(raw) : u32x4{};
+    }
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -89,45 +115,6 @@ __device__ __forceinline__ u32x4 load_x_chunk_scalar(const LinearArgs& a, int64_
     return out;
 }
 
-// A staged x chunk: raw bits as loaded plus their liveness, so that the
-// loads of the next tile stay in flight while the current tile is multiplied
-// and only their conversion waits for them.
-struct XChunk {
-    u32x4 raw;
-    int live;
-};
-
-template <int XT, bool XVEC>
-__device__ __forceinline__ XChunk fetch_x_chunk(const LinearArgs& a, int64_t row, int64_t k0) {
-    XChunk c;
-    if constexpr (XVEC) {
-        const bool in_range = row < a.rows && k0 < a.in_features;
-        const int64_t safe_row = row < a.rows ? row : a.rows - 1;
-        const uint16_t* x = static_cast<const uint16_t*>(a.x) + safe_row * a.x_stride;
-        c.raw = *reinterpret_cast<const u32x4*>(x + (in_range ? k0 : 0));
-        c.live = in_range;
-    } else {
-        c.raw = load_x_chunk_scalar<XT>(a, row, k0);
-        c.live = 1;
-    }
-    return c;
-}
-
-// BF16 bits of a staged chunk (zero outside the matrix).
-template <int XT, bool XVEC>
-__device__ __forceinline__ u32x4 finish_x_chunk(const XChunk& c) {
-    u32x4 out;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        uint32_t value = c.raw[p];
-        if constexpr (XVEC && XT == LSSO_HIP_F16) {
-            value = pack_bf16(f16_lo(value), f16_hi(value));
-        }
-        out[p] = c.live ? value : 0u;
-    }
-    return out;
-}
-
 template <int YT>
 __device__ __forceinline__ uint16_t to_output_bits(float value) {
     if constexpr (YT == LSSO_HIP_BF16) {
@@ -137,15 +124,13 @@ __device__ __forceinline__ uint16_t to_output_bits(float value) {
     }
 }
 
-template <int KSTEPS, int XT, int YT, bool XVEC>
-__global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(LinearArgs a) {
-    constexpr int kWaves = linear_waves<KSTEPS>();
-    constexpr int KSPLIT = linear_ksplit<KSTEPS>();
-    constexpr int KW = KSTEPS / KSPLIT;                 // K steps per wave
-    constexpr int kSlices = kWaves / KSPLIT;            // 32-column slices per group
+// VEC: whole 16-byte pieces of x and y (a.x_vector, a.y_vector).
+template <int KSTEPS, int XT, int YT, bool VEC>
+__global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a) {
+    constexpr int kWaves = kLinearWaves;
     constexpr int kTileRows = linear_tile_rows_k<KSTEPS>();
     constexpr int MB = kTileRows / 32;                  // 32-row MFMA blocks per tile
-    constexpr int kGroupColumns = kSlices * 32;
+    constexpr int kGroupColumns = kWaves * 32;
     constexpr int KP = 16 * KSTEPS + 8;                  // LDS row pitch (bf16)
     constexpr int kChunksPerRow = 2 * KSTEPS;           // 8-element chunks
     constexpr int kThreads = kWaves * 64;
@@ -157,14 +142,12 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
     constexpr int kStoreChunks = kTileRows * kGroupColumns / 8 / kThreads;
     static_assert(kTileRows * kGroupColumns / 8 % kThreads == 0, "store split");
     __shared__ __attribute__((aligned(16))) uint16_t s_y[kTileRows * YP];
-    // Upper-K partial accumulators of a split tile, per slice, block, element and lane.
-    __shared__ float s_part[KSPLIT == 2 ? kSlices * MB * 16 * 64 : 1];
     // Row flags of the tile being multiplied and of the next one.
     __shared__ int s_keep[2][kTileRows];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: the weight buffer below is
     const int half = lane >> 5;
     // Workgroups are dealt to the eight XCDs round-robin by block index.  When
     // the grid allows, the column groups of one row tile are given to blocks
@@ -180,88 +163,109 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
         group_index = blockIdx.x / a.column_groups;
     }
     const int64_t group_count = gridDim.x / a.column_groups;
-    const int slice = wave % kSlices;
-    const int khalf = wave / kSlices;
-    const int kofs = KW * khalf;                        // first K step of this wave
+    const int slice = wave;
     const int64_t n0 = cg * kGroupColumns + slice * 32;
-    const bool slice_live = __builtin_amdgcn_readfirstlane(n0 < a.out_features ? 1 : 0) != 0;
     const int64_t K = a.in_features;
     const int64_t N = a.out_features;
 
-    u32x4 wreg[1][KW];
+    u32x4 wreg[1][KSTEPS];
     // The output stage (or, where it is too small, the second x tile) is not
     // written before the first tile's products.
     constexpr bool kStageHolds = kTileRows * YP >= kWaves * kWeightScratch;
     static_assert(kStageHolds || kTileRows * KP >= kWaves * kWeightScratch, "weight scratch");
-    load_weight_slice<KW>(wreg, a.weight, N, K, n0, lane, a.w_vector != 0,
-                          (kStageHolds ? s_y : s_x[1]) + wave * kWeightScratch, int64_t{16} * kofs);
+    load_weight_slice<KSTEPS>(wreg, a.weight, N, K, n0, lane, a.w_vector != 0,
+                              (kStageHolds ? s_y : s_x[1]) + wave * kWeightScratch);
     for (int c = tid; c < kGroupColumns; c += kThreads) {
         const int64_t n = cg * kGroupColumns + c;
         s_bias[c] = (a.bias != nullptr && n < N) ? a.bias[n] : 0.0f;
     }
 
-    // A tile's row flags are staged with its x: thread r < kTileRows reads
-    // the mask byte of row r through a raw buffer over the tile's valid rows
-    // (rows past the matrix, and every row when there is no mask, read as
-    // zero without an access), so no load waits inside the tile loop.
-    XChunk stage[kChunksPerThread];
-    uint32_t stage_mask = 0;
-    int64_t stage_rows = 0;
-    auto load_stage = [&](int64_t tile) {
-#pragma unroll
-        for (int c = 0; c < kChunksPerThread; ++c) {
-            const int chunk = tid + c * kThreads;
-            const int rr = chunk / kChunksPerRow;
-            const int cc = chunk - rr * kChunksPerRow;
-            stage[c] = fetch_x_chunk<XT, XVEC>(a, tile * kTileRows + rr, 8 * cc);
-        }
-        stage_rows = a.rows - tile * kTileRows;
-        const BufferRsrc mask = make_buffer(a.row_mask != nullptr ? a.row_mask + tile * kTileRows : nullptr,
-                                            a.row_mask != nullptr ? stage_rows : 0);
-        stage_mask = buffer_load_byte(mask, static_cast<uint32_t>(tid));
+    // One tile of x in flight: 16-byte pieces as loaded (BF16 already without
+    // VEC) and the row's mask byte.  Row flags travel with their x: thread r <
+    // kTileRows reads the byte of row r through a raw buffer over the tile's
+    // valid rows (rows past the matrix, and every row when there is no mask,
+    // read as zero without an access).
+    struct Stage {
+        u32x4 x[kChunksPerThread];
+        uint32_t mask;
+        int64_t rows;
     };
-    auto write_stage = [&](int buf) {
+    const uint16_t* x = static_cast<const uint16_t*>(a.x);
+    constexpr bool kWholeRows = kThreads % kChunksPerRow == 0;
+    const int piece_k = 8 * (tid % kChunksPerRow);
+    const uint32_t piece0 = piece_k < K ? 2u * static_cast<uint32_t>(tid / kChunksPerRow * static_cast<int>(a.x_stride) + piece_k)
+                                        : kOutOfRange;
+    const uint32_t piece_step = piece_k < K ? 2u * static_cast<uint32_t>(kThreads / kChunksPerRow) *
+                                                  static_cast<uint32_t>(a.x_stride) : 0u;
+    auto load_chunk = [&](Stage& stage, int64_t t, BufferRsrc buffer, int c) {
+        const int chunk = tid + c * kThreads;
+        const int rr = chunk / kChunksPerRow;
+        const int k0 = 8 * (chunk - rr * kChunksPerRow);
+        if constexpr (VEC) {
+            // Rows past the matrix end the buffer; columns past K get an
+            // offset beyond it.  Where the workgroup covers whole rows, a
+            // thread keeps its column and one offset serves all its pieces.
+            if constexpr (kWholeRows) {
+                stage.x[c] = buffer_load16(buffer, piece0 + c * piece_step);
+            } else {
+                const int rr_c = opaque_int(rr);
+                stage.x[c] = buffer_load16(
+                    buffer, k0 < K ? 2u * static_cast<uint32_t>(rr_c * static_cast<int>(a.x_stride) + k0) : kOutOfRange);
+            }
+        } else {
+            stage.x[c] = load_x_chunk<XT>(a, t * kTileRows + rr, k0);
+        }
+    };
+    auto tile_buffer = [&](int64_t t) {
+        return make_buffer(x + t * kTileRows * a.x_stride, 2 * (a.rows - t * kTileRows) * a.x_stride);
+    };
+    auto load_flags = [&](Stage& stage, int64_t t) {
+        stage.rows = a.rows - t * kTileRows;
+        const BufferRsrc mask = make_buffer(a.row_mask != nullptr ? a.row_mask + t * kTileRows : nullptr,
+                                            a.row_mask != nullptr ? stage.rows : 0);
+        stage.mask = buffer_load_byte(mask, static_cast<uint32_t>(tid));
+    };
+    auto load_stage = [&](Stage& stage, int64_t t) {
+        const BufferRsrc buffer = tile_buffer(t);
 #pragma unroll
         for (int c = 0; c < kChunksPerThread; ++c) {
-            const int chunk = tid + c * kThreads;
-            const int rr = chunk / kChunksPerRow;
-            const int cc = chunk - rr * kChunksPerRow;
-            *reinterpret_cast<u32x4*>(&s_x[buf][rr * KP + 8 * cc]) = finish_x_chunk<XT, XVEC>(stage[c]);
+            load_chunk(stage, t, buffer, c);
         }
+        load_flags(stage, t);
+    };
+    auto write_chunk = [&](const Stage& stage, int buf, int c) {
+        const int chunk = tid + c * kThreads;
+        const int rr = chunk / kChunksPerRow;
+        const int cc = chunk - rr * kChunksPerRow;
+        *reinterpret_cast<u32x4*>(&s_x[buf][rr * KP + 8 * cc]) = VEC ? to_bf16_piece<XT>(stage.x[c]) : stage.x[c];
+    };
+    auto write_flags = [&](const Stage& stage, int buf) {
         if (tid < kTileRows) {
-            s_keep[buf][tid] = tid < stage_rows && (a.row_mask == nullptr || stage_mask != 0);
+            s_keep[buf][tid] = tid < stage.rows && (a.row_mask == nullptr || stage.mask != 0);
         }
     };
 
-    int64_t tile = group_index;
-    if (tile < a.tiles) {
-        load_stage(tile);
-        write_stage(0);
-    }
-    __syncthreads();
-    int buf = 0;
-    for (; tile < a.tiles; tile += group_count) {
-        const int64_t next = tile + group_count;
-        // Memory operations complete in issue order as far as the wait
-        // counter is concerned, so the order below matters: the row mask
-        // bytes (needed first) are requested before the next tile's x, and the
-        // next tile's x is consumed before this tile's y stores are issued.
+    // One tile from LDS buffer `buf`.  `stage` holds the next tile of this
+    // workgroup, loaded two tiles ago (one where the registers hold a single
+    // stage): between the MFMAs its pieces are converted into the other buffer,
+    // and each piece's registers take their piece of the tile `ahead`.  Memory
+    // operations complete in issue order as far as the wait counter is
+    // concerned and nothing here is conditional, so each wait covers that one
+    // stage only: the stage behind it and the y stores stay in flight.
+    // Without VEC, `ahead` is the next tile, loaded before the products and
+    // written after them.
+    auto step = [&](int buf, int64_t tile, Stage& stage, int64_t ahead) {
         bool keep[MB];
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
             keep[mb] = s_keep[buf][mb * 32 + (lane & 31)] != 0;
         }
-        if (next < a.tiles) {
-            load_stage(next);
-        }
-        // The FP32 bias is the accumulators' starting value (in the lower-K
-        // wave of a split slice): element 4 qd + e is feature
-        // slice * 32 + 8 qd + 4 half + e of the group.
+        // The FP32 bias is the accumulators' starting value: element 4 qd + e
+        // is feature slice * 32 + 8 qd + 4 half + e of the group.
         f32x16 acc[MB];
 #pragma unroll
         for (int qd = 0; qd < 4; ++qd) {
-            const f32x4 bias = khalf == 0 ? *reinterpret_cast<const f32x4*>(&s_bias[slice * 32 + 8 * qd + 4 * half])
-                                          : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+            const f32x4 bias = *reinterpret_cast<const f32x4*>(&s_bias[slice * 32 + 8 * qd + 4 * half]);
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
@@ -273,6 +277,7 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
         // Operand reads run one group of two K steps ahead of the MFMAs, so
         // at most eight x fragments are live next to the resident W slice.
         constexpr int kGroup = 2;
+        constexpr int kGroups = KSTEPS / kGroup;
         u32x4 xb[2][kGroup][MB];
         auto read_group = [&](int slot, int k_base) {
 #pragma unroll
@@ -280,55 +285,53 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) {
                     xb[slot][ks][mb] = *reinterpret_cast<const u32x4*>(
-                        &s_x[buf][(mb * 32 + (lane & 31)) * KP + 16 * (kofs + k_base + ks) + 8 * half]);
+                        &s_x[buf][(mb * 32 + (lane & 31)) * KP + 16 * (k_base + ks) + 8 * half]);
                 }
             }
         };
-        // A slice wholly past the output width (the last column group of an
-        // output that is not a whole number of groups: 384 or 640 columns)
-        // skips its products, which would only multiply zero weights, and
-        // leaves its SIMD to the other wave; it still stages, stores and
-        // meets every barrier.
-        if (slice_live) {
-            read_group(0, 0);
-#pragma unroll
-            for (int k2 = 0; k2 < KW; k2 += kGroup) {
-                const int slot = (k2 / kGroup) & 1;
-                if (k2 + kGroup < KW) {
-                    read_group(slot ^ 1, k2 + kGroup);
-                }
-#pragma unroll
-                for (int ks = 0; ks < kGroup; ++ks) {
-#pragma unroll
-                    for (int mb = 0; mb < MB; ++mb) {
-                        acc[mb] = mfma32x32x16(wreg[0][k2 + ks], xb[slot][ks][mb], acc[mb]);
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
+        const BufferRsrc buffer = tile_buffer(ahead);
+        if constexpr (!VEC) {
+            load_stage(stage, ahead);
         }
-        if constexpr (KSPLIT == 2) {
-            // The upper-K waves hand their accumulators to the lower-K waves
-            // of the same slice, which add them (lower + upper) and finish.
-            if (khalf == 1) {
+        read_group(0, 0);
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+            const int slot = g & 1;
+            if (g + 1 < kGroups) {
+                read_group(slot ^ 1, kGroup * (g + 1));
+            }
+#pragma unroll
+            for (int ks = 0; ks < kGroup; ++ks) {
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        s_part[((slice * MB + mb) * 16 + i) * 64 + lane] = acc[mb][i];
-                    }
+                    acc[mb] = mfma32x32x16(wreg[0][kGroup * g + ks], xb[slot][ks][mb], acc[mb]);
                 }
             }
-            __syncthreads();
-            if (khalf == 0) {
+            // This group's share of the next tile's pieces.
 #pragma unroll
-                for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        acc[mb][i] += s_part[((slice * MB + mb) * 16 + i) * 64 + lane];
-                    }
+            for (int c = 0; c < kChunksPerThread; ++c) {
+                if (VEC && c * kGroups / kChunksPerThread == g) {
+                    write_chunk(stage, buf ^ 1, c);
+                    load_chunk(stage, ahead, buffer, c);
                 }
             }
+            __builtin_amdgcn_sched_group_barrier(kSchedDsRead, kGroup * MB, 0);
+#pragma unroll
+            for (int i = 0; i < kGroup * MB; ++i) {
+                __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(kSchedValu, 6, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (VEC) {
+            write_flags(stage, buf ^ 1);
+            load_flags(stage, ahead);
+        } else {
+#pragma unroll
+            for (int c = 0; c < kChunksPerThread; ++c) {
+                write_chunk(stage, buf ^ 1, c);
+            }
+            write_flags(stage, buf ^ 1);
         }
         // y^T block: lane holds row m = lane%32 of the 32-row block and
         // features n0 + 8 q + 4 half + r for q, r in 0..3.  The tile is
@@ -336,9 +339,6 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
         // each store instruction covers whole contiguous row segments.
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
-            if (khalf != 0) {
-                break;   // wave-uniform: the upper-K waves have handed over
-            }
             const int mr = mb * 32 + (lane & 31);
             if (__ballot(keep[mb]) != ~0ull) {
 #pragma unroll
@@ -365,13 +365,10 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
             }
         }
         __syncthreads();
-        if (next < a.tiles) {
-            write_stage(buf ^ 1);
-        }
-        if (a.y_vector) {
+        const int64_t col0 = cg * kGroupColumns;
+        if constexpr (VEC) {
             // 16-byte pieces through a raw buffer over the tile's valid rows:
             // pieces past the matrix are dropped without a branch.
-            const int64_t col0 = cg * kGroupColumns;
             const int64_t tile_rows = a.rows - tile * kTileRows < kTileRows ? a.rows - tile * kTileRows : kTileRows;
             const BufferRsrc ybuf = make_buffer(static_cast<uint16_t*>(a.y) + tile * kTileRows * N, 2 * tile_rows * N);
 #pragma unroll
@@ -384,7 +381,6 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
                                n < N ? 2u * static_cast<uint32_t>(mr * N + n) : kOutOfRange);
             }
         } else {
-            const int64_t col0 = cg * kGroupColumns;
 #pragma unroll
             for (int i = 0; i < kStoreChunks; ++i) {
                 const int chunk = tid + i * kThreads;
@@ -409,7 +405,40 @@ __global__ __launch_bounds__(linear_waves<KSTEPS>() * 64) void linear_kernel(Lin
             }
         }
         __syncthreads();
-        buf ^= 1;
+    };
+
+    int64_t tile = group_index;
+    if (tile >= a.tiles) {
+        return;
+    }
+    // Stages of x in flight: two where the registers hold them beside W.
+    constexpr int kSets = VEC && KSTEPS <= 32 ? 2 : 1;
+    constexpr int kAhead = VEC ? kSets + 1 : 1;
+    Stage sets[kSets];
+    load_stage(sets[0], tile);
+    if constexpr (kSets == 2) {
+        load_stage(sets[1], tile + group_count);
+    }
+#pragma unroll
+    for (int c = 0; c < kChunksPerThread; ++c) {
+        write_chunk(sets[0], 0, c);
+    }
+    write_flags(sets[0], 0);
+    if constexpr (VEC) {
+        load_stage(sets[0], tile + kSets * group_count);
+    }
+    __syncthreads();
+    for (;;) {
+        step(0, tile, sets[kSets - 1], tile + kAhead * group_count);
+        tile += group_count;
+        if (tile >= a.tiles) {
+            break;
+        }
+        step(1, tile, sets[0], tile + kAhead * group_count);
+        tile += group_count;
+        if (tile >= a.tiles) {
+            break;
+        }
     }
 }
 
@@ -626,21 +655,21 @@ __global__ __launch_bounds__(kStreamThreads) void linear_stream_kernel(LinearArg
     }
 }
 
-template <int KSTEPS, bool XVEC>
+template <int KSTEPS, bool VEC>
 static hipError_t launch_linear_kv(const LinearArgs& a, int x_dtype, int y_dtype, dim3 grid,
                                    hipStream_t stream) {
-    const dim3 block(linear_waves<KSTEPS>() * 64);
+    const dim3 block(kLinearWaves * 64);
     if (x_dtype == LSSO_HIP_F16) {
         if (y_dtype == LSSO_HIP_F16) {
-            dispatch(linear_kernel<KSTEPS, LSSO_HIP_F16, LSSO_HIP_F16, XVEC>, grid, block, stream, a);
+            dispatch(linear_kernel<KSTEPS, LSSO_HIP_F16, LSSO_HIP_F16, VEC>, grid, block, stream, a);
         } else {
-            dispatch(linear_kernel<KSTEPS, LSSO_HIP_F16, LSSO_HIP_BF16, XVEC>, grid, block, stream, a);
+            dispatch(linear_kernel<KSTEPS, LSSO_HIP_F16, LSSO_HIP_BF16, VEC>, grid, block, stream, a);
         }
     } else {
         if (y_dtype == LSSO_HIP_F16) {
-            dispatch(linear_kernel<KSTEPS, LSSO_HIP_BF16, LSSO_HIP_F16, XVEC>, grid, block, stream, a);
+            dispatch(linear_kernel<KSTEPS, LSSO_HIP_BF16, LSSO_HIP_F16, VEC>, grid, block, stream, a);
         } else {
-            dispatch(linear_kernel<KSTEPS, LSSO_HIP_BF16, LSSO_HIP_BF16, XVEC>, grid, block, stream, a);
+            dispatch(linear_kernel<KSTEPS, LSSO_HIP_BF16, LSSO_HIP_BF16, VEC>, grid, block, stream, a);
         }
     }
     return hipGetLastError();
@@ -649,7 +678,9 @@ static hipError_t launch_linear_kv(const LinearArgs& a, int x_dtype, int y_dtype
 template <int KSTEPS>
 static hipError_t launch_linear_k(const LinearArgs& a, int x_dtype, int y_dtype, dim3 grid,
                                   hipStream_t stream) {
-    return a.x_vector ? launch_linear_kv<KSTEPS, true>(a, x_dtype, y_dtype, grid, stream)
+    // The vector form's 32-bit offsets reach one tile's rows.
+    const bool vec = a.x_vector && a.y_vector && a.x_stride < (1 << 23) && a.out_features < (1 << 23);
+    return vec ? launch_linear_kv<KSTEPS, true>(a, x_dtype, y_dtype, grid, stream)
                       : launch_linear_kv<KSTEPS, false>(a, x_dtype, y_dtype, grid, stream);
 }
 
