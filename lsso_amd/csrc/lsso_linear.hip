@@ -49,6 +49,7 @@ constexpr int kLinearWaves = 8;
 constexpr int kSchedValu = 0x2;
 constexpr int kSchedMfma = 0x8;
 constexpr int kSchedDsRead = 0x100;
+constexpr int kSchedDsWrite = 0x200;
 
 // Tier 0 is the K-streaming kernel (any in_features above 640).
 int linear_tile_rows(int k_steps) { return k_steps == 0 ? kStreamRowsHost : (k_steps <= 24 ? 64 : 32); }
@@ -446,30 +447,46 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
 // K-streaming tier (in_features > 640): the W rows no longer fit the waves'
 // registers, so both operands stream through LDS.  A workgroup of four waves
 // computes a 128-row x 128-column output tile; each wave a 64 x 64 quarter
-// (2 x 2 blocks of v_mfma_f32_32x32x16_bf16 on y^T = W x^T).  K is taken in
-// stages of 64: the x and W stages of k-tile t + 1 are loaded into registers
-// (W converted from FP32 to BF16, x from FP16 to BF16, round to nearest even)
-// while k-tile t is multiplied from the other LDS buffer.  The K order is one
-// FP32 chain per output, ascending.  Row tiles sharing x are dealt to one XCD.
+// (2 x 2 blocks of v_mfma_f32_32x32x16_bf16 on y^T = W x^T).  The K order is
+// one FP32 chain per output, ascending.  Row tiles sharing x are dealt to one
+// XCD.
+//
+// Bound: the matrix cores and LDS (a stage's fragments and writes take about
+// 1.5 times its MFMA cycles), where enough workgroups share a CU to cover each
+// other's prologue and epilogue.  K is taken in stages of 32: two stages of
+// loads are in flight in registers while a third is multiplied, and the next
+// stage's conversions (W FP32 to BF16, x FP16 to BF16, round to nearest even)
+// and LDS writes run between its MFMAs.  The output tile is staged in the
+// operands' LDS, which leaves 40 KB per workgroup and three workgroups per CU;
+// the former kernel (64-wide stages, one in flight, 107 KB) had one.  (FP16 x
+// keeps two: at three, its conversions spill inside the loop, and a scratch
+// load there waits for the loads in flight.)  Before and now (us, graph launch
+// included): 12,608 x 768 -> 1,344 91 / 56, 8,192 x 768 -> 1,344 57 / 36, x 1,344
+// -> 768 59 / 36, x 768 -> 768 38 / 26.
 constexpr int kStreamRows = 128;
 constexpr int kStreamCols = 128;
-constexpr int kStreamK = 64;
+constexpr int kStreamK = 32;
 constexpr int kStreamThreads = 256;
 
-template <int XT, int YT>
-__global__ __launch_bounds__(kStreamThreads) void linear_stream_kernel(LinearArgs a) {
-    constexpr int KP = kStreamK + 8;                 // LDS row pitch (bf16)
-    constexpr int kChunks = kStreamRows * (kStreamK / 8) / kStreamThreads;   // 16-byte pieces per thread
+// VEC: whole 16-byte pieces of x, W and y.
+template <int XT, int YT, bool VEC>
+__global__ __launch_bounds__(kStreamThreads, VEC && XT == LSSO_HIP_BF16 ? 3 : 2) void linear_stream_kernel(LinearArgs a) {
+    constexpr int KP = kStreamK + 8;                 // LDS row pitch (bf16): 16 rows' 16-byte reads cover all banks
     constexpr int YP = kStreamCols + 8;
-    __shared__ __attribute__((aligned(16))) uint16_t s_x[2][kStreamRows * KP];
-    __shared__ __attribute__((aligned(16))) uint16_t s_w[2][kStreamCols * KP];
-    __shared__ __attribute__((aligned(16))) uint16_t s_y[kStreamRows * YP];
+    constexpr int kXPieces = kStreamRows * kStreamK / 8 / kStreamThreads;   // 16-byte pieces per thread and stage
+    constexpr int kWPieces = kStreamCols * kStreamK / 4 / kStreamThreads;
+    constexpr int kXRows = kStreamThreads / (kStreamK / 8);   // rows between a thread's pieces
+    constexpr int kWRows = kStreamThreads / (kStreamK / 4);
+    constexpr int kOperand = kStreamRows * KP;
+    static_assert(kStreamRows == kStreamCols && kStreamRows * YP <= 4 * kOperand, "the output tile fits the operands'");
+    // Two buffers of (x, W); afterwards the output tile.
+    __shared__ __attribute__((aligned(16))) uint16_t s_t[4 * kOperand];
     __shared__ __attribute__((aligned(16))) float s_bias[kStreamCols];
     __shared__ int s_keep[kStreamRows];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5;
     const int64_t M = a.rows;
     const int64_t N = a.out_features;
@@ -485,76 +502,76 @@ __global__ __launch_bounds__(kStreamThreads) void linear_stream_kernel(LinearArg
     }
     const int64_t m0 = mt * kStreamRows;
     const int64_t n0 = nt * kStreamCols;
-    for (int c = tid; c < kStreamCols; c += kStreamThreads) {
-        const int64_t n = n0 + c;
-        s_bias[c] = (a.bias != nullptr && n < N) ? a.bias[n] : 0.0f;
-    }
-    for (int r = tid; r < kStreamRows; r += kStreamThreads) {
-        const int64_t m = m0 + r;
-        s_keep[r] = m < M && (a.row_mask == nullptr || a.row_mask[m] != 0);
-    }
 
-    const uint16_t* x = static_cast<const uint16_t*>(a.x);
-    u32x4 xs[kChunks];
-    f32x4 ws[kChunks][2];
-    // Piece i of this thread: row (tid + 256 i) / 8, columns 8 ((tid + 256 i) % 8) .. + 7.
-    auto load = [&](int64_t k0) {
+    struct Stage {
+        u32x4 x[kXPieces];
+        f32x4 w[kWPieces];
+    };
+    const uint16_t* x = static_cast<const uint16_t*>(a.x) + m0 * a.x_stride;
+    const float* w = a.weight + n0 * K;
+    const int x_row = tid / (kStreamK / 8);
+    const int x_k = 8 * (tid % (kStreamK / 8));
+    const int w_row = tid / (kStreamK / 4);
+    const int w_k = 4 * (tid % (kStreamK / 4));
+    const uint32_t x_at = 2u * static_cast<uint32_t>(x_row * static_cast<int>(a.x_stride) + x_k);
+    const uint32_t w_at = 4u * static_cast<uint32_t>(w_row * static_cast<int>(K) + w_k);
+    const uint32_t x_step = 2u * static_cast<uint32_t>(kXRows * static_cast<int>(a.x_stride));
+    const uint32_t w_step = 4u * static_cast<uint32_t>(kWRows * static_cast<int>(K));
+    auto load = [&](Stage& stage, int64_t k0) {
+        if constexpr (VEC) {
+            // Rows past the matrices end the buffers; columns past K get an
+            // offset beyond them.
+            const BufferRsrc xb = make_buffer(x + k0, 2 * ((M - m0) * a.x_stride - k0));
+            const BufferRsrc wb = make_buffer(w + k0, 4 * ((N - n0) * K - k0));
+            const uint32_t xo = k0 + x_k < K ? x_at : kOutOfRange;
+            const uint32_t wo = k0 + w_k < K ? w_at : kOutOfRange;
 #pragma unroll
-        for (int i = 0; i < kChunks; ++i) {
-            const int piece = tid + i * kStreamThreads;
-            const int r = piece >> 3;
-            const int64_t k = k0 + 8 * (piece & 7);
-            const int64_t m = m0 + r;
-            const int64_t n = n0 + r;
-            if (a.x_vector) {
-                const bool live = m < M && k < K;
-                xs[i] = live ? *reinterpret_cast<const u32x4*>(x + m * a.x_stride + k) : u32x4{};
-            } else {
-                uint32_t v[4];
+            for (int i = 0; i < kXPieces; ++i) {
+                stage.x[i] = buffer_load16(xb, xo + i * x_step);
+            }
+#pragma unroll
+            for (int i = 0; i < kWPieces; ++i) {
+                stage.w[i] = __builtin_bit_cast(f32x4, buffer_load16(wb, wo + i * w_step));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kXPieces; ++i) {
+                const int64_t r = x_row + kXRows * i;
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
-                    const uint32_t lo = (m < M && k + 2 * p < K) ? x[m * a.x_stride + k + 2 * p] : 0u;
-                    const uint32_t hi = (m < M && k + 2 * p + 1 < K) ? x[m * a.x_stride + k + 2 * p + 1] : 0u;
-                    v[p] = lo | (hi << 16);
+                    const int64_t k = k0 + x_k + 2 * p;
+                    const uint32_t lo = (m0 + r < M && k < K) ? x[r * a.x_stride + k] : 0u;
+                    const uint32_t hi = (m0 + r < M && k + 1 < K) ? x[r * a.x_stride + k + 1] : 0u;
+                    stage.x[i][p] = lo | (hi << 16);
                 }
-                xs[i] = (u32x4){v[0], v[1], v[2], v[3]};
             }
-            if (a.w_vector) {
-                const bool live0 = n < N && k < K;
-                const bool live1 = n < N && k + 4 < K;
-                ws[i][0] = live0 ? *reinterpret_cast<const f32x4*>(a.weight + n * K + k) : f32x4{};
-                ws[i][1] = live1 ? *reinterpret_cast<const f32x4*>(a.weight + n * K + k + 4) : f32x4{};
-            } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const bool live = n < N && k + e < K;
-                    ws[i][e / 4][e % 4] = live ? a.weight[n * K + k + e] : 0.0f;
+            for (int i = 0; i < kWPieces; ++i) {
+                const int64_t r = w_row + kWRows * i;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int64_t k = k0 + w_k + e;
+                    stage.w[i][e] = (n0 + r < N && k < K) ? w[r * K + k] : 0.0f;
                 }
             }
         }
     };
-    auto store = [&](int buf) {
+    auto commit = [&](const Stage& stage, int buf) {
+        uint16_t* s_x = s_t + 2 * buf * kOperand;
+        uint16_t* s_w = s_x + kOperand;
 #pragma unroll
-        for (int i = 0; i < kChunks; ++i) {
-            const int piece = tid + i * kStreamThreads;
-            const int r = piece >> 3;
-            const int c = 8 * (piece & 7);
-            u32x4 xv = xs[i];
-            if constexpr (XT == LSSO_HIP_F16) {
+        for (int i = 0; i < kXPieces; ++i) {
+            *reinterpret_cast<u32x4*>(s_x + (x_row + kXRows * i) * KP + x_k) = to_bf16_piece<XT>(stage.x[i]);
+        }
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    xv[p] = pack_bf16(f16_lo(xv[p]), f16_hi(xv[p]));
-                }
-            }
-            *reinterpret_cast<u32x4*>(&s_x[buf][r * KP + c]) = xv;
-            const u32x4 wv = {pack_bf16(ws[i][0][0], ws[i][0][1]), pack_bf16(ws[i][0][2], ws[i][0][3]),
-                              pack_bf16(ws[i][1][0], ws[i][1][1]), pack_bf16(ws[i][1][2], ws[i][1][3])};
-            *reinterpret_cast<u32x4*>(&s_w[buf][r * KP + c]) = wv;
+        for (int i = 0; i < kWPieces; ++i) {
+            const u32x2 packed = {pack_bf16(stage.w[i][0], stage.w[i][1]), pack_bf16(stage.w[i][2], stage.w[i][3])};
+            *reinterpret_cast<u32x2*>(s_w + (w_row + kWRows * i) * KP + w_k) = packed;
         }
     };
 
-    const int wn = wave & 1;    // 64-column half of the tile
-    const int wm = wave >> 1;   // 64-row half of the tile
+    const int wn = 64 * (wave & 1);    // this wave's columns and rows of the tile
+    const int wm = 64 * (wave >> 1);
     f32x16 acc[2][2];
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
@@ -566,52 +583,83 @@ __global__ __launch_bounds__(kStreamThreads) void linear_stream_kernel(LinearArg
             }
         }
     }
-    const int64_t k_tiles = (K + kStreamK - 1) / kStreamK;
-    load(0);
-    store(0);
-    __syncthreads();
-    for (int64_t kt = 0; kt < k_tiles; ++kt) {
-        const int buf = static_cast<int>(kt & 1);
-        if (kt + 1 < k_tiles) {
-            load((kt + 1) * kStreamK);
-        }
-        const uint16_t* wt = s_w[buf];
-        const uint16_t* xt = s_x[buf];
+    const int fragment = (lane & 31) * KP + 8 * half;
+    auto step = [&](int buf, Stage& stage, int64_t ahead) {
+        const uint16_t* xt = s_t + 2 * buf * kOperand + wm * KP + fragment;
+        const uint16_t* wt = s_t + (2 * buf + 1) * kOperand + wn * KP + fragment;
+        u32x4 wf[2][2];
+        u32x4 xf[2][2];
 #pragma unroll
-        for (int kk = 0; kk < kStreamK / 16; ++kk) {
-            u32x4 wf[2];
-            u32x4 xf[2];
+        for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
-                wf[b] = *reinterpret_cast<const u32x4*>(&wt[(wn * 64 + b * 32 + (lane & 31)) * KP + 16 * kk + 8 * half]);
-                xf[b] = *reinterpret_cast<const u32x4*>(&xt[(wm * 64 + b * 32 + (lane & 31)) * KP + 16 * kk + 8 * half]);
+                wf[kk][b] = *reinterpret_cast<const u32x4*>(wt + 32 * b * KP + 16 * kk);
+                xf[kk][b] = *reinterpret_cast<const u32x4*>(xt + 32 * b * KP + 16 * kk);
+            }
+        }
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            if (kk == 1) {
+                commit(stage, buf ^ 1);
+                load(stage, ahead);
             }
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
                 for (int mb = 0; mb < 2; ++mb) {
-                    acc[nb][mb] = mfma32x32x16(wf[nb], xf[mb], acc[nb][mb]);
+                    acc[nb][mb] = mfma32x32x16(wf[kk][nb], xf[kk][mb], acc[nb][mb]);
                 }
             }
         }
-        if (kt + 1 < k_tiles) {
-            store(buf ^ 1);
+        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(kSchedValu, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedDsWrite, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
         }
         __syncthreads();
+    };
+    Stage even;
+    Stage odd;
+    load(even, 0);
+    load(odd, kStreamK);
+    for (int c = tid; c < kStreamCols; c += kStreamThreads) {
+        const int64_t n = n0 + c;
+        s_bias[c] = (a.bias != nullptr && n < N) ? a.bias[n] : 0.0f;
+    }
+    for (int r = tid; r < kStreamRows; r += kStreamThreads) {
+        const int64_t m = m0 + r;
+        s_keep[r] = m < M && (a.row_mask == nullptr || a.row_mask[m] != 0);
+    }
+    commit(even, 0);
+    load(even, 2 * kStreamK);
+    __syncthreads();
+    // An odd last stage is followed by one of zeros: a second exit from the
+    // loop would make it carry copies of the accumulators.
+    for (int64_t k0 = 0; k0 < K; k0 += 2 * kStreamK) {
+        step(0, odd, k0 + 3 * kStreamK);
+        step(1, even, k0 + 4 * kStreamK);
     }
 
     // Epilogue: bias, row mask, one rounding; the tile goes out through LDS
     // as 16-byte pieces of whole row segments.  Lane (half, m) of block
     // (nb, mb) holds row m of the 32-row block and features 8 q + 4 half + r.
+    uint16_t* s_y = s_t;
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb) {
-            const int mr = wm * 64 + mb * 32 + (lane & 31);
+            const int mr = wm + mb * 32 + (lane & 31);
             const bool keep = s_keep[mr] != 0;
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
-                const int c = wn * 64 + nb * 32 + 8 * qd + 4 * half;
+                const int c = wn + nb * 32 + 8 * qd + 4 * half;
                 const f32x4 bias = *reinterpret_cast<const f32x4*>(&s_bias[c]);
                 const float v0 = keep ? acc[nb][mb][4 * qd + 0] + bias[0] : 0.0f;
                 const float v1 = keep ? acc[nb][mb][4 * qd + 1] + bias[1] : 0.0f;
@@ -641,7 +689,7 @@ __global__ __launch_bounds__(kStreamThreads) void linear_stream_kernel(LinearArg
         if (m < M && n < N) {
             const u32x4 v = *reinterpret_cast<const u32x4*>(&s_y[mr * YP + c8]);
             uint16_t* dst = static_cast<uint16_t*>(a.y) + m * N + n;
-            if (a.y_vector) {
+            if (VEC) {
                 *reinterpret_cast<u32x4*>(dst) = v;
             } else {
 #pragma unroll
@@ -692,17 +740,24 @@ hipError_t launch_linear(const LinearArgs& a, int k_steps, int x_dtype, int y_dt
         const int64_t rounds = (a.tiles + kXcds - 1) / kXcds;
         const dim3 grid(static_cast<unsigned>(rounds * kXcds * a.column_groups));
         const dim3 block(kStreamThreads);
+        // The vector form's 32-bit offsets reach one tile's rows.
+        const bool vec = a.x_vector && a.w_vector && a.y_vector && a.x_stride < (1 << 23) && a.in_features < (1 << 22);
+        const auto run = [&](auto kernel) { dispatch(kernel, grid, block, stream, a); };
         if (x_dtype == LSSO_HIP_F16) {
             if (y_dtype == LSSO_HIP_F16) {
-                dispatch(linear_stream_kernel<LSSO_HIP_F16, LSSO_HIP_F16>, grid, block, stream, a);
+                vec ? run(linear_stream_kernel<LSSO_HIP_F16, LSSO_HIP_F16, true>)
+                    : run(linear_stream_kernel<LSSO_HIP_F16, LSSO_HIP_F16, false>);
             } else {
-                dispatch(linear_stream_kernel<LSSO_HIP_F16, LSSO_HIP_BF16>, grid, block, stream, a);
+                vec ? run(linear_stream_kernel<LSSO_HIP_F16, LSSO_HIP_BF16, true>)
+                    : run(linear_stream_kernel<LSSO_HIP_F16, LSSO_HIP_BF16, false>);
             }
         } else {
             if (y_dtype == LSSO_HIP_F16) {
-                dispatch(linear_stream_kernel<LSSO_HIP_BF16, LSSO_HIP_F16>, grid, block, stream, a);
+                vec ? run(linear_stream_kernel<LSSO_HIP_BF16, LSSO_HIP_F16, true>)
+                    : run(linear_stream_kernel<LSSO_HIP_BF16, LSSO_HIP_F16, false>);
             } else {
-                dispatch(linear_stream_kernel<LSSO_HIP_BF16, LSSO_HIP_BF16>, grid, block, stream, a);
+                vec ? run(linear_stream_kernel<LSSO_HIP_BF16, LSSO_HIP_BF16, true>)
+                    : run(linear_stream_kernel<LSSO_HIP_BF16, LSSO_HIP_BF16, false>);
             }
         }
         return hipGetLastError();
