@@ -404,6 +404,34 @@ int lsso_hip_layer_forward_train(const lsso_hip_mixer_shape* shape,
                                  size_t workspace_bytes,
                                  void* stream);
 
+/* Device scratch bytes needed by lsso_hip_layer_backward. */
+int lsso_hip_layer_backward_workspace_bytes(const lsso_hip_mixer_shape* shape, int positions_mode,
+                                            size_t* bytes);
+
+/* Backward of lsso_hip_layer_forward_train in one call: the output
+ * projection's VJP (lsso_hip_linear with the transposed weight,
+ * lsso_hip_linear_weight_grad), the mixer's (lsso_hip_mixer_backward_ex) and
+ * the input projection's, each bitwise that of the separate calls.
+ * grad_y: [B * N, D] of grad_y_dtype with row stride grad_y_stride elements;
+ * x, packed, mixed, tape: the forward's input and what it wrote (contiguous);
+ * row_mask, positions and counts as in the forward.  Any of the gradients may
+ * be NULL and is then not computed; grad_x has x's dtype, the parameters'
+ * gradients are float32, written and not accumulated.  workspace: at least
+ * lsso_hip_layer_backward_workspace_bytes, 256-byte aligned.
+ * Replaces: the backward of K1 + forward_train + K5
+ * (lsso/ball/reference.py:205-247, lsso/ball/cuda.py:256-280). */
+int lsso_hip_layer_backward(const lsso_hip_mixer_shape* shape, const void* grad_y, int grad_y_dtype,
+                            int64_t grad_y_stride, const void* x, int x_dtype,
+                            const float* in_weight, const uint8_t* row_mask, const void* packed,
+                            const void* mixed, const float* core_base_raw,
+                            const float* core_drive_weight, const float* eta_raw,
+                            const float* inverse_frequency, const float* centered_positions,
+                            int positions_mode, const float* valid_counts, const float* tape,
+                            const float* out_weight, void* grad_x, float* grad_in_weight,
+                            float* grad_in_bias, float* grad_base, float* grad_drive,
+                            float* grad_eta, float* grad_out_weight, float* grad_out_bias,
+                            void* workspace, size_t workspace_bytes, void* stream);
+
 /* Types of the position ids of lsso_hip_center_positions. */
 #define LSSO_HIP_IDS_NONE 0 /* 0 .. length - 1 */
 #define LSSO_HIP_IDS_I32 1

@@ -13,6 +13,7 @@ not loaded or an input is outside the native contract.
 from __future__ import annotations
 
 import ctypes
+from functools import lru_cache
 import os
 from pathlib import Path
 from threading import Lock
@@ -31,6 +32,7 @@ _INVERSE_FREQUENCY: dict[int, ctypes.Array] = {}
 
 _F16 = 1
 _BF16 = 2
+_DTYPE_CODES = {torch.float16: _F16, torch.bfloat16: _BF16}
 _POSITIONS_DEFAULT = 0
 _POSITIONS_SHARED = 1
 _POSITIONS_BATCHED = 2
@@ -62,6 +64,8 @@ _SYMBOLS = (
     "lsso_hip_layer_forward_timed",
     "lsso_hip_project_mix_forward",
     "lsso_hip_layer_forward_train",
+    "lsso_hip_layer_backward_workspace_bytes",
+    "lsso_hip_layer_backward",
     "lsso_hip_linear_weight_grad_workspace_bytes",
     "lsso_hip_linear_weight_grad",
 )
@@ -177,6 +181,15 @@ def _declare(library: ctypes.CDLL) -> None:
     ]  # shape, x, x_dtype, in_weight, in_bias, row_mask, base, drive, eta, inv_freq, positions,
     #    mode, counts, out_weight, out_bias, packed, mixed, tape, y, y_dtype, workspace,
     #    workspace_bytes, stream
+    library.lsso_hip_layer_backward_workspace_bytes.restype = ctypes.c_int
+    library.lsso_hip_layer_backward_workspace_bytes.argtypes = [shape_p, ctypes.c_int, size_p]
+    library.lsso_hip_layer_backward.restype = ctypes.c_int
+    library.lsso_hip_layer_backward.argtypes = [
+        shape_p, vp, ctypes.c_int, i64, vp, ctypes.c_int, vp, vp, vp, vp, vp, vp, vp, vp, vp, ctypes.c_int, vp, vp,
+        vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, ctypes.c_size_t, vp,
+    ]  # shape, grad_y, dtype, stride, x, x_dtype, in_weight, row_mask, packed, mixed, base, drive, eta, inv_freq,
+    #    positions, mode, counts, tape, out_weight, grads (x, in_weight, in_bias, base, drive, eta, out_weight,
+    #    out_bias), workspace, workspace_bytes, stream
 
 
 def default_library_path() -> Path:
@@ -319,15 +332,50 @@ def _stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def _inverse_frequency(rank: int) -> ctypes.Array:
-    """Host FP32 frequencies computed exactly as the reference does (reference.py:704-707)."""
+def _launch(entry, device: torch.device, *arguments, after: tuple = ()) -> int:
+    """entry(*arguments, current stream of ``device``, *after) with that
+    device current; the device is only switched where it is not (the switch
+    and the stream object cost more host time than a launch)."""
+
+    index = device.index
+    if torch.cuda.current_device() == index:
+        return entry(*arguments, torch._C._cuda_getCurrentRawStream(index), *after)
+    with torch.cuda.device(device):
+        return entry(*arguments, torch._C._cuda_getCurrentRawStream(index), *after)
+
+
+@lru_cache(maxsize=1024)
+def _plan_size(query: str, mode: int | None, *shape: int) -> int:
+    """A size query of the library for a geometry: it depends on these
+    integers alone, and a program asks for the same few on every call."""
+
+    library = _library()
+    arguments = [ctypes.byref(MixerShape(*shape))] + ([] if mode is None else [mode])
+    size = ctypes.c_size_t()
+    _check(getattr(library, query)(*arguments, ctypes.byref(size)), library)
+    return size.value
+
+
+@lru_cache(maxsize=1024)
+def _layer_geometry_supported(*shape: int) -> bool:
+    """lsso_hip_layer_supported of (batch, length, heads, rank, head_dim)."""
+
+    library = _library()
+    status = library.lsso_hip_layer_supported(ctypes.byref(MixerShape(*shape)))
+    if status < 0:
+        _check(status, library)
+    return status == 1
+
+
+def _inverse_frequency(rank: int) -> int:
+    """Address of the host FP32 frequencies, computed exactly as the reference does (reference.py:704-707)."""
 
     cached = _INVERSE_FREQUENCY.get(rank)
     if cached is None:
         values = rotary_inverse_frequency(rank, torch.float32).tolist()
         cached = (ctypes.c_float * len(values))(*values)
-        _INVERSE_FREQUENCY[rank] = cached
-    return cached
+        cached = _INVERSE_FREQUENCY.setdefault(rank, cached)
+    return ctypes.addressof(cached)
 
 
 def _require_device_tensor(value: torch.Tensor, name: str, device: torch.device) -> None:
@@ -335,6 +383,10 @@ def _require_device_tensor(value: torch.Tensor, name: str, device: torch.device)
         raise RuntimeError(f"{name} must be a CUDA (ROCm device) tensor")
     if value.device != device:
         raise RuntimeError(f"{name} must share projected.device() (got {value.device} vs {device})")
+
+
+def _dims(shape: MixerShape) -> tuple[int, int, int, int, int]:
+    return shape.batch, shape.length, shape.heads, shape.rank, shape.head_dim
 
 
 def _validate_mixer(
@@ -474,11 +526,12 @@ def center_positions(
     shared = rows == 1 and valid_mask is None and position_ids.dim() == 1
     centered = torch.empty((length,) if shared else (batch, length), dtype=torch.float32, device=device)
     library = _library()
-    with torch.cuda.device(device):
-        status = library.lsso_hip_center_positions(
-            mask_ptr, ids, kind, batch_stride, token_stride, rows, length, centered.data_ptr(),
-            None if counts is None else counts.data_ptr(), _stream(device),
-        )
+    status = _launch(
+        library.lsso_hip_center_positions,
+        device,
+        mask_ptr, ids, kind, batch_stride, token_stride, rows, length, centered.data_ptr(),
+        None if counts is None else counts.data_ptr(),
+    )
     _check(status, library)
     return centered, counts
 
@@ -497,34 +550,32 @@ def _mixer_forward(
         projected, core_base_raw, core_drive_weight, eta_raw, centered_positions, valid_counts
     )
     device = projected.device
-    workspace_bytes = ctypes.c_size_t()
-    _check(library.lsso_hip_mixer_workspace_bytes(ctypes.byref(shape), mode, ctypes.byref(workspace_bytes)), library)
+    workspace_bytes = _plan_size("lsso_hip_mixer_workspace_bytes", mode, *_dims(shape))
     output = torch.empty(
         (shape.batch, shape.length, shape.heads * shape.head_dim), dtype=torch.bfloat16, device=device
     )
-    workspace = torch.empty(workspace_bytes.value, dtype=torch.uint8, device=device)
+    workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device)
     tape = None
     if record_tape:
-        floats = ctypes.c_size_t()
-        _check(library.lsso_hip_mixer_tape_floats(ctypes.byref(shape), ctypes.byref(floats)), library)
-        tape = torch.empty(floats.value, dtype=torch.float32, device=device)
-    with torch.cuda.device(device):
-        status = library.lsso_hip_mixer_forward(
-            ctypes.byref(shape),
-            projected.data_ptr(),
-            core_base_raw.data_ptr(),
-            core_drive_weight.data_ptr(),
-            eta_raw.data_ptr(),
-            ctypes.cast(_inverse_frequency(shape.rank), ctypes.c_void_p),
-            None if centered_positions is None else centered_positions.data_ptr(),
-            mode,
-            None if valid_counts is None else valid_counts.data_ptr(),
-            output.data_ptr(),
-            None if tape is None else tape.data_ptr(),
-            workspace.data_ptr(),
-            workspace_bytes.value,
-            _stream(device),
-        )
+        floats = _plan_size("lsso_hip_mixer_tape_floats", None, *_dims(shape))
+        tape = torch.empty(floats, dtype=torch.float32, device=device)
+    status = _launch(
+        library.lsso_hip_mixer_forward,
+        device,
+        ctypes.byref(shape),
+        projected.data_ptr(),
+        core_base_raw.data_ptr(),
+        core_drive_weight.data_ptr(),
+        eta_raw.data_ptr(),
+        _inverse_frequency(shape.rank),
+        None if centered_positions is None else centered_positions.data_ptr(),
+        mode,
+        None if valid_counts is None else valid_counts.data_ptr(),
+        output.data_ptr(),
+        None if tape is None else tape.data_ptr(),
+        workspace.data_ptr(),
+        workspace_bytes,
+    )
     _check(status, library)
     return output, tape
 
@@ -610,43 +661,38 @@ def backward(
     _require_device_tensor(grad_output, "grad_output", device)
     _require_device_tensor(tape, "tape", device)
     grad_output = grad_output.contiguous()
-    floats = ctypes.c_size_t()
-    _check(library.lsso_hip_mixer_tape_floats(ctypes.byref(shape), ctypes.byref(floats)), library)
-    if tape.dtype != torch.float32 or tape.numel() != floats.value or not tape.is_contiguous():
+    floats = _plan_size("lsso_hip_mixer_tape_floats", None, *_dims(shape))
+    if tape.dtype != torch.float32 or tape.numel() != floats or not tape.is_contiguous():
         raise RuntimeError("tape does not match this geometry's lsso_hip_mixer_tape_floats()")
-    workspace_bytes = ctypes.c_size_t()
-    _check(
-        library.lsso_hip_mixer_backward_workspace_bytes(ctypes.byref(shape), mode, ctypes.byref(workspace_bytes)),
-        library,
-    )
-    workspace = torch.empty(workspace_bytes.value, dtype=torch.uint8, device=device)
+    workspace_bytes = _plan_size("lsso_hip_mixer_backward_workspace_bytes", mode, *_dims(shape))
+    workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device)
     grad_projected = torch.empty_like(projected)
     grad_base = torch.empty_like(core_base_raw)
     grad_drive = torch.empty_like(core_drive_weight)
     grad_eta = torch.empty_like(eta_raw)
     sums = torch.empty(projected.shape[-1], dtype=torch.float32, device=device) if column_sums else None
-    with torch.cuda.device(device):
-        status = library.lsso_hip_mixer_backward_ex(
-            ctypes.byref(shape),
-            grad_output.data_ptr(),
-            projected.data_ptr(),
-            core_base_raw.data_ptr(),
-            core_drive_weight.data_ptr(),
-            eta_raw.data_ptr(),
-            ctypes.cast(_inverse_frequency(shape.rank), ctypes.c_void_p),
-            None if centered_positions is None else centered_positions.data_ptr(),
-            mode,
-            None if valid_counts is None else valid_counts.data_ptr(),
-            tape.data_ptr(),
-            grad_projected.data_ptr(),
-            grad_base.data_ptr(),
-            grad_drive.data_ptr(),
-            grad_eta.data_ptr(),
-            None if sums is None else sums.data_ptr(),
-            workspace.data_ptr(),
-            workspace_bytes.value,
-            _stream(device),
-        )
+    status = _launch(
+        library.lsso_hip_mixer_backward_ex,
+        device,
+        ctypes.byref(shape),
+        grad_output.data_ptr(),
+        projected.data_ptr(),
+        core_base_raw.data_ptr(),
+        core_drive_weight.data_ptr(),
+        eta_raw.data_ptr(),
+        _inverse_frequency(shape.rank),
+        None if centered_positions is None else centered_positions.data_ptr(),
+        mode,
+        None if valid_counts is None else valid_counts.data_ptr(),
+        tape.data_ptr(),
+        grad_projected.data_ptr(),
+        grad_base.data_ptr(),
+        grad_drive.data_ptr(),
+        grad_eta.data_ptr(),
+        None if sums is None else sums.data_ptr(),
+        workspace.data_ptr(),
+        workspace_bytes,
+    )
     _check(status, library)
     if column_sums:
         return grad_projected, grad_base, grad_drive, grad_eta, sums
@@ -771,8 +817,7 @@ def mix_project(
     )
     device = projected.device
     dim = shape.heads * shape.head_dim
-    dtype_codes = {torch.float16: _F16, torch.bfloat16: _BF16}
-    if output_dtype not in dtype_codes:
+    if output_dtype not in _DTYPE_CODES:
         raise TypeError("the fused projection supports float16/bfloat16 outputs")
     if out_weight.dtype != torch.float32 or tuple(out_weight.shape) != (dim, dim):
         raise TypeError(f"out_weight must be float32 [{dim}, {dim}]")
@@ -789,30 +834,29 @@ def mix_project(
             raise ValueError("row_mask must be a bool [B, N] tensor")
         row_mask = row_mask.contiguous()
         mask_ptr = row_mask.data_ptr()
-    workspace_bytes = ctypes.c_size_t()
-    _check(library.lsso_hip_mixer_workspace_bytes(ctypes.byref(shape), mode, ctypes.byref(workspace_bytes)), library)
-    workspace = torch.empty(workspace_bytes.value, dtype=torch.uint8, device=device)
+    workspace_bytes = _plan_size("lsso_hip_mixer_workspace_bytes", mode, *_dims(shape))
+    workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device)
     output = torch.empty((shape.batch, shape.length, dim), dtype=output_dtype, device=device)
-    with torch.cuda.device(device):
-        status = library.lsso_hip_mixer_forward_projected(
-            ctypes.byref(shape),
-            projected.data_ptr(),
-            core_base_raw.data_ptr(),
-            core_drive_weight.data_ptr(),
-            eta_raw.data_ptr(),
-            ctypes.cast(_inverse_frequency(shape.rank), ctypes.c_void_p),
-            None if centered_positions is None else centered_positions.data_ptr(),
-            mode,
-            None if valid_counts is None else valid_counts.data_ptr(),
-            out_weight.data_ptr(),
-            None if out_bias is None else out_bias.data_ptr(),
-            mask_ptr,
-            output.data_ptr(),
-            dtype_codes[output_dtype],
-            workspace.data_ptr(),
-            workspace_bytes.value,
-            _stream(device),
-        )
+    status = _launch(
+        library.lsso_hip_mixer_forward_projected,
+        device,
+        ctypes.byref(shape),
+        projected.data_ptr(),
+        core_base_raw.data_ptr(),
+        core_drive_weight.data_ptr(),
+        eta_raw.data_ptr(),
+        _inverse_frequency(shape.rank),
+        None if centered_positions is None else centered_positions.data_ptr(),
+        mode,
+        None if valid_counts is None else valid_counts.data_ptr(),
+        out_weight.data_ptr(),
+        None if out_bias is None else out_bias.data_ptr(),
+        mask_ptr,
+        output.data_ptr(),
+        _DTYPE_CODES[output_dtype],
+        workspace.data_ptr(),
+        workspace_bytes,
+    )
     _check(status, library)
     return output
 
@@ -851,12 +895,9 @@ def layer_supported(
 ) -> bool:
     """Whether the fused whole-layer forward covers this geometry."""
 
-    library = _library()
+    _library()
     shape, _mode = _layer_shape(x, in_weight, core_base_raw, core_drive_weight, eta_raw, None, None)
-    status = library.lsso_hip_layer_supported(ctypes.byref(shape))
-    if status < 0:
-        _check(status, library)
-    return status == 1 and x.dtype in (torch.float16, torch.bfloat16)
+    return _layer_geometry_supported(*_dims(shape)) and x.dtype in _DTYPE_CODES
 
 
 def layer_forward(
@@ -901,8 +942,7 @@ def layer_forward(
     device = x.device
     dim = x.shape[-1]
     width = in_weight.shape[0]
-    dtype_codes = {torch.float16: _F16, torch.bfloat16: _BF16}
-    if x.dtype not in dtype_codes:
+    if x.dtype not in _DTYPE_CODES:
         raise TypeError("the fused layer supports float16/bfloat16 x")
     if in_bias is not None and (in_bias.dtype != torch.float32 or tuple(in_bias.shape) != (width,)):
         raise TypeError(f"in_bias must be float32 [{width}]")
@@ -925,11 +965,10 @@ def layer_forward(
             raise ValueError("row_mask must be a bool [B, N] tensor")
         row_mask = row_mask.contiguous()
         mask_ptr = row_mask.data_ptr()
-    workspace_bytes = ctypes.c_size_t()
-    _check(library.lsso_hip_layer_workspace_bytes(ctypes.byref(shape), mode, ctypes.byref(workspace_bytes)), library)
-    workspace = torch.empty(workspace_bytes.value, dtype=torch.uint8, device=device)
+    workspace_bytes = _plan_size("lsso_hip_layer_workspace_bytes", mode, *_dims(shape))
+    workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device)
     output = torch.empty((shape.batch, shape.length, dim), dtype=x.dtype, device=device)
-    arguments = []
+    after = ()
     entry = library.lsso_hip_layer_forward
     if stage_events is not None:
         if len(stage_events) != 8:
@@ -940,32 +979,32 @@ def layer_forward(
             if event is not None and handle == 0:
                 raise ValueError("stage events must have been recorded once (torch creates them lazily)")
             handles.append(handle)
-        arguments = [(ctypes.c_void_p * 8)(*[h or None for h in handles])]
+        after = ((ctypes.c_void_p * 8)(*[h or None for h in handles]),)
         entry = library.lsso_hip_layer_forward_timed
-    with torch.cuda.device(device):
-        status = entry(
-            ctypes.byref(shape),
-            x.data_ptr(),
-            dtype_codes[x.dtype],
-            in_weight.data_ptr(),
-            None if in_bias is None else in_bias.data_ptr(),
-            mask_ptr,
-            core_base_raw.data_ptr(),
-            core_drive_weight.data_ptr(),
-            eta_raw.data_ptr(),
-            ctypes.cast(_inverse_frequency(shape.rank), ctypes.c_void_p),
-            None if centered_positions is None else centered_positions.data_ptr(),
-            mode,
-            None if valid_counts is None else valid_counts.data_ptr(),
-            out_weight.data_ptr(),
-            None if out_bias is None else out_bias.data_ptr(),
-            output.data_ptr(),
-            dtype_codes[x.dtype],
-            workspace.data_ptr(),
-            workspace_bytes.value,
-            _stream(device),
-            *arguments,
-        )
+    status = _launch(
+        entry,
+        device,
+        ctypes.byref(shape),
+        x.data_ptr(),
+        _DTYPE_CODES[x.dtype],
+        in_weight.data_ptr(),
+        None if in_bias is None else in_bias.data_ptr(),
+        mask_ptr,
+        core_base_raw.data_ptr(),
+        core_drive_weight.data_ptr(),
+        eta_raw.data_ptr(),
+        _inverse_frequency(shape.rank),
+        None if centered_positions is None else centered_positions.data_ptr(),
+        mode,
+        None if valid_counts is None else valid_counts.data_ptr(),
+        out_weight.data_ptr(),
+        None if out_bias is None else out_bias.data_ptr(),
+        output.data_ptr(),
+        _DTYPE_CODES[x.dtype],
+        workspace.data_ptr(),
+        workspace_bytes,
+        after=after,
+    )
     _check(status, library)
     return output
 
@@ -994,8 +1033,7 @@ def _project_mix_forward(
     )
     device = x.device
     width = in_weight.shape[0]
-    dtype_codes = {torch.float16: _F16, torch.bfloat16: _BF16}
-    if x.dtype not in dtype_codes:
+    if x.dtype not in _DTYPE_CODES:
         raise TypeError("the fused projection + mixer supports float16/bfloat16 x")
     if in_bias is not None and (in_bias.dtype != torch.float32 or tuple(in_bias.shape) != (width,)):
         raise TypeError(f"in_bias must be float32 [{width}]")
@@ -1010,44 +1048,42 @@ def _project_mix_forward(
             raise ValueError("row_mask must be a bool [B, N] tensor")
         row_mask = row_mask.contiguous()
         mask_ptr = row_mask.data_ptr()
-    workspace_bytes = ctypes.c_size_t()
-    _check(library.lsso_hip_mixer_workspace_bytes(ctypes.byref(shape), mode, ctypes.byref(workspace_bytes)), library)
-    workspace = torch.empty(workspace_bytes.value, dtype=torch.uint8, device=device)
+    workspace_bytes = _plan_size("lsso_hip_mixer_workspace_bytes", mode, *_dims(shape))
+    workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device)
     packed = torch.empty((shape.batch, shape.length, width), dtype=torch.bfloat16, device=device)
     mixed = torch.empty(
         (shape.batch, shape.length, shape.heads * shape.head_dim), dtype=torch.bfloat16, device=device
     )
     tape = None
     if record_tape:
-        floats = ctypes.c_size_t()
-        _check(library.lsso_hip_mixer_tape_floats(ctypes.byref(shape), ctypes.byref(floats)), library)
-        tape = torch.empty(floats.value, dtype=torch.float32, device=device)
+        floats = _plan_size("lsso_hip_mixer_tape_floats", None, *_dims(shape))
+        tape = torch.empty(floats, dtype=torch.float32, device=device)
     common = (
         ctypes.byref(shape),
         x.data_ptr(),
-        dtype_codes[x.dtype],
+        _DTYPE_CODES[x.dtype],
         in_weight.data_ptr(),
         None if in_bias is None else in_bias.data_ptr(),
         mask_ptr,
         core_base_raw.data_ptr(),
         core_drive_weight.data_ptr(),
         eta_raw.data_ptr(),
-        ctypes.cast(_inverse_frequency(shape.rank), ctypes.c_void_p),
+        _inverse_frequency(shape.rank),
         None if centered_positions is None else centered_positions.data_ptr(),
         mode,
         None if valid_counts is None else valid_counts.data_ptr(),
     )
     if out_weight is None:
-        with torch.cuda.device(device):
-            status = library.lsso_hip_project_mix_forward(
-                *common,
-                packed.data_ptr(),
-                mixed.data_ptr(),
-                None if tape is None else tape.data_ptr(),
-                workspace.data_ptr(),
-                workspace_bytes.value,
-                _stream(device),
-            )
+        status = _launch(
+            library.lsso_hip_project_mix_forward,
+            device,
+            *common,
+            packed.data_ptr(),
+            mixed.data_ptr(),
+            None if tape is None else tape.data_ptr(),
+            workspace.data_ptr(),
+            workspace_bytes,
+        )
         _check(status, library)
         return packed, mixed, tape
     dim = shape.heads * shape.head_dim
@@ -1061,20 +1097,20 @@ def _project_mix_forward(
     out_weight = out_weight.contiguous()
     out_bias = None if out_bias is None else out_bias.contiguous()
     y = torch.empty((shape.batch, shape.length, dim), dtype=x.dtype, device=device)
-    with torch.cuda.device(device):
-        status = library.lsso_hip_layer_forward_train(
-            *common,
-            out_weight.data_ptr(),
-            None if out_bias is None else out_bias.data_ptr(),
-            packed.data_ptr(),
-            mixed.data_ptr(),
-            None if tape is None else tape.data_ptr(),
-            y.data_ptr(),
-            dtype_codes[x.dtype],
-            workspace.data_ptr(),
-            workspace_bytes.value,
-            _stream(device),
-        )
+    status = _launch(
+        library.lsso_hip_layer_forward_train,
+        device,
+        *common,
+        out_weight.data_ptr(),
+        None if out_bias is None else out_bias.data_ptr(),
+        packed.data_ptr(),
+        mixed.data_ptr(),
+        None if tape is None else tape.data_ptr(),
+        y.data_ptr(),
+        _DTYPE_CODES[x.dtype],
+        workspace.data_ptr(),
+        workspace_bytes,
+    )
     _check(status, library)
     return packed, mixed, tape, y
 
@@ -1176,24 +1212,24 @@ def project_mix(
 class _Layer(torch.autograd.Function):
     """Autograd of the whole layer run as one native training call
     (lsso_hip_layer_forward_train: input projection, mixer with the tape and
-    output projection).  The backward is the output projection's VJP
+    output projection).  The backward is one native call as well
+    (lsso_hip_layer_backward): the output projection's VJP
     (reference.py:205-247), the mixer VJP (cuda.py:256-280) and the input
-    projection's VJP, exactly as when the three run separately."""
+    projection's VJP, bitwise as when the three run separately."""
 
     @staticmethod
     def forward(ctx, x, in_weight, in_bias, core_base_raw, core_drive_weight, eta_raw,
                 out_weight, out_bias, centered_positions, valid_counts, row_mask):
-        with torch.no_grad():
-            packed, mixed, tape, y = _project_mix_forward(
-                x, in_weight, in_bias, core_base_raw, core_drive_weight, eta_raw,
-                centered_positions, valid_counts, row_mask, True, out_weight, out_bias,
-            )
+        packed, mixed, tape, y = _project_mix_forward(
+            x, in_weight, in_bias, core_base_raw, core_drive_weight, eta_raw,
+            centered_positions, valid_counts, row_mask, True, out_weight, out_bias,
+        )
         ctx.save_for_backward(x, in_weight, packed, core_base_raw, core_drive_weight, eta_raw, tape,
                               row_mask, mixed, out_weight)
         ctx.centered_positions = centered_positions
         ctx.valid_counts = valid_counts
-        ctx.in_bias_dtype = None if in_bias is None else in_bias.dtype
-        ctx.out_bias_dtype = None if out_bias is None else out_bias.dtype
+        ctx.has_in_bias = in_bias is not None
+        ctx.has_out_bias = out_bias is not None
         return y
 
     @staticmethod
@@ -1201,45 +1237,65 @@ class _Layer(torch.autograd.Function):
     def backward(ctx, grad_y):
         (x, in_weight, packed, core_base_raw, core_drive_weight, eta_raw, tape, row_mask, mixed,
          out_weight) = ctx.saved_tensors
+        library = _library()
         needs = ctx.needs_input_grad
-        need_mixer = any(needs[:6])
-        grad_mixed, grad_out_weight, grad_out_bias = _linear_vjp(
-            grad_y, mixed, out_weight, row_mask, need_mixer, needs[6],
-            ctx.out_bias_dtype is not None and needs[7], ctx.out_bias_dtype,
+        shape, mode = _layer_shape(
+            x, in_weight, core_base_raw, core_drive_weight, eta_raw, ctx.centered_positions, ctx.valid_counts
         )
-        grad_x = grad_in_weight = grad_in_bias = grad_base = grad_drive = grad_eta = None
-        if need_mixer:
-            need_in_bias = ctx.in_bias_dtype is not None and needs[2]
-            fused_sums = need_in_bias and row_mask is None
-            grads = backward(
-                grad_mixed.to(dtype=torch.bfloat16),
-                packed,
-                core_base_raw,
-                core_drive_weight,
-                eta_raw,
-                tape,
-                ctx.centered_positions,
-                ctx.valid_counts,
-                column_sums=fused_sums,
-            )
-            grad_packed, grad_base, grad_drive, grad_eta = grads[:4]
-            grad_x, grad_in_weight, grad_in_bias = _linear_vjp(
-                grad_packed, x, in_weight, row_mask, needs[0], needs[1], need_in_bias,
-                ctx.in_bias_dtype, grads[4] if fused_sums else None,
-            )
-        return (
-            grad_x,
-            grad_in_weight,
-            grad_in_bias,
-            grad_base if needs[3] else None,
-            grad_drive if needs[4] else None,
-            grad_eta if needs[5] else None,
-            grad_out_weight,
-            grad_out_bias,
-            None,
-            None,
-            None,
+        device = x.device
+        dim = x.shape[-1]
+        flat_grad = _rows(grad_y, dim)
+        if flat_grad.dtype not in _DTYPE_CODES:
+            flat_grad = flat_grad.to(dtype=torch.bfloat16).contiguous()
+        in_weight = in_weight.contiguous()
+        out_weight = out_weight.contiguous()
+        if row_mask is not None:
+            row_mask = row_mask.contiguous()
+
+        def empty(wanted, *sizes, dtype=torch.float32):
+            return torch.empty(sizes, dtype=dtype, device=device) if wanted else None
+
+        width = in_weight.shape[0]
+        grads = (
+            empty(needs[0], *x.shape, dtype=x.dtype),
+            empty(needs[1], width, dim),
+            empty(ctx.has_in_bias and needs[2], width),
+            empty(needs[3], *core_base_raw.shape),
+            empty(needs[4], *core_drive_weight.shape),
+            empty(needs[5], *eta_raw.shape),
+            empty(needs[6], dim, dim),
+            empty(ctx.has_out_bias and needs[7], dim),
         )
+        workspace_bytes = _plan_size("lsso_hip_layer_backward_workspace_bytes", mode, *_dims(shape))
+        workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device)
+        status = _launch(
+            library.lsso_hip_layer_backward,
+            device,
+            ctypes.byref(shape),
+            flat_grad.data_ptr(),
+            _DTYPE_CODES[flat_grad.dtype],
+            flat_grad.stride(0) if flat_grad.shape[0] > 1 else dim,
+            x.data_ptr(),
+            _DTYPE_CODES[x.dtype],
+            in_weight.data_ptr(),
+            None if row_mask is None else row_mask.data_ptr(),
+            packed.data_ptr(),
+            mixed.data_ptr(),
+            core_base_raw.data_ptr(),
+            core_drive_weight.data_ptr(),
+            eta_raw.data_ptr(),
+            _inverse_frequency(shape.rank),
+            None if ctx.centered_positions is None else ctx.centered_positions.data_ptr(),
+            mode,
+            None if ctx.valid_counts is None else ctx.valid_counts.data_ptr(),
+            tape.data_ptr(),
+            out_weight.data_ptr(),
+            *[None if grad is None else grad.data_ptr() for grad in grads],
+            workspace.data_ptr(),
+            workspace_bytes,
+        )
+        _check(status, library)
+        return (*grads, None, None, None)
 
 
 def layer_train(
@@ -1304,8 +1360,7 @@ def _linear_forward(
     library = _library()
     if value.device.type != "cuda":
         raise RuntimeError("value must be a CUDA (ROCm device) tensor")
-    dtype_codes = {torch.float16: _F16, torch.bfloat16: _BF16}
-    if value.dtype not in dtype_codes or output_dtype not in dtype_codes:
+    if value.dtype not in _DTYPE_CODES or output_dtype not in _DTYPE_CODES:
         raise TypeError("the HIP projection supports float16/bfloat16 activations and outputs")
     if weight.dtype != torch.float32 or weight.dim() != 2:
         raise TypeError("the HIP projection requires a float32 [out, in] weight")
@@ -1328,23 +1383,23 @@ def _linear_forward(
             raise ValueError("row_mask must be a bool tensor shaped like the leading dimensions")
         row_mask = row_mask.contiguous()
         mask_ptr = row_mask.data_ptr()
-    with torch.cuda.device(value.device):
-        status = library.lsso_hip_linear(
-            flat.data_ptr(),
-            dtype_codes[value.dtype],
-            rows,
-            in_features,
-            flat.stride(0) if rows > 1 else in_features,
-            weight.data_ptr(),
-            None if bias is None else bias.data_ptr(),
-            mask_ptr,
-            out_features,
-            output.data_ptr(),
-            dtype_codes[output_dtype],
-            None,
-            0,
-            _stream(value.device),
-        )
+    status = _launch(
+        library.lsso_hip_linear,
+        value.device,
+        flat.data_ptr(),
+        _DTYPE_CODES[value.dtype],
+        rows,
+        in_features,
+        flat.stride(0) if rows > 1 else in_features,
+        weight.data_ptr(),
+        None if bias is None else bias.data_ptr(),
+        mask_ptr,
+        out_features,
+        output.data_ptr(),
+        _DTYPE_CODES[output_dtype],
+        None,
+        0,
+    )
     _check(status, library)
     return output
 
@@ -1363,7 +1418,6 @@ def _grad_columns(
 
     library = _library()
     rows, cols = flat.shape
-    dtype_codes = {torch.float16: _F16, torch.bfloat16: _BF16}
     copy = torch.empty((rows, cols), dtype=torch.bfloat16, device=flat.device) if want_copy else None
     sums = torch.empty(cols, dtype=torch.float32, device=flat.device) if want_sums else None
     workspace = None
@@ -1372,20 +1426,20 @@ def _grad_columns(
         _check(library.lsso_hip_linear_grad_columns_workspace_bytes(rows, cols, ctypes.byref(size)), library)
         workspace = torch.empty(max(size.value, 1), dtype=torch.uint8, device=flat.device)
     mask = None if row_mask is None else row_mask.reshape(-1).contiguous()
-    with torch.cuda.device(flat.device):
-        status = library.lsso_hip_linear_grad_columns(
-            flat.data_ptr(),
-            dtype_codes[flat.dtype],
-            rows,
-            cols,
-            flat.stride(0) if rows > 1 else cols,
-            None if mask is None else mask.data_ptr(),
-            None if copy is None else copy.data_ptr(),
-            None if sums is None else sums.data_ptr(),
-            None if workspace is None else workspace.data_ptr(),
-            size.value,
-            _stream(flat.device),
-        )
+    status = _launch(
+        library.lsso_hip_linear_grad_columns,
+        flat.device,
+        flat.data_ptr(),
+        _DTYPE_CODES[flat.dtype],
+        rows,
+        cols,
+        flat.stride(0) if rows > 1 else cols,
+        None if mask is None else mask.data_ptr(),
+        None if copy is None else copy.data_ptr(),
+        None if sums is None else sums.data_ptr(),
+        None if workspace is None else workspace.data_ptr(),
+        size.value,
+    )
     _check(status, library)
     return copy, sums
 
@@ -1404,7 +1458,6 @@ def _weight_gradient(
     library = _library()
     rows, out_features = flat_grad.shape
     in_features = flat_value.shape[1]
-    dtype_codes = {torch.float16: _F16, torch.bfloat16: _BF16}
     device = flat_grad.device
     grad_weight = torch.empty((out_features, in_features), dtype=torch.float32, device=device)
     grad_bias = torch.empty(out_features, dtype=torch.float32, device=device) if want_bias else None
@@ -1413,24 +1466,24 @@ def _weight_gradient(
         rows, in_features, out_features, ctypes.byref(size)), library)
     workspace = torch.empty(max(size.value, 1), dtype=torch.uint8, device=device)
     mask = None if row_mask is None else row_mask.reshape(-1).contiguous()
-    with torch.cuda.device(device):
-        status = library.lsso_hip_linear_weight_grad(
-            flat_grad.data_ptr(),
-            dtype_codes[flat_grad.dtype],
-            flat_grad.stride(0) if rows > 1 else out_features,
-            flat_value.data_ptr(),
-            dtype_codes[flat_value.dtype],
-            flat_value.stride(0) if rows > 1 else in_features,
-            rows,
-            in_features,
-            out_features,
-            None if mask is None else mask.data_ptr(),
-            grad_weight.data_ptr(),
-            None if grad_bias is None else grad_bias.data_ptr(),
-            workspace.data_ptr(),
-            size.value,
-            _stream(device),
-        )
+    status = _launch(
+        library.lsso_hip_linear_weight_grad,
+        device,
+        flat_grad.data_ptr(),
+        _DTYPE_CODES[flat_grad.dtype],
+        flat_grad.stride(0) if rows > 1 else out_features,
+        flat_value.data_ptr(),
+        _DTYPE_CODES[flat_value.dtype],
+        flat_value.stride(0) if rows > 1 else in_features,
+        rows,
+        in_features,
+        out_features,
+        None if mask is None else mask.data_ptr(),
+        grad_weight.data_ptr(),
+        None if grad_bias is None else grad_bias.data_ptr(),
+        workspace.data_ptr(),
+        size.value,
+    )
     _check(status, library)
     return grad_weight, grad_bias
 

@@ -251,21 +251,32 @@ class LSSO(nn.Module):
             )
         if self.core_base_raw is None or self.core_drive_weight is None:
             raise RuntimeError("dynamic compact parameters are missing")
-        for name, parameter in self.named_parameters():
-            if parameter.device != x.device:
-                raise RuntimeError(
-                    f"implementation={implementation!r} requires {name} on {x.device}, "
-                    f"got {parameter.device}"
-                )
-        for name, parameter in (
-            ("w_bc.weight", self.w_bc.weight),
-            ("w_bc.bias", self.w_bc.bias),
-            ("w_o.weight", self.w_o.weight),
-            ("w_o.bias", self.w_o.bias),
+        w_bc, w_o = self.w_bc, self.w_o
+        device = x.device
+        parameters = (
+            ("w_bc.weight", w_bc.weight),
+            ("w_bc.bias", w_bc.bias),
+            ("w_o.weight", w_o.weight),
+            ("w_o.bias", w_o.bias),
             ("core_base_raw", self.core_base_raw),
             ("core_drive_weight", self.core_drive_weight),
             ("eta_raw", self.eta_raw),
-        ):
+        )
+        # The layer as constructed has exactly these parameters; one that was
+        # given more is walked in full (a walk costs more host time than the
+        # smallest call's launches).
+        plain = (
+            len(self._parameters) == 3 and len(self._modules) == 2
+            and len(w_bc._parameters) == 2 and len(w_o._parameters) == 2
+            and not w_bc._modules and not w_o._modules
+        )
+        for name, parameter in (*parameters[4:], *parameters[:4]) if plain else self.named_parameters():
+            if parameter is not None and parameter.device != device:
+                raise RuntimeError(
+                    f"implementation={implementation!r} requires {name} on {device}, "
+                    f"got {parameter.device}"
+                )
+        for name, parameter in parameters:
             if parameter is None:
                 continue
             if parameter.dtype != torch.float32:
@@ -278,54 +289,29 @@ class LSSO(nn.Module):
 
         from . import hip
 
-        needs_grad = torch.is_grad_enabled() and any(
-            parameter.requires_grad for parameter in (x, *self.parameters())
+        needs_grad = torch.is_grad_enabled() and (
+            x.requires_grad
+            or any(parameter is not None and parameter.requires_grad for _name, parameter in parameters)
+            or (not plain and any(parameter.requires_grad for parameter in self.parameters()))
         )
-        if not needs_grad and x.is_contiguous() and hip.layer_supported(
-            x, self.w_bc.weight, self.core_base_raw, self.core_drive_weight, self.eta_raw
-        ):
-            # Inference: the whole layer in one native call (input projection
-            # fused with the reductions, apply with the output projection),
-            # bitwise equal to the three-step path below.
-            centered_positions, valid_counts, mask = self._native_geometry(
-                x, valid_mask, position_ids
-            )
+        layer_call = x.is_contiguous() and hip.layer_supported(
+            x, w_bc.weight, self.core_base_raw, self.core_drive_weight, self.eta_raw
+        )
+        if layer_call:
+            # The whole layer in one native call, bitwise equal to the separate
+            # steps below: the input projection runs fused with the token
+            # reductions and the apply with the output projection where the
+            # shapes allow; with gradients the call also keeps packed, mixed
+            # and the tape for the backward.
+            centered_positions, valid_counts, mask = self._native_geometry(x, valid_mask, position_ids)
+            if needs_grad:
+                return hip.layer_train(
+                    x, w_bc.weight, w_bc.bias, self.core_base_raw, self.core_drive_weight, self.eta_raw,
+                    w_o.weight, w_o.bias, centered_positions, valid_counts, row_mask=mask,
+                )
             return hip.layer_forward(
-                x,
-                self.w_bc.weight,
-                self.w_bc.bias,
-                self.core_base_raw,
-                self.core_drive_weight,
-                self.eta_raw,
-                centered_positions,
-                valid_counts,
-                self.w_o.weight,
-                self.w_o.bias,
-                row_mask=mask,
-            )
-        if needs_grad and x.is_contiguous() and hip.layer_supported(
-            x, self.w_bc.weight, self.core_base_raw, self.core_drive_weight, self.eta_raw
-        ):
-            # Training: the whole layer in one native call that also keeps
-            # packed, mixed and the tape for the backward (the input
-            # projection runs fused with the token reductions, the apply with
-            # the output projection where the shapes allow), bitwise equal to
-            # the separate linear + fast_mix + linear below.
-            centered_positions, valid_counts, mask = self._native_geometry(
-                x, valid_mask, position_ids
-            )
-            return hip.layer_train(
-                x,
-                self.w_bc.weight,
-                self.w_bc.bias,
-                self.core_base_raw,
-                self.core_drive_weight,
-                self.eta_raw,
-                self.w_o.weight,
-                self.w_o.bias,
-                centered_positions,
-                valid_counts,
-                row_mask=mask,
+                x, w_bc.weight, w_bc.bias, self.core_base_raw, self.core_drive_weight, self.eta_raw,
+                centered_positions, valid_counts, w_o.weight, w_o.bias, row_mask=mask,
             )
         projected, centered_positions, valid_counts, mask = self._native_inputs(
             x, valid_mask, position_ids

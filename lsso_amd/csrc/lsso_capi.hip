@@ -1625,3 +1625,179 @@ int layer_forward_impl(const lsso_hip_mixer_shape* shape, const void* x, int x_d
 }
 
 }  // namespace
+
+// ---------------------------------------------------------------------------
+// Backward of the whole layer in one call.
+namespace {
+
+struct LayerBackwardPlan {
+    size_t off_out_t, off_in_t, off_grad_mixed, off_grad_packed, off_params, off_scratch;
+    size_t scratch_bytes, total;
+};
+
+// The parts share one scratch region: they run one after the other on a stream.
+int make_layer_backward_plan(const lsso_hip_mixer_shape* shape, int positions_mode, MixerPlan* plan,
+                             LayerBackwardPlan* lb) {
+    int status = make_plan(shape, positions_mode, plan);
+    if (status != LSSO_HIP_OK) {
+        return status;
+    }
+    BackwardPlan bp;
+    status = make_backward_plan(*plan, &bp);
+    if (status != LSSO_HIP_OK) {
+        return status;
+    }
+    const int64_t rows = plan->batch * plan->length;
+    const int64_t dim = plan->out_width;
+    WeightGradPlan in_plan;
+    WeightGradPlan out_plan;
+    make_weight_grad_plan(rows, dim, plan->width, &in_plan);
+    make_weight_grad_plan(rows, dim, dim, &out_plan);
+    GradColumnsPlan columns;
+    plan_grad_columns(rows, plan->width, &columns);
+    size_t scratch = std::max(bp.total, std::max(in_plan.total, out_plan.total));
+    scratch = std::max(scratch, align_up(sizeof(float) * columns.splits * plan->width));
+    plan_grad_columns(rows, dim, &columns);
+    scratch = std::max(scratch, align_up(sizeof(float) * columns.splits * dim));
+    size_t offset = 0;
+    lb->off_out_t = offset;
+    offset = align_up(offset + sizeof(float) * dim * dim);
+    lb->off_in_t = offset;
+    offset = align_up(offset + sizeof(float) * plan->width * dim);
+    lb->off_grad_mixed = offset;
+    offset = align_up(offset + sizeof(uint16_t) * rows * dim);
+    lb->off_grad_packed = offset;
+    offset = align_up(offset + sizeof(uint16_t) * rows * plan->width);
+    // Stand-ins for compact gradients that the caller does not want.
+    lb->off_params = offset;
+    offset = align_up(offset + sizeof(float) * plan->heads * (plan->rank * plan->rank + plan->head_dim * plan->rank + 1));
+    lb->off_scratch = offset;
+    lb->scratch_bytes = scratch;
+    lb->total = offset + scratch;
+    return LSSO_HIP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int lsso_hip_layer_backward_workspace_bytes(const lsso_hip_mixer_shape* shape, int positions_mode,
+                                            size_t* bytes) {
+    if (bytes == nullptr) {
+        return fail(LSSO_HIP_EINVAL, "bytes must not be NULL");
+    }
+    MixerPlan plan;
+    LayerBackwardPlan lb;
+    const int status = make_layer_backward_plan(shape, positions_mode, &plan, &lb);
+    if (status != LSSO_HIP_OK) {
+        return status;
+    }
+    *bytes = lb.total;
+    return LSSO_HIP_OK;
+}
+
+int lsso_hip_layer_backward(const lsso_hip_mixer_shape* shape, const void* grad_y, int grad_y_dtype,
+                            int64_t grad_y_stride, const void* x, int x_dtype,
+                            const float* in_weight, const uint8_t* row_mask, const void* packed,
+                            const void* mixed, const float* core_base_raw,
+                            const float* core_drive_weight, const float* eta_raw,
+                            const float* inverse_frequency, const float* centered_positions,
+                            int positions_mode, const float* valid_counts, const float* tape,
+                            const float* out_weight, void* grad_x, float* grad_in_weight,
+                            float* grad_in_bias, float* grad_base, float* grad_drive,
+                            float* grad_eta, float* grad_out_weight, float* grad_out_bias,
+                            void* workspace, size_t workspace_bytes, void* stream_handle) {
+    MixerPlan plan;
+    LayerBackwardPlan lb;
+    int status = make_layer_backward_plan(shape, positions_mode, &plan, &lb);
+    if (status != LSSO_HIP_OK) {
+        return status;
+    }
+    if (grad_y == nullptr || x == nullptr || in_weight == nullptr || out_weight == nullptr || packed == nullptr ||
+        mixed == nullptr) {
+        return fail(LSSO_HIP_EINVAL, "grad_y, x, packed, mixed and the weights must not be NULL");
+    }
+    if ((grad_y_dtype != LSSO_HIP_F16 && grad_y_dtype != LSSO_HIP_BF16) ||
+        (x_dtype != LSSO_HIP_F16 && x_dtype != LSSO_HIP_BF16)) {
+        return fail(LSSO_HIP_EUNSUPPORTED, "projection dtypes must be float16 or bfloat16");
+    }
+    if (workspace == nullptr || workspace_bytes < lb.total || !aligned(workspace, 256)) {
+        return fail(LSSO_HIP_EINVAL,
+                    "workspace must be 256-byte aligned and hold lsso_hip_layer_backward_workspace_bytes()");
+    }
+    const int64_t rows = plan.batch * plan.length;
+    const int64_t dim = plan.out_width;
+    char* ws = static_cast<char*>(workspace);
+    float* out_t = reinterpret_cast<float*>(ws + lb.off_out_t);
+    float* in_t = reinterpret_cast<float*>(ws + lb.off_in_t);
+    void* grad_mixed = ws + lb.off_grad_mixed;
+    void* grad_packed = ws + lb.off_grad_packed;
+    float* params = reinterpret_cast<float*>(ws + lb.off_params);
+    void* scratch = ws + lb.off_scratch;
+    hipStream_t stream = static_cast<hipStream_t>(stream_handle);
+
+    const bool need_packed = grad_x != nullptr || grad_in_weight != nullptr || grad_in_bias != nullptr;
+    const bool need_mixer = need_packed || grad_base != nullptr || grad_drive != nullptr || grad_eta != nullptr;
+    const hipError_t error = lsso_hip::launch_transpose2(
+        out_weight, need_mixer ? dim : 0, dim, out_t, in_weight, grad_x != nullptr ? plan.width : 0, dim, in_t, stream);
+    if (error != hipSuccess) {
+        return hip_failure(error, "transpose2_kernel launch");
+    }
+
+    // Output projection.
+    if (need_mixer) {
+        status = lsso_hip_linear(grad_y, grad_y_dtype, rows, dim, grad_y_stride, out_t, nullptr, row_mask, dim,
+                                 grad_mixed, LSSO_HIP_BF16, nullptr, 0, stream_handle);
+        if (status != LSSO_HIP_OK) {
+            return status;
+        }
+    }
+    if (grad_out_weight != nullptr) {
+        status = lsso_hip_linear_weight_grad(grad_y, grad_y_dtype, grad_y_stride, mixed, LSSO_HIP_BF16, dim, rows, dim,
+                                             dim, row_mask, grad_out_weight, grad_out_bias, scratch, lb.scratch_bytes,
+                                             stream_handle);
+    } else if (grad_out_bias != nullptr) {
+        status = lsso_hip_linear_grad_columns(grad_y, grad_y_dtype, rows, dim, grad_y_stride, row_mask, nullptr,
+                                              grad_out_bias, scratch, lb.scratch_bytes, stream_handle);
+    }
+    if (status != LSSO_HIP_OK || !need_mixer) {
+        return status;
+    }
+
+    // Mixer.  Without a row mask the column sums of grad_packed taken inside
+    // the token map are the bias gradient; with one, rows the mask excludes
+    // must not count, and only the projection's own pass knows them.
+    const bool fused_sums = grad_in_bias != nullptr && row_mask == nullptr;
+    const int64_t base_floats = plan.heads * plan.rank * plan.rank;
+    const int64_t drive_floats = plan.heads * plan.head_dim * plan.rank;
+    status = lsso_hip_mixer_backward_ex(
+        shape, grad_mixed, packed, core_base_raw, core_drive_weight, eta_raw, inverse_frequency, centered_positions,
+        positions_mode, valid_counts, tape, grad_packed, grad_base != nullptr ? grad_base : params,
+        grad_drive != nullptr ? grad_drive : params + base_floats,
+        grad_eta != nullptr ? grad_eta : params + base_floats + drive_floats, fused_sums ? grad_in_bias : nullptr,
+        scratch, lb.scratch_bytes, stream_handle);
+    if (status != LSSO_HIP_OK) {
+        return status;
+    }
+
+    // Input projection.
+    if (grad_x != nullptr) {
+        status = lsso_hip_linear(grad_packed, LSSO_HIP_BF16, rows, plan.width, plan.width, in_t, nullptr, row_mask, dim,
+                                 grad_x, x_dtype, nullptr, 0, stream_handle);
+        if (status != LSSO_HIP_OK) {
+            return status;
+        }
+    }
+    float* own_bias = fused_sums ? nullptr : grad_in_bias;
+    if (grad_in_weight != nullptr) {
+        return lsso_hip_linear_weight_grad(grad_packed, LSSO_HIP_BF16, plan.width, x, x_dtype, dim, rows, dim, plan.width,
+                                           row_mask, grad_in_weight, own_bias, scratch, lb.scratch_bytes, stream_handle);
+    }
+    if (own_bias != nullptr) {
+        return lsso_hip_linear_grad_columns(grad_packed, LSSO_HIP_BF16, rows, plan.width, plan.width, row_mask, nullptr,
+                                            own_bias, scratch, lb.scratch_bytes, stream_handle);
+    }
+    return LSSO_HIP_OK;
+}
+
+}  // extern "C"

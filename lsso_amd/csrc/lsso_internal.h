@@ -329,6 +329,10 @@ int project_reduce_group_heads(int64_t rank, int64_t heads, int64_t head_dim,
 int project_reduce_tile_rows();
 hipError_t launch_project_reduce(int rank, const ProjectReduceArgs& a, int x_dtype, int grid,
                                  hipStream_t stream);
+// out[cols, rows] = in[rows, cols]^T of two FP32 matrices in one launch
+// (either may be absent: rows 0).
+hipError_t launch_transpose2(const float* in1, int64_t rows1, int64_t cols1, float* out1, const float* in2,
+                             int64_t rows2, int64_t cols2, float* out2, hipStream_t stream);
 hipError_t launch_grad_columns(const GradColumnsArgs& a, int g_dtype, bool vec, int64_t splits,
                                int64_t slabs, float* column_sums, hipStream_t stream);
 void plan_weight_grad(int64_t rows, int64_t in_features, int64_t out_features, int64_t* splits,

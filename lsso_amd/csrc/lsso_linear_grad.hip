@@ -291,4 +291,61 @@ hipError_t launch_grad_columns(const GradColumnsArgs& a, int g_dtype, bool vec, 
     return launch_column_sum(a.partials, splits, a.cols, column_sums, stream);
 }
 
+// Transposed weights of the projections' value gradients (dX = dY W reads W
+// by output feature).  32 x 32 tiles through LDS, both of a layer's weights in
+// one launch: two tensor copies before took 3.2-6.8 us each and their host time.
+constexpr int kTransposeTile = 32;
+
+struct TransposeArgs {
+    const float* in;
+    int64_t rows, cols;
+    float* out;
+    int64_t tiles_c, tiles;
+};
+
+__global__ __launch_bounds__(kGradThreads) void transpose2_kernel(TransposeArgs first, TransposeArgs second) {
+    __shared__ float s_tile[kTransposeTile][kTransposeTile + 1];
+    int64_t tile = blockIdx.x;
+    TransposeArgs a = first;
+    if (tile >= first.tiles) {   // uniform over the workgroup
+        tile -= first.tiles;
+        a = second;
+    }
+    const int64_t r0 = tile / a.tiles_c * kTransposeTile;
+    const int64_t c0 = tile % a.tiles_c * kTransposeTile;
+    const int c = threadIdx.x % kTransposeTile;
+    const int r = threadIdx.x / kTransposeTile;
+    constexpr int kRows = kGradThreads / kTransposeTile;
+#pragma unroll
+    for (int i = 0; i < kTransposeTile; i += kRows) {
+        if (r0 + r + i < a.rows && c0 + c < a.cols) {
+            s_tile[r + i][c] = a.in[(r0 + r + i) * a.cols + c0 + c];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTransposeTile; i += kRows) {
+        if (c0 + r + i < a.cols && r0 + c < a.rows) {
+            a.out[(c0 + r + i) * a.rows + r0 + c] = s_tile[c][r + i];
+        }
+    }
+}
+
+hipError_t launch_transpose2(const float* in1, int64_t rows1, int64_t cols1, float* out1, const float* in2,
+                             int64_t rows2, int64_t cols2, float* out2, hipStream_t stream) {
+    const auto plan = [](const float* in, int64_t rows, int64_t cols, float* out) {
+        const int64_t tiles_r = (rows + kTransposeTile - 1) / kTransposeTile;
+        const int64_t tiles_c = (cols + kTransposeTile - 1) / kTransposeTile;
+        return TransposeArgs{in, rows, cols, out, tiles_c, tiles_r * tiles_c};
+    };
+    const TransposeArgs first = plan(in1, rows1, cols1, out1);
+    const TransposeArgs second = plan(in2, rows2, cols2, out2);
+    if (first.tiles + second.tiles == 0) {
+        return hipSuccess;
+    }
+    const dim3 grid(static_cast<unsigned>(first.tiles + second.tiles));
+    transpose2_kernel<<<grid, kGradThreads, 0, stream>>>(first, second);
+    return hipGetLastError();
+}
+
 }  // namespace lsso_hip
