@@ -58,8 +58,15 @@ constexpr int64_t kApplyStagedTargetGroups = 512;   // workgroups of the staged 
 // tokens, two chunks per sequence leave the standalone reduce too few waves
 // (the C5 step 1,166 against 1,139 us).  The choice depends on the sequence
 // length only, never on the batch.
+//
+// The chunks of a sequence are then evened out (in whole 64-token tiles): a
+// chunk's tiles run one after the other, about 3 us each, so a 513-token
+// sequence cut into 512 + 1 tokens took the time of eight tiles where 320 + 193
+// takes five (the masked 8 x 513 layer call 60 -> 52 us).
 int64_t reduce_chunk_tokens(int64_t length) {
-    return length >= 4096 ? 2 * kReduceChunkTokens : kReduceChunkTokens;
+    const int64_t most = length >= 4096 ? 2 * kReduceChunkTokens : kReduceChunkTokens;
+    const int64_t chunks = ceil_div(length, most);
+    return ceil_div(ceil_div(length, chunks), 64) * 64;
 }
 
 struct MixerPlan {
@@ -371,7 +378,8 @@ int run_reduce(const MixerPlan& plan, const MixerBuffers& buf, const void* proje
     reduce.partial_stride = plan.partial_stride;
     reduce.total_waves = plan.batch * plan.heads * plan.reduce_chunks * plan.column_groups;
     reduce.group_heads = plan.cpw == 1 ? lsso_hip::reduce_staged_group_heads(plan.rank, plan.heads, plan.head_dim,
-                                                                              plan.column_groups, reduce.content_stride,
+                                                                              plan.column_groups,
+                                                                              plan.batch * plan.reduce_chunks,
                                                                               vec && plan.head_dim % 8 == 0)
                                        : 0;
     const hipError_t error =
@@ -910,7 +918,8 @@ int lsso_hip_mixer_backward_ex(const lsso_hip_mixer_shape* shape, const void* gr
     reduce.partial_stride = plan.partial_stride;
     reduce.total_waves = plan.batch * plan.heads * plan.reduce_chunks * plan.column_groups;
     reduce.group_heads = plan.cpw == 1 ? lsso_hip::reduce_staged_group_heads(plan.rank, plan.heads, plan.head_dim,
-                                                                              plan.column_groups, reduce.content_stride,
+                                                                              plan.column_groups,
+                                                                              plan.batch * plan.reduce_chunks,
                                                                               vec && plan.head_dim % 8 == 0)
                                        : 0;
     error = lsso_hip::launch_reduce(static_cast<int>(plan.rank), reduce, plan.cpw, vec, stream);

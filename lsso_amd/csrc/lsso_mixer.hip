@@ -190,6 +190,7 @@ __global__ __launch_bounds__(256, 2) void reduce_kernel(ReduceArgs a) {
 // k + 1 are in flight during step k's reductions.
 constexpr int kStagedWaves = 8;              // at most, per workgroup
 constexpr int kStagedCols = 512;             // group columns (relation + content) per row, at most
+constexpr int64_t kStagedComputeUnits = 256;
 constexpr int kStagedRelPieces = 3;          // 16-byte pieces per thread and step, at most
 constexpr int kStagedConPieces = 2;
 constexpr int kStagedPhasePieces = 1;
@@ -403,7 +404,7 @@ __global__ __launch_bounds__(kStagedWaves * 64) void reduce_staged_kernel(Reduce
 }
 
 int64_t reduce_staged_group_heads(int64_t rank, int64_t heads, int64_t head_dim, int64_t column_groups,
-                                  int64_t content_stride, bool vec) {
+                                  int64_t items, bool vec) {
     // Rows read as 16-byte pieces: relation and content runs whole pieces.
     if (!vec || rank < 48 || head_dim % 8 != 0 || column_groups < 1 || column_groups > kStagedWaves) {
         return 0;
@@ -416,12 +417,22 @@ int64_t reduce_staged_group_heads(int64_t rank, int64_t heads, int64_t head_dim,
     if (group * 2 > heads && heads > 1) group = (heads + 1) / 2;
     if (group < 1) return 0;
     // Pieces per thread within the staging registers.
-    const int64_t threads = 64 * group * column_groups;
-    if (32 * group * rank / 8 > kStagedRelPieces * threads || 32 * group * head_dim / 8 > kStagedConPieces * threads ||
-        32 * (rank / 2) / 4 > kStagedPhasePieces * threads) {
+    const auto fits = [&](int64_t g) {
+        const int64_t threads = 64 * g * column_groups;
+        return 32 * g * rank / 8 <= kStagedRelPieces * threads && 32 * g * head_dim / 8 <= kStagedConPieces * threads &&
+               32 * (rank / 2) / 4 <= kStagedPhasePieces * threads;
+    };
+    if (!fits(group)) {
         return 0;
     }
-    (void)content_stride;
+    // Few samples and chunks leave CUs idle, while the waves that share a SIMD
+    // in a group of eight take turns through a chain of 32-token steps: spread
+    // the heads over more workgroups as long as each finds a CU of its own (2
+    // x 4,096 tokens, 12 heads of 48 + 64: 68 us in 24 workgroups, 50 in 48).
+    while (group > 1 && fits((group + 1) / 2) &&
+           items * ((heads + (group + 1) / 2 - 1) / ((group + 1) / 2)) <= kStagedComputeUnits) {
+        group = (group + 1) / 2;
+    }
     return group;
 }
 
