@@ -1271,7 +1271,7 @@ constexpr int kBwdStagedPh = 1;
 constexpr int kBwdStagedOutPieces = 3;  //   and stored dR / dC pieces
 
 template <int R, int D16>
-__global__ __launch_bounds__(kBwdStagedWaves * 64) void bwd_apply_staged_kernel(BwdApplyArgs a, int group_heads) {
+__global__ __launch_bounds__(kBwdStagedWaves * 64, 2) void bwd_apply_staged_kernel(BwdApplyArgs a, int group_heads) {
     using In = BwdTokenInputs<R, D16>;
     using RR = typename In::RR;
     using RD = typename In::RD;
@@ -1462,15 +1462,27 @@ __global__ __launch_bounds__(kBwdStagedWaves * 64) void bwd_apply_staged_kernel(
     }
 
     float dot = 0.0f;
-    // Column sums of this head's [dR | dC] columns over the chunk, from the
-    // output tiles: lane j holds columns 2 j, 2 j + 1.
-    constexpr int kPairColumns = (R + D) / 2;
-    static_assert(kPairColumns <= 64, "one column pair per lane");
-    float col_even = 0.0f;
-    float col_odd = 0.0f;
     const int rel_col = unit * R;
     const int my_con = con_col + unit * D;
     const int my_dy = dy_col + unit * D;
+    // Column sums of this head's [dR | dC] columns over the chunk, from the
+    // output tiles: ones (16 x 16) times the tile's 16 tokens x 16 columns on
+    // the matrix cores, whose operand a transposed LDS read delivers (four
+    // tokens of its column per lane).  Added up by the lanes (16 reads, 32
+    // conversions and 32 additions per step) they took a quarter of the map's
+    // time: 152 -> 116 us at 64 x 4,096 tokens, 8 heads of 32 + 32 (670 MB: 5.8
+    // TB/s), 103 -> 88 us at 64 x 2,048, 48 + 32 (two workgroups per CU, forced:
+    // the accumulators would else take the registers past half a SIMD's).
+    constexpr int kSumBlocks = (R + D) / 16;
+    f32x4 col_acc[kSumBlocks];
+#pragma unroll
+    for (int i = 0; i < kSumBlocks; ++i) {
+        col_acc[i] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const auto sum_column = [&](int block) {   // first column of a block in the output tile
+        return 16 * block < R ? rel_col + 16 * block : con_col + unit * D + 16 * block - R;
+    };
+    const u32x2 ones = {0x3f803f80u, 0x3f803f80u};
     auto compute = [&](int buf, int obuf, int64_t t0) {
         if (!active) {
             return;
@@ -1585,22 +1597,15 @@ __global__ __launch_bounds__(kBwdStagedWaves * 64) void bwd_apply_staged_kernel(
             packed.y = pack_bf16(fmaf(eta, bf16_lo(dyv.y), acc[2]), fmaf(eta, bf16_hi(dyv.y), acc[3]));
             *reinterpret_cast<u32x2*>(orow + con_col + unit * D + f0) = packed;
         }
-        if (a.column_part != nullptr && lane < kPairColumns) {
+        if (a.column_part != nullptr) {
             // The wave's own tile rows: its reads follow its writes in order.
-            const int c = 2 * lane;
-            const int col = c < R ? rel_col + c : con_col + unit * D + (c - R);
-            float even = 0.0f;
-            float odd = 0.0f;
+            // Rows past the chunk are zero, as their inputs are.
+            const uint16_t* sums = &s_out[obuf][(4 * g + q / 4) * out_pitch + 4 * (q % 4)];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                if (t0 + r < end) {
-                    const uint32_t v = *reinterpret_cast<const uint32_t*>(&s_out[obuf][r * out_pitch + col]);
-                    even += bf16_lo(v);
-                    odd += bf16_hi(v);
-                }
+            for (int i = 0; i < kSumBlocks; ++i) {
+                const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS16x4*)(sums + sum_column(i)));
+                col_acc[i] = mfma16x16x16(ones, __builtin_bit_cast(u32x2, v), col_acc[i]);
             }
-            col_even += even;
-            col_odd += odd;
         }
     };
     auto store = [&](int obuf, int64_t t0) {
@@ -1636,12 +1641,12 @@ __global__ __launch_bounds__(kBwdStagedWaves * 64) void bwd_apply_staged_kernel(
         store(1, t0 + 16);
     }
     if (active) {
-        if (a.column_part != nullptr && lane < kPairColumns) {
-            const int c = 2 * lane;
-            const int64_t column = c < R ? h * R + c : a.heads * R + h * D + c - R;
-            float* row = a.column_part + (b * a.chunks + chunk) * a.width + column;
-            row[0] = col_even;
-            row[1] = col_odd;
+        if (a.column_part != nullptr && g == 0) {
+            float* row = a.column_part + (b * a.chunks + chunk) * a.width;
+#pragma unroll
+            for (int i = 0; i < kSumBlocks; ++i) {
+                row[(16 * i < R ? h * R + 16 * i : a.heads * R + h * D + 16 * i - R) + q] = col_acc[i][0];
+            }
         }
         for (int offset = 32; offset > 0; offset >>= 1) {
             dot += __shfl_xor(dot, offset);

@@ -15,6 +15,11 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// Operand of __builtin_amdgcn_ds_read_tr16_b64_v4i16: 16 lanes read 4 rows x 16
+// columns of 16-bit values (lane i: 4 columns of row i / 4), and lane i receives
+// the 4 rows of column i.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 LdsS16x4;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // 1 - 2^-23: the one-ULP interior scale of the complement

@@ -78,9 +78,6 @@ constexpr int kSchedMfma = 0x8;
 constexpr int kSchedDsRead = 0x100;
 constexpr int kSchedDsWrite = 0x200;
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 LdsS16x4;
-
 template <int T>
 __device__ __forceinline__ float bits_to_float(uint32_t bits) {
     if constexpr (T == LSSO_HIP_BF16) {
