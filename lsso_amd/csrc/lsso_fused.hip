@@ -252,6 +252,15 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
     // operand records, MFMA order and rounding; thread io stages the rows.
     const int j = wave - kMixProjWaves;
     const int io = tid - 64 * kMixProjWaves;
+    // Slots past the heads repeat head j, and feature blocks past the head's
+    // repeat block 0: they compute and store the same values to the same
+    // places.  A branch around each would end the basic block, and with it the
+    // interleaving of the slots' independent MFMA chains (below).
+    const bool has_head = j < H;
+    const auto head = [&](int u) {
+        return has_head ? (j + kMixApplyWaves * u < H ? j + kMixApplyWaves * u : j) : 0;
+    };
+    const auto block = [&](int f) { return f < a.feature_blocks ? f : 0; };
     u32x4 op_hi32[HPW][NFB][S32];
     u32x4 op_lo32[HPW][NFB][S32];
     u32x2 op_hi16[HPW][NFB][S16];
@@ -259,14 +268,12 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
     float eta[HPW];
 #pragma unroll
     for (int u = 0; u < HPW; ++u) {
-        const int64_t h = j + kMixApplyWaves * u < H ? j + kMixApplyWaves * u : 0;
+        const int64_t h = head(u);
         eta[u] = bounded_complement(a.eta_raw[h]);
         const int64_t system = b * H + h;
 #pragma unroll
         for (int f = 0; f < NFB; ++f) {
-            const bool live = f < a.feature_blocks;
-            const uint16_t* record =
-                a.mop + ((system * a.feature_blocks + (live ? f : 0)) * 64 + lane) * AL::kLaneHalfs;
+            const uint16_t* record = a.mop + ((system * a.feature_blocks + block(f)) * 64 + lane) * AL::kLaneHalfs;
 #pragma unroll
             for (int s = 0; s < AL::kSteps32; ++s) {
                 op_hi32[u][f][s] = *reinterpret_cast<const u32x4*>(record + AL::offset32(s));
@@ -292,9 +299,12 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
     for (int c = 0; c < kMixChunks; ++c) {
         const int idx = io + c * kMixIoThreads;
         const int row = idx / row_chunks;
-        lds_chunk[c] = idx < tile_chunks ? row * kMixPitch + 8 * (idx - row * row_chunks) : -1;
+        // Pieces past the tile go to the rows' padding, which nothing reads.
+        lds_chunk[c] = idx < tile_chunks ? row * kMixPitch + 8 * (idx - row * row_chunks)
+                                         : (io % kMixRows) * kMixPitch + WMAX;
     }
-    const int phase_lds = io < kMixRows * (PAIRS / 4) ? (io / (PAIRS / 4)) * PHP + 4 * (io % (PAIRS / 4)) : -1;
+    const bool phase_live = io < kMixRows * (PAIRS / 4);
+    const int phase_lds = phase_live ? (io / (PAIRS / 4)) * PHP + 4 * (io % (PAIRS / 4)) : (io % kMixRows) * PHP + PAIRS;
     const uint16_t* sample_rows = a.projected + b * a.length * W;
     const uint32_t* sample_phases = a.phases + b * a.phase_batch_stride;
     struct Stage {
@@ -312,7 +322,7 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
         }
         const BufferRsrc ph = make_buffer(sample_phases + static_cast<int64_t>(t0) * PAIRS,
                                           int64_t{4} * rows * PAIRS);
-        st.phase = buffer_load16(ph, phase_lds >= 0 ? 16u * static_cast<uint32_t>(io) : kOutOfRange);
+        st.phase = buffer_load16(ph, phase_live ? 16u * static_cast<uint32_t>(io) : kOutOfRange);
         if constexpr (MASKED) {
             const BufferRsrc mbuf = make_buffer(a.row_mask + b * a.length + t0, rows);
             st.mask = buffer_load_byte(mbuf, static_cast<uint32_t>(io < kMixRows ? io : kMixRows));
@@ -322,13 +332,9 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
         uint16_t* pk = s_pk[t & 1];
 #pragma unroll
         for (int c = 0; c < kMixChunks; ++c) {
-            if (lds_chunk[c] >= 0) {
-                *reinterpret_cast<u32x4*>(pk + lds_chunk[c]) = st.chunk[c];
-            }
+            *reinterpret_cast<u32x4*>(pk + lds_chunk[c]) = st.chunk[c];
         }
-        if (phase_lds >= 0) {
-            *reinterpret_cast<u32x4*>(s_ph[t & 1] + phase_lds) = st.phase;
-        }
+        *reinterpret_cast<u32x4*>(s_ph[t & 1] + phase_lds) = st.phase;
         if (io < kMixRows) {
             s_keep[t % 3][io] = io < tile_rows(t) && (!MASKED || st.mask != 0);
         }
@@ -345,108 +351,144 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
         u32x2 ph16[S16];
         u32x2 con[NFB];
     };
+    // Head slots advanced together: both, unless their accumulators and
+    // operands would not fit beside the records (which then also means reading
+    // a slot's operands when its turn comes).
+    constexpr bool kReadFirst = HPW * NFB <= 4;
+    constexpr int kTogether = kReadFirst ? HPW : 1;
     auto apply_tile = [&](int t) {
         const uint16_t* pk = s_pk[t & 1];
         const uint32_t* phs = s_ph[t & 1];
         uint16_t* mx = s_mx[t & 1];
         const int q = lane & 15;
         const int g = lane >> 4;
+        auto read = [&](int u, int sub) {
+            ApplyIn in;
+            const int64_t h = head(u);
+            const int r = sub * 16 + q;
+            const uint16_t* prow = pk + r * kMixPitch;
+            const uint32_t* phrow = phs + r * PHP;
+#pragma unroll
+            for (int s = 0; s < AL::kSteps32; ++s) {
+                const int first_rank = 32 * s + 8 * g;
+                in.rel32[s] = *reinterpret_cast<const u32x4*>(prow + h * R + first_rank);
+                in.ph32[s] = *reinterpret_cast<const u32x4*>(phrow + first_rank / 2);
+            }
+#pragma unroll
+            for (int s = 0; s < AL::kSteps16; ++s) {
+                const int first_rank = 16 * s + 4 * g;
+                in.rel16[s] = *reinterpret_cast<const u32x2*>(prow + h * R + first_rank);
+                in.ph16[s] = *reinterpret_cast<const u32x2*>(phrow + first_rank / 2);
+            }
+#pragma unroll
+            for (int f = 0; f < NFB; ++f) {
+                const int64_t feature = h * d + 16 * block(f) + 4 * g;
+                in.con[f] = *reinterpret_cast<const u32x2*>(prow + H * R + feature);
+            }
+            return in;
+        };
         ApplyIn in[HPW][kMixRows / 16];
+        if constexpr (kReadFirst) {
 #pragma unroll
-        for (int u = 0; u < HPW; ++u) {
-            const int64_t h = j + kMixApplyWaves * u < H ? j + kMixApplyWaves * u : j;
+            for (int u = 0; u < HPW; ++u) {
 #pragma unroll
-            for (int sub = 0; sub < kMixRows / 16; ++sub) {
-                const int r = sub * 16 + q;
-                const uint16_t* prow = pk + r * kMixPitch;
-                const uint32_t* phrow = phs + r * PHP;
-#pragma unroll
-                for (int s = 0; s < AL::kSteps32; ++s) {
-                    const int first_rank = 32 * s + 8 * g;
-                    in[u][sub].rel32[s] = *reinterpret_cast<const u32x4*>(prow + h * R + first_rank);
-                    in[u][sub].ph32[s] = *reinterpret_cast<const u32x4*>(phrow + first_rank / 2);
-                }
-#pragma unroll
-                for (int s = 0; s < AL::kSteps16; ++s) {
-                    const int first_rank = 16 * s + 4 * g;
-                    in[u][sub].rel16[s] = *reinterpret_cast<const u32x2*>(prow + h * R + first_rank);
-                    in[u][sub].ph16[s] = *reinterpret_cast<const u32x2*>(phrow + first_rank / 2);
-                }
-#pragma unroll
-                for (int f = 0; f < NFB; ++f) {
-                    const int64_t feature = h * d + 16 * (f < a.feature_blocks ? f : 0) + 4 * g;
-                    in[u][sub].con[f] = *reinterpret_cast<const u32x2*>(prow + H * R + feature);
+                for (int sub = 0; sub < kMixRows / 16; ++sub) {
+                    in[u][sub] = read(u, sub);
                 }
             }
         }
 #pragma unroll
-        for (int sub = 0; sub < kMixRows / 16; ++sub) {
+        for (int step = 0; step < kMixRows / 16 * (HPW / kTogether); ++step) {
+            const int sub = step / (HPW / kTogether);
+            const int u0 = step % (HPW / kTogether) * kTogether;
+            if constexpr (!kReadFirst) {
 #pragma unroll
-            for (int u = 0; u < HPW; ++u) {
-                const int64_t h = j + kMixApplyWaves * u;
-                if (h >= H) {
-                    continue;   // wave-uniform
+                for (int u = 0; u < kTogether; ++u) {
+                    in[u0 + u][sub] = read(u0 + u, sub);
                 }
-                const ApplyIn& op = in[u][sub];
-                const int r = sub * 16 + q;
-                u32x4 b_hi32[S32];
-                u32x4 b_lo32[S32];
+            }
+            u32x4 b_hi32[kTogether][S32];
+            u32x4 b_lo32[kTogether][S32];
+            u32x2 b_hi16[kTogether][S16];
+            u32x2 b_lo16[kTogether][S16];
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u) {
+                const ApplyIn& op = in[u0 + u][sub];
 #pragma unroll
                 for (int s = 0; s < AL::kSteps32; ++s) {
-                    float v[8];
 #pragma unroll
                     for (int p = 0; p < 4; ++p) {
-                        rotate_pair(op.rel32[s][p], op.ph32[s][p], v[2 * p], v[2 * p + 1]);
-                    }
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) {
+                        float even, odd;
+                        rotate_pair(op.rel32[s][p], op.ph32[s][p], even, odd);
                         uint32_t hi, lo;
-                        split_bf16(v[2 * p], v[2 * p + 1], hi, lo);
-                        b_hi32[s][p] = hi;
-                        b_lo32[s][p] = lo;
+                        split_bf16(even, odd, hi, lo);
+                        b_hi32[u][s][p] = hi;
+                        b_lo32[u][s][p] = lo;
                     }
                 }
-                u32x2 b_hi16[S16];
-                u32x2 b_lo16[S16];
 #pragma unroll
                 for (int s = 0; s < AL::kSteps16; ++s) {
-                    float v[4];
 #pragma unroll
                     for (int p = 0; p < 2; ++p) {
-                        rotate_pair(op.rel16[s][p], op.ph16[s][p], v[2 * p], v[2 * p + 1]);
-                    }
-#pragma unroll
-                    for (int p = 0; p < 2; ++p) {
+                        float even, odd;
+                        rotate_pair(op.rel16[s][p], op.ph16[s][p], even, odd);
                         uint32_t hi, lo;
-                        split_bf16(v[2 * p], v[2 * p + 1], hi, lo);
-                        b_hi16[s][p] = hi;
-                        b_lo16[s][p] = lo;
+                        split_bf16(even, odd, hi, lo);
+                        b_hi16[u][s][p] = hi;
+                        b_lo16[u][s][p] = lo;
                     }
                 }
+            }
+            // The chains of a sub-tile's heads and feature blocks advance
+            // together: each MFMA depends on the one a round before it, and a
+            // wave whose chains ran one after the other waited for each result
+            // (the apply waves, one per SIMD, set the tile's pace: 79.4 -> 74.5
+            // us at 64 x 4,096, rank 32, 62 -> 58 us at 64 x 2,048, rank 48).
+            f32x4 acc[kTogether][NFB];
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u) {
 #pragma unroll
                 for (int f = 0; f < NFB; ++f) {
-                    if (f < a.feature_blocks) {
-                        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+                    acc[u][f] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+                }
+            }
+            const auto round = [&](auto product) {
 #pragma unroll
-                        for (int s = 0; s < AL::kSteps32; ++s) {
-                            acc = mfma16x16x32(op_hi32[u][f][s], b_hi32[s], acc);
-                            acc = mfma16x16x32(op_hi32[u][f][s], b_lo32[s], acc);
-                            acc = mfma16x16x32(op_lo32[u][f][s], b_hi32[s], acc);
-                        }
+                for (int u = 0; u < kTogether; ++u) {
 #pragma unroll
-                        for (int s = 0; s < AL::kSteps16; ++s) {
-                            acc = mfma16x16x16(op_hi16[u][f][s], b_hi16[s], acc);
-                            acc = mfma16x16x16(op_hi16[u][f][s], b_lo16[s], acc);
-                            acc = mfma16x16x16(op_lo16[u][f][s], b_hi16[s], acc);
-                        }
-                        const int64_t feature = h * d + 16 * f + 4 * g;
-                        const u32x2 c = op.con[f];
-                        u32x2 y;
-                        y.x = pack_bf16(fmaf(eta[u], bf16_lo(c.x), acc[0]), fmaf(eta[u], bf16_hi(c.x), acc[1]));
-                        y.y = pack_bf16(fmaf(eta[u], bf16_lo(c.y), acc[2]), fmaf(eta[u], bf16_hi(c.y), acc[3]));
-                        *reinterpret_cast<u32x2*>(mx + r * kMixDPitch + feature) = y;
+                    for (int f = 0; f < NFB; ++f) {
+                        acc[u][f] = product(u, f, acc[u][f]);
                     }
                 }
+            };
+#pragma unroll
+            for (int s = 0; s < AL::kSteps32; ++s) {
+                round([&](int u, int f, const f32x4& c) { return mfma16x16x32(op_hi32[u0 + u][f][s], b_hi32[u][s], c); });
+                round([&](int u, int f, const f32x4& c) { return mfma16x16x32(op_hi32[u0 + u][f][s], b_lo32[u][s], c); });
+                round([&](int u, int f, const f32x4& c) { return mfma16x16x32(op_lo32[u0 + u][f][s], b_hi32[u][s], c); });
+            }
+#pragma unroll
+            for (int s = 0; s < AL::kSteps16; ++s) {
+                round([&](int u, int f, const f32x4& c) { return mfma16x16x16(op_hi16[u0 + u][f][s], b_hi16[u][s], c); });
+                round([&](int u, int f, const f32x4& c) { return mfma16x16x16(op_hi16[u0 + u][f][s], b_lo16[u][s], c); });
+                round([&](int u, int f, const f32x4& c) { return mfma16x16x16(op_lo16[u0 + u][f][s], b_hi16[u][s], c); });
+            }
+            const int r = sub * 16 + q;
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u) {
+#pragma unroll
+                for (int f = 0; f < NFB; ++f) {
+                    const int64_t feature = head(u0 + u) * d + 16 * block(f) + 4 * g;
+                    const u32x2 c = in[u0 + u][sub].con[f];
+                    const f32x4 v = acc[u][f];
+                    u32x2 y;
+                    y.x = pack_bf16(fmaf(eta[u0 + u], bf16_lo(c.x), v[0]), fmaf(eta[u0 + u], bf16_hi(c.x), v[1]));
+                    y.y = pack_bf16(fmaf(eta[u0 + u], bf16_lo(c.y), v[2]), fmaf(eta[u0 + u], bf16_hi(c.y), v[3]));
+                    *reinterpret_cast<u32x2*>(mx + r * kMixDPitch + feature) = y;
+                }
+            }
+            if constexpr (!kReadFirst) {
+                __builtin_amdgcn_sched_barrier(0);   // one slot's operands live at a time
             }
         }
     };
@@ -472,10 +514,10 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
             if (k < n_tiles) {
                 fetch(refill, k + 2);
                 __builtin_amdgcn_sched_barrier(0);
-                apply_tile(k);
-                if (k + 1 < n_tiles) {
-                    commit(next, k + 1);
+                if (has_head) {
+                    apply_tile(k);
                 }
+                commit(next, k + 1);   // zeros past the range
             }
             __syncthreads();
         };
@@ -489,10 +531,10 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
         for (int k = 0; k <= n_tiles; ++k) {
             if (k < n_tiles) {
                 fetch(stage_a, k + 1);
-                apply_tile(k);
-                if (k + 1 < n_tiles) {
-                    commit(stage_a, k + 1);
+                if (has_head) {
+                    apply_tile(k);
                 }
+                commit(stage_a, k + 1);   // zeros past the range
             }
             __syncthreads();
         }
