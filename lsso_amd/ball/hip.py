@@ -328,10 +328,6 @@ def _check(status: int, library: ctypes.CDLL) -> None:
         raise RuntimeError(message)
 
 
-def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
-
-
 def _launch(entry, device: torch.device, *arguments, after: tuple = ()) -> int:
     """entry(*arguments, current stream of ``device``, *after) with that
     device current; the device is only switched where it is not (the switch

@@ -116,15 +116,6 @@ __device__ __forceinline__ u32x4 load_x_chunk(const LinearArgs& a, int64_t row, 
     return out;
 }
 
-template <int YT>
-__device__ __forceinline__ uint16_t to_output_bits(float value) {
-    if constexpr (YT == LSSO_HIP_BF16) {
-        return to_bf16_bits(value);
-    } else {
-        return to_f16_bits(value);
-    }
-}
-
 // VEC: whole 16-byte pieces of x and y (a.x_vector, a.y_vector).
 template <int KSTEPS, int XT, int YT, bool VEC>
 __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a) {
