@@ -1205,6 +1205,19 @@ def project_mix(
     return mixed
 
 
+def _saved(value: torch.Tensor, name: str, dtype: torch.dtype, sizes: tuple, device: torch.device) -> torch.Tensor:
+    """``value`` as the native backward reads it.  A program's saved-tensor
+    hooks (offloading, compression) may hand back another tensor than the
+    one that was saved, so its extent is checked before its pointer is taken."""
+
+    if value.device != device or value.dtype != dtype or value.shape != sizes:
+        raise RuntimeError(
+            f"the saved {name} must be {dtype} {list(sizes)} on {device}, "
+            f"got {value.dtype} {list(value.shape)} on {value.device}"
+        )
+    return value
+
+
 class _Layer(torch.autograd.Function):
     """Autograd of the whole layer run as one native training call
     (lsso_hip_layer_forward_train: input projection, mixer with the tape and
@@ -1235,11 +1248,27 @@ class _Layer(torch.autograd.Function):
          out_weight) = ctx.saved_tensors
         library = _library()
         needs = ctx.needs_input_grad
+        x = x.contiguous()
         shape, mode = _layer_shape(
             x, in_weight, core_base_raw, core_drive_weight, eta_raw, ctx.centered_positions, ctx.valid_counts
         )
         device = x.device
         dim = x.shape[-1]
+        tokens = (shape.batch, shape.length)
+        tape_floats = _plan_size("lsso_hip_mixer_tape_floats", None, *_dims(shape))
+        if x.dtype not in _DTYPE_CODES:
+            raise TypeError("the fused layer supports float16/bfloat16 x")
+        mixed = _saved(mixed.to(torch.bfloat16), "mixed", torch.bfloat16, (*tokens, dim), device).contiguous()
+        _saved(in_weight, "in_weight", torch.float32, (in_weight.shape[0], dim), device)
+        _saved(out_weight, "out_weight", torch.float32, (dim, dim), device)
+        if row_mask is not None:
+            _saved(row_mask, "row_mask", torch.bool, tokens, device)
+        for name, value, dtype, sizes in (
+            ("packed", packed, torch.bfloat16, (*tokens, in_weight.shape[0])),
+            ("tape", tape, torch.float32, (tape_floats,)),
+        ):
+            if not _saved(value, name, dtype, sizes, device).is_contiguous():
+                raise RuntimeError(f"the saved {name} must be contiguous")
         flat_grad = _rows(grad_y, dim)
         if flat_grad.dtype not in _DTYPE_CODES:
             flat_grad = flat_grad.to(dtype=torch.bfloat16).contiguous()

@@ -92,6 +92,56 @@ def test_layers_with_more_parameters_are_checked_in_full(native) -> None:
         layer(x, implementation="hip")
 
 
+@pytest.mark.gpu
+def test_saved_tensor_hooks(native) -> None:
+    """Saved tensors that hooks hand back are read as they are: offloaded and
+    strided copies give the same gradients, tensors of another type, size or
+    device are refused before any kernel runs."""
+
+    layer = _layer(64, 2, 16, True)
+    x = torch.randn(2, 70, 64, device="cuda", dtype=torch.float16).requires_grad_()
+    mask = torch.arange(70, device="cuda")[None, :] < torch.tensor([[70], [31]], device="cuda")
+    dy = torch.randn_like(x)
+    wanted = [x, *layer.parameters()]
+
+    def gradients(pack, unpack):
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            y = layer(x, valid_mask=mask, implementation="hip")
+        return torch.autograd.grad(y, wanted, dy)
+
+    expected = gradients(lambda t: t, lambda t: t)
+
+    def strided(t):
+        keeps = t.dim() == 1 or t.shape[-1] == 2 * 16 + 64 or t.shape[-1] == 16   # packed, tape and compact parameters
+        return t if keeps else t.transpose(-1, -2).contiguous().transpose(-1, -2)
+
+    for pack, unpack in ((lambda t: t.cpu(), lambda t: t.cuda()), (lambda t: t, strided)):
+        for a, b in zip(gradients(pack, unpack), expected):
+            assert torch.equal(a, b)
+    # packed: another type, fewer rows, the host; tape: cut short; W_o: another type; x: another type.
+    packed = lambda t: t.dim() == 3 and t.shape[-1] == 2 * 16 + 64
+    tape = lambda t: t.dim() == 1 and t.numel() > 2
+    changes = (
+        (packed, lambda t: t.float()), (packed, lambda t: t[:1]), (packed, lambda t: t.cpu()), (tape, lambda t: t[:-1]),
+        (lambda t: tuple(t.shape) == (64, 64), lambda t: t.bfloat16()),
+        (lambda t: t.dtype == torch.float16, lambda t: t.float()),
+    )
+    for match, change in changes:
+        with pytest.raises((RuntimeError, TypeError)):
+            gradients(lambda t: t, lambda t, m=match, c=change: c(t) if m(t) else t)
+
+
+def test_saved_extents_are_checked() -> None:
+    from lsso_amd.ball import hip
+
+    value = torch.zeros(2, 3)
+    assert hip._saved(value, "tape", torch.float32, (2, 3), value.device) is value
+    for dtype, sizes, device in ((torch.float16, (2, 3), "cpu"), (torch.float32, (2, 4), "cpu"),
+                                 (torch.float32, (2, 3), "meta")):
+        with pytest.raises(RuntimeError, match="saved tape"):
+            hip._saved(value, "tape", dtype, sizes, torch.device(device))
+
+
 def test_layer_backward_rejects_bad_arguments() -> None:
     """Host-side validation of the C entry (no launch, no GPU)."""
 
