@@ -439,8 +439,10 @@ int lsso_hip_layer_backward(const lsso_hip_mixer_shape* shape, const void* grad_
 #define LSSO_HIP_IDS_F32 3
 #define LSSO_HIP_IDS_F64 4
 
-/* Longest row lsso_hip_center_positions takes (one workgroup walks it). */
+/* Longest row lsso_hip_center_positions takes (one workgroup of 1,024 threads
+ * walks it), and most rows (a launch takes fewer than 2^32 threads). */
 #define LSSO_HIP_CENTER_MAX_LENGTH 65536
+#define LSSO_HIP_CENTER_MAX_ROWS 4194303
 
 /* Centred positions and valid counts of the mixer, in one launch.
  * valid_mask: uint8 [rows, length] contiguous or NULL (all valid).

@@ -37,6 +37,7 @@ _POSITIONS_DEFAULT = 0
 _POSITIONS_SHARED = 1
 _POSITIONS_BATCHED = 2
 _CENTER_MAX_LENGTH = 65536
+_CENTER_MAX_ROWS = 4194303
 _ID_TYPES = {torch.int32: 1, torch.int64: 2, torch.float32: 3, torch.float64: 4}
 
 _SYMBOLS = (
@@ -495,11 +496,21 @@ def center_positions(
     The values of LSSO._center_positions (reference model.py:163-243), the
     mean from an FP64 sum.
 
-    None where the kernel does not apply: rows longer than
-    ``_CENTER_MAX_LENGTH`` (one workgroup walks a row), and ids of another
-    type, shape or device, which the tensor path converts or rejects."""
+    ``valid_mask``: bool [B, N] on ``device``.  None where the kernel does not
+    apply: rows longer than ``_CENTER_MAX_LENGTH`` or more than
+    ``_CENTER_MAX_ROWS`` (one workgroup of 1,024 threads walks a row, a launch
+    takes fewer than 2^32 threads), and ids of another type, shape or device,
+    which the tensor path converts or rejects."""
 
-    if length > _CENTER_MAX_LENGTH or (position_ids is None and valid_mask is None):
+    if device.type != "cuda":
+        raise RuntimeError("device must be a CUDA (ROCm) device")
+    if device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    if valid_mask is not None:
+        if valid_mask.dtype != torch.bool or valid_mask.shape != (batch, length):
+            raise ValueError("valid_mask must be a bool [B, N] tensor")
+        _require_device_tensor(valid_mask, "valid_mask", device)
+    if length > _CENTER_MAX_LENGTH or batch > _CENTER_MAX_ROWS or (position_ids is None and valid_mask is None):
         return None
     rows, kind, ids, batch_stride, token_stride = batch, 0, None, 0, 0
     if position_ids is not None:

@@ -217,9 +217,10 @@ int lsso_hip_center_positions(const uint8_t* valid_mask, const void* position_id
     if (rows <= 0 || length <= 0) {
         return fail(LSSO_HIP_EINVAL, "rows and length must be positive");
     }
-    if (length > LSSO_HIP_CENTER_MAX_LENGTH || rows > INT32_MAX) {
-        return fail(LSSO_HIP_EUNSUPPORTED, "center_positions takes rows of up to " +
-                                               std::to_string(LSSO_HIP_CENTER_MAX_LENGTH) + " tokens");
+    if (length > LSSO_HIP_CENTER_MAX_LENGTH || rows > LSSO_HIP_CENTER_MAX_ROWS) {
+        return fail(LSSO_HIP_EUNSUPPORTED, "center_positions takes up to " + std::to_string(LSSO_HIP_CENTER_MAX_ROWS) +
+                                               " rows of up to " + std::to_string(LSSO_HIP_CENTER_MAX_LENGTH) +
+                                               " tokens");
     }
     if (position_type < LSSO_HIP_IDS_NONE || position_type > LSSO_HIP_IDS_F64) {
         return fail(LSSO_HIP_EINVAL, "position_type must be one of LSSO_HIP_IDS_*");

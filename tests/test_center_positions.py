@@ -118,6 +118,44 @@ def test_center_positions_rejects_bad_arguments() -> None:
     call = library.lsso_hip_center_positions
     assert call(None, None, 0, 0, 0, 1, 0, 256, None, None) == -1
     assert call(None, None, 0, 0, 0, 1, 65537, 256, None, None) == -2
+    assert call(None, None, 0, 0, 0, 1 << 22, 1, 256, None, None) == -2      # 2^32 threads
     assert call(None, None, 2, 0, 1, 1, 8, 256, None, None) == -1
     assert call(256, None, 0, 0, 0, 1, 8, 256, None, None) == -1
     assert call(None, 256, 9, 0, 1, 1, 8, 256, None, None) == -1
+
+
+@pytest.mark.parametrize(("mask", "error"), (
+    (torch.ones(4, dtype=torch.bool), ValueError),                    # [N], not broadcast
+    (torch.ones(1, 4, dtype=torch.bool), ValueError),                 # [1, N], not broadcast
+    (torch.ones(3, 2, dtype=torch.bool), ValueError),                 # shorter rows
+    (torch.ones(3, 4), ValueError),                                   # read bytewise otherwise
+    (torch.ones(3, 4, dtype=torch.int64), ValueError),
+    (torch.ones(3, 4, dtype=torch.uint8), ValueError),
+    (torch.ones(3, 4, dtype=torch.bool), RuntimeError),               # on the host
+))
+def test_center_positions_rejects_other_masks(mask, error) -> None:
+    """A mask is read as batch x length bytes on the device, so its type,
+    shape and device are checked before its pointer is taken (no launch, no
+    GPU)."""
+
+    from lsso_amd.ball import hip
+
+    with pytest.raises(error, match="valid_mask"):
+        hip.center_positions(None, mask, 3, 4, torch.device("cuda", 0))
+
+
+def test_center_positions_rejects_other_devices() -> None:
+    from lsso_amd.ball import hip
+
+    with pytest.raises(RuntimeError, match="device"):
+        hip.center_positions(None, torch.ones(3, 4, dtype=torch.bool), 3, 4, torch.device("cpu"))
+    with pytest.raises(RuntimeError, match="device"):
+        hip.center_positions(torch.arange(4), None, 3, 4, torch.device("cpu"))
+
+
+@pytest.mark.gpu
+def test_center_positions_takes_a_device_without_index(native) -> None:
+    mask = torch.tensor([[True, False, True, True]], device="cuda")
+    centered, counts = native.center_positions(None, mask, 1, 4, torch.device("cuda"))
+    assert counts.tolist() == [3.0]
+    assert torch.allclose(centered.cpu(), torch.tensor([[-5.0, 0.0, 1.0, 4.0]]) / 3.0)
