@@ -1598,8 +1598,9 @@ __global__ __launch_bounds__(kBwdStagedWaves * 64, 2) void bwd_apply_staged_kern
             *reinterpret_cast<u32x2*>(orow + con_col + unit * D + f0) = packed;
         }
         if (a.column_part != nullptr) {
-            // The wave's own tile rows: its reads follow its writes in order.
-            // Rows past the chunk are zero, as their inputs are.
+            // The wave's own tile rows, written by other lanes; rows past the
+            // chunk are zero, as their inputs are.
+            wave_lds_order();
             const uint16_t* sums = &s_out[obuf][(4 * g + q / 4) * out_pitch + 4 * (q % 4)];
 #pragma unroll
             for (int i = 0; i < kSumBlocks; ++i) {

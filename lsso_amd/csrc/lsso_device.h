@@ -48,6 +48,13 @@ __device__ __forceinline__ float f16_bits_to_float(uint16_t bits) {
     return static_cast<float>(__builtin_bit_cast(_Float16, bits));
 }
 
+// LDS ordering between lanes of one wave: its LDS instructions execute in
+// issue order, so only the compiler must be kept from reordering.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The value unchanged, but opaque to the optimizer: lane-dependent offsets
 // computed from it stay next to their use inside a loop instead of being
 // hoisted out of it and held in registers across the whole loop.
@@ -298,13 +305,14 @@ __device__ __forceinline__ void load_weight_rows(u32x4 (&wreg)[NB][KSTEPS], Buff
         if (i + kRing < kTotal) {
             issue(i + kRing);
         }
-        // LDS operations of one wave execute in order: these reads see the
-        // writes above, and the next piece's writes follow them.
+        // Written and read by different lanes of the wave.
+        wave_lds_order();
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             wreg[i / kPieces][2 * (i % kPieces) + s] = *reinterpret_cast<const u32x4*>(
                 scratch + (lane & 31) * kWeightPitch + 16 * s + 8 * (lane >> 5));
         }
+        wave_lds_order();   // the next piece's writes follow these reads
         __builtin_amdgcn_sched_barrier(0);
     }
 }

@@ -217,8 +217,7 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
                         *reinterpret_cast<u32x2*>(stage + lane_c * kMixStPitch + c) = packed;
                     }
                 }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                wave_lds_order();
                 const BufferRsrc ybuf = make_buffer(
                     static_cast<uint16_t*>(a.y) + (b * a.length + tile_t0(t)) * D, int64_t{2} * tile_rows(t) * Di);
 #pragma unroll

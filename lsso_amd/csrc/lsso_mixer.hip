@@ -487,13 +487,6 @@ __device__ __forceinline__ void unroll_to(F&& f) {
     }
 }
 
-// LDS ordering between lanes of one wave: its LDS instructions execute in
-// issue order, so only the compiler must be kept from reordering.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Cholesky factor of an R-column block of an SPD matrix whose rows are held
 // one per lane in l (the block's R diagonal rows in lanes 0 .. R - 1, rows
 // below the block in the lanes after them, zero rows past the matrix), by
