@@ -504,9 +504,8 @@ int run_linear(const void* x, int x_dtype, int64_t rows, int64_t in_features,
     args.y = y;
     args.tiles = ceil_div(rows, lsso_hip::linear_tile_rows(tier));
     args.column_groups = ceil_div(out_features, lsso_hip::linear_columns_per_group(tier));
-    args.x_vector = (in_features % 8 == 0 && x_row_stride % 8 == 0 && aligned(x, 16)) ? 1 : 0;
-    args.w_vector = (in_features % 4 == 0 && aligned(weight, 16)) ? 1 : 0;
-    args.y_vector = (out_features % 8 == 0 && aligned(y, 16)) ? 1 : 0;
+    args.vector = (in_features % 8 == 0 && x_row_stride % 8 == 0 && aligned(x, 16) && out_features % 8 == 0 &&
+                   aligned(y, 16)) ? 1 : 0;
     int64_t groups = units / args.column_groups;
     // With several column groups, a whole number of XCD rounds lets the
     // kernel deal the column groups of one row tile to one XCD, so x is

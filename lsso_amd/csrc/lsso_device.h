@@ -119,6 +119,46 @@ __device__ __forceinline__ void buffer_store16_stream(u32x4 value, BufferRsrc bu
                                            buffer, offset, 0, 2 | 16);
 }
 
+// Pieces of rows that are not whole 16-byte pieces (odd lengths, strides or
+// bases).  A piece is one 16-byte access at an address aligned to its elements
+// only: it starts early enough to end within its row, so that it never leaves
+// the matrix, and is moved down by the elements it started early, which brings
+// zeros in past the row's end.  Element by element, a piece took eight loads,
+// eight registers in flight and eight conditional addresses.
+__device__ __forceinline__ u32x4 load16_unaligned(const void* at) {
+    u32x4 v;
+    __builtin_memcpy(&v, at, sizeof(v));
+    return v;
+}
+__device__ __forceinline__ void store16_unaligned(void* at, const u32x4& v) {
+    __builtin_memcpy(at, &v, sizeof(v));
+}
+// First element of the access to elements k .. k + N - 1 of a row of `cols` >= N.
+template <int N, typename I>
+__device__ __forceinline__ I piece_start(I k, I cols) {
+    return k < cols - N ? k : cols - N;
+}
+__device__ __forceinline__ u32x4 drop_dwords(const u32x4& v, uint32_t count) {   // zeros from 4 on
+    u32x4 out = (count & 2) != 0 ? (u32x4){v[2], v[3], 0u, 0u} : v;
+    out = (count & 1) != 0 ? (u32x4){out[1], out[2], out[3], 0u} : out;
+    return count < 4 ? out : (u32x4){0u, 0u, 0u, 0u};
+}
+// 16-bit elements k .. k + 7 from the access at piece_start<8>(k, cols).
+template <typename I>
+__device__ __forceinline__ u32x4 align_piece16(const u32x4& raw, I k, I cols) {
+    const I start = piece_start<8>(k, cols);
+    const uint32_t early = k - start < 8 ? static_cast<uint32_t>(k - start) : 8u;
+    const u32x4 v = drop_dwords(raw, early >> 1);
+    const u32x4 odd = {(v[0] >> 16) | (v[1] << 16), (v[1] >> 16) | (v[2] << 16), (v[2] >> 16) | (v[3] << 16), v[3] >> 16};
+    return (early & 1) != 0 ? odd : v;
+}
+// 32-bit elements k .. k + 3 from the access at piece_start<4>(k, cols).
+template <typename I>
+__device__ __forceinline__ u32x4 align_piece32(const u32x4& raw, I k, I cols) {
+    const I start = piece_start<4>(k, cols);
+    return drop_dwords(raw, k - start < 4 ? static_cast<uint32_t>(k - start) : 4u);
+}
+
 // Round two floats to BF16 (round to nearest even, v_cvt_pk_bf16_f32) and
 // pack them, first value in the low half.
 __device__ __forceinline__ uint32_t pack_bf16(float low, float high) {
@@ -214,55 +254,30 @@ struct ApplyLayout {
     __device__ static constexpr int offset16(int s) { return 8 * s; }
 };
 
-// Resident BF16 row of an FP32 weight [N, K] for y^T = W x^T on
-// v_mfma_f32_32x32x16_bf16: the lane holds row n (zeros when n < 0) at
-// columns 16 ks + 8 (lane / 32) + 0..7, RNE-rounded, zero past K.  Element
-// loads, for weights that load_weight_rows does not take (K not a multiple of
-// 4, or a base that is not 16-byte aligned).
-template <int KSTEPS>
-__device__ __forceinline__ void load_weight_row(u32x4 (&wreg)[KSTEPS], const float* weight,
-                                                int64_t n, int64_t K, int lane) {
-    const float* wrow = weight + (n >= 0 ? n : 0) * K;
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-        const int k0 = 16 * ks + 8 * (lane >> 5);
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const bool live = n >= 0 && k0 + i < K;
-            const float value = wrow[live ? k0 + i : 0];
-            v[i] = live ? value : 0.0f;
-        }
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            wreg[ks][p] = pack_bf16(v[2 * p], v[2 * p + 1]);
-        }
-        // One K step at a time: keeps the FP32 staging of W from being
-        // hoisted next to the whole BF16 slice.
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-// load_weight_row of NB x 32 rows for K a multiple of 4, coalesced: 8 lanes
-// read one row's 32 columns (one 128-byte line) per 16-byte load, the BF16
-// values pass through `scratch` (kWeightScratch bf16 of LDS of this wave's
+// Resident BF16 rows of an FP32 weight [N, K] for y^T = W x^T on
+// v_mfma_f32_32x32x16_bf16: NB x 32 rows of which lane i holds row i % 32 at
+// columns 16 ks + 8 (i / 32) + 0..7, RNE-rounded, zero past K.  Coalesced: 8
+// lanes read one row's 32 columns (one 128-byte line) per 16-byte load, the
+// BF16 values pass through `scratch` (kWeightScratch bf16 of LDS of this wave's
 // own, so no barrier) and come back in the lane layout.  row_offset(nb, r) is
-// the byte offset of row r of block nb in the raw buffer, or kOutOfRange;
-// columns past K read as zeros.  A persistent kernel cannot start its first
-// tile before its weights are in registers.  Read by the lanes that keep them
-// (row n at 16 bytes per lane, one K step at a time, as load_weight_row does),
-// every load touches 32 lines for a quarter of their bytes and waits for the
-// one before; with eight steps in flight instead, the lines of all waves no
-// longer fit the L1 and are fetched four times (the training step at 262,144
-// tokens 4% slower).  Four 2-step pieces are in flight here; the scheduling
-// barriers keep the FP32 staging of the whole slice from being live at once.
-// With it the layer call at 64 x 1,024 x 256 (rank 32) takes 84 us instead of
-// 92, at 64 x 4,096 212 instead of 221; and the fused kernels, which spilled 12
-// to 36 registers around the per-lane addresses, spill none.
+// the byte offset of row r of block nb in the raw buffer, or kOutOfRange.
+// WHOLE: rows of whole 4-column pieces (K a multiple of 4); else K is at least
+// 4 and the last piece of a row is read from 4 columns before its end.  A
+// buffer access of several dwords needs dword alignment only, so any FP32
+// weight will do.  A persistent kernel cannot start its first tile before its
+// weights are in registers.  Read by the lanes that keep them (row n at 16
+// bytes per lane, one K step at a time), every load touches 32 lines for a
+// quarter of their bytes and waits for the one before; with eight steps in
+// flight instead, the lines of all waves no longer fit the L1 and are fetched
+// four times (the training step at 262,144 tokens 4% slower).  Four 2-step
+// pieces are in flight here; the scheduling barriers keep the FP32 staging of
+// the whole slice from being live at once.  With it the layer call at 64 x
+// 1,024 x 256 (rank 32) takes 84 us instead of 92, at 64 x 4,096 212 instead of
+// 221.
 constexpr int kWeightPitch = 40;                      // bf16 per row of 32: 16 rows' 16-byte reads cover all banks
 constexpr int kWeightScratch = 32 * kWeightPitch;     // bf16 per wave
 constexpr int kWeightRing = 4;
-template <int NB, int KSTEPS, typename RowOffset>
+template <bool WHOLE, int NB, int KSTEPS, typename RowOffset>
 __device__ __forceinline__ void load_weight_rows(u32x4 (&wreg)[NB][KSTEPS], BufferRsrc buffer, RowOffset row_offset,
                                                  int64_t K, int lane, uint16_t* scratch) {
     static_assert(KSTEPS % 2 == 0, "a piece is two K steps");
@@ -281,12 +296,14 @@ __device__ __forceinline__ void load_weight_rows(u32x4 (&wreg)[NB][KSTEPS], Buff
         }
     }
     u32x4 raw[kRing][4];
+    const auto start = [&](uint32_t k0) { return WHOLE ? k0 : piece_start<4>(k0, k_end); };
     auto issue = [&](int i) {
         const uint32_t k0 = 32 * (i % kPieces) + k_lane;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const uint32_t row = offset[i / kPieces][j];
-            raw[i % kRing][j] = buffer_load16(buffer, k0 < k_end && row != kOutOfRange ? row + 4 * k0 : kOutOfRange);
+            raw[i % kRing][j] =
+                buffer_load16(buffer, k0 < k_end && row != kOutOfRange ? row + 4 * start(k0) : kOutOfRange);
         }
     };
 #pragma unroll
@@ -298,7 +315,9 @@ __device__ __forceinline__ void load_weight_rows(u32x4 (&wreg)[NB][KSTEPS], Buff
     for (int i = 0; i < kTotal; ++i) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const f32x4 v = __builtin_bit_cast(f32x4, raw[i % kRing][j]);
+            const u32x4 piece = raw[i % kRing][j];
+            const f32x4 v = __builtin_bit_cast(
+                f32x4, WHOLE ? piece : align_piece32<uint32_t>(piece, 32 * (i % kPieces) + k_lane, k_end));
             const u32x2 packed = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
             *reinterpret_cast<u32x2*>(scratch + (8 * j + row8) * kWeightPitch + k_lane) = packed;
         }
@@ -317,20 +336,19 @@ __device__ __forceinline__ void load_weight_rows(u32x4 (&wreg)[NB][KSTEPS], Buff
     }
 }
 
-// Resident slice of rows n0 .. n0 + 31 (one row per lane % 32); vector: K is
-// a multiple of 4 and the weight 16-byte aligned; n0 is wave-uniform.
+// load_weight_rows of rows n0 .. n0 + 31 (n0 wave-uniform; rows past N are
+// zeros); whole: K is a multiple of 4.
 template <int KSTEPS>
 __device__ __forceinline__ void load_weight_slice(u32x4 (&wreg)[1][KSTEPS], const float* weight,
-                                                  int64_t N, int64_t K, int64_t n0, int lane, bool vector,
+                                                  int64_t N, int64_t K, int64_t n0, int lane, bool whole,
                                                   uint16_t* scratch) {
-    if (vector) {   // uniform
-        const int64_t rows = N - n0 < 32 ? N - n0 : 32;
-        const auto row_offset = [&](int, int r) { return static_cast<uint32_t>(4 * r * K); };
-        load_weight_rows<1, KSTEPS>(wreg, make_buffer(weight + (n0 < N ? n0 : 0) * K, 4 * rows * K), row_offset,
-                                    K, lane, scratch);
+    const int64_t rows = N - n0 < 32 ? N - n0 : 32;
+    const BufferRsrc buffer = make_buffer(weight + (n0 < N ? n0 : 0) * K, 4 * rows * K);
+    const auto row_offset = [&](int, int r) { return static_cast<uint32_t>(4 * r * K); };
+    if (whole) {   // uniform
+        load_weight_rows<true, 1, KSTEPS>(wreg, buffer, row_offset, K, lane, scratch);
     } else {
-        const int64_t n = n0 + (lane & 31);
-        load_weight_row<KSTEPS>(wreg[0], weight, n < N ? n : -1, K, lane);
+        load_weight_rows<false, 1, KSTEPS>(wreg, buffer, row_offset, K, lane, scratch);
     }
 }
 

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
         const int ksteps = (Di + 15) / 16;
         u32x4 wreg[2][kMixKSteps];
         static_assert(kMixRows * kMixStPitch >= kWeightScratch, "the output stage holds the weight scratch");
-        load_weight_rows<2, kMixKSteps>(
+        load_weight_rows<true, 2, kMixKSteps>(
             wreg, make_buffer(a.weight, 4 * D * D),
             [&](int nb, int r) {
                 const int n = n0 + 32 * nb + r;

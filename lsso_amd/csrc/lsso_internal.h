@@ -215,9 +215,7 @@ struct LinearArgs {
     void* y;
     int64_t tiles;              // ceil(rows / tile_rows)
     int64_t column_groups;
-    int x_vector;               // 16-byte x loads are legal
-    int w_vector;               // 16-byte W loads are legal (K % 4 == 0, W 16-byte aligned)
-    int y_vector;               // 16-byte y stores are legal
+    int vector;                 // x and y rows are whole aligned 16-byte pieces
 };
 
 // Upstream-gradient pass of the projection's backward: BF16 copy and FP32

@@ -26,6 +26,16 @@
 // 256 outputs.  Before and now (us): 262,144 x 256 -> 256 68 / 57, x 512 -> 256
 // 142 / 98, 131,072 x 640 -> 256 79 / 55, x 256 -> 640 84 / 68, x 384 -> 768
 // 111 / 97.
+//
+// Rows, strides, bases and outputs that are not whole aligned 16-byte pieces
+// run the same loop (a second instantiation) on pieces aligned to their
+// elements.  Element by element (eight loads and eight addresses a piece beside
+// the resident W) that form spilled 25 to 187 registers, and one odd operand
+// put all of them on it.  Element loads with W shared by two waves from K =
+// 385, the former element loads, these pieces (us, 65,536 rows): 256 -> 260
+// 55 / 68 / 34, 300 -> 300 185 / 228 / 41, 640 -> 260 75 / 209 / 53, 256 -> 256
+// at an odd stride 38 / 46 / 20; K-streaming, 16,384 rows: 768 -> 1,001 88 /
+// 276 / 58, 1,001 -> 768 307 / 222 / 61.
 
 #include "lsso_device.h"
 #include "lsso_internal.h"
@@ -81,42 +91,55 @@ __device__ __forceinline__ u32x4 to_bf16_piece(const u32x4& raw) {
     return out;
 }
 
-// Load 8 consecutive x elements as BF16, for shapes outside the vector form
-// of the kernel: one 16-byte piece where x allows it (only y does not), else
-// one element at a time.  Out-of-range rows and columns
-// read a clamped in-bounds address and are zeroed by select.  Masked rows are
-// loaded like any other: the output rows they feed are zeroed in the epilogue.
-template <int XT>
-__device__ __forceinline__ u32x4 load_x_chunk(const LinearArgs& a, int64_t row, int64_t k0) {
-    const int64_t safe_row = row < a.rows ? row : a.rows - 1;
-    const uint16_t* x = static_cast<const uint16_t*>(a.x) + safe_row * a.x_stride;
-    if (a.x_vector) {
-        const bool live = row < a.rows && k0 < a.in_features;
-        const u32x4 raw = *reinterpret_cast<const u32x4*>(x + (live ? k0 : 0));
-        return live ? to_bf16_piece<XT>(raw) : u32x4{};
-    }
-    float v[8];
+// Rows of fewer than 8 elements, which hold no whole piece: element loads.
+__device__ __forceinline__ u32x4 load_short_piece(const uint16_t* row, int k0, int K) {
+    u32x4 out = {0u, 0u, 0u, 0u};
+    if (k0 == 0) {
+        for (int i = 0; i < K; ++i) {
+            const uint32_t bits = static_cast<uint32_t>(row[i]) << (16 * (i & 1));
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const bool live = row < a.rows && k0 + i < a.in_features;
-        const uint16_t bits = x[live ? k0 + i : 0];
-        float value;
-        if constexpr (XT == LSSO_HIP_BF16) {
-            value = bf16_bits_to_float(bits);
-        } else {
-            value = f16_bits_to_float(bits);
+            for (int p = 0; p < 4; ++p) {
+                out[p] |= p == i / 2 ? bits : 0u;
+            }
         }
-        v[i] = live ? value : 0.0f;
-    }
-    u32x4 out;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        out[p] = pack_bf16(v[2 * p], v[2 * p + 1]);
     }
     return out;
 }
+template <int KSTEPS>
+__device__ __forceinline__ void load_short_weights(u32x4 (&wreg)[1][KSTEPS], const float* weight, int64_t N, int K,
+                                                   int64_t n, int lane) {
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+        wreg[0][ks] = (u32x4){0u, 0u, 0u, 0u};
+    }
+    if (lane < 32 && n < N) {
+        for (int i = 0; i < K; ++i) {
+            const uint32_t bits = static_cast<uint32_t>(to_bf16_bits(weight[n * K + i])) << (16 * (i & 1));
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                wreg[0][0][p] |= p == i / 2 ? bits : 0u;
+            }
+        }
+    }
+}
 
-// VEC: whole 16-byte pieces of x and y (a.x_vector, a.y_vector).
+// A 16-byte piece of an output row at column n, of which the row may hold
+// fewer than eight elements.
+__device__ __forceinline__ void store_piece(uint16_t* row, int64_t n, int64_t N, const u32x4& v) {
+    if (n + 8 <= N) {
+        store16_unaligned(row + n, v);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            if (n + r < N) {
+                row[n + r] = static_cast<uint16_t>(v[r >> 1] >> (16 * (r & 1)));
+            }
+        }
+    }
+}
+
+// VEC: whole 16-byte pieces of x and y (a.vector); else pieces aligned to their
+// elements (x) and stores of whole or part pieces (y).
 template <int KSTEPS, int XT, int YT, bool VEC>
 __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a) {
     constexpr int kWaves = kLinearWaves;
@@ -165,15 +188,20 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
     // written before the first tile's products.
     constexpr bool kStageHolds = kTileRows * YP >= kWaves * kWeightScratch;
     static_assert(kStageHolds || kTileRows * KP >= kWaves * kWeightScratch, "weight scratch");
-    load_weight_slice<KSTEPS>(wreg, a.weight, N, K, n0, lane, a.w_vector != 0,
-                              (kStageHolds ? s_y : s_x[1]) + wave * kWeightScratch);
+    // Rows too short for a piece: only where they would be the lowest tier's.
+    const bool short_rows = !VEC && KSTEPS == 4 && K < 8;   // uniform
+    if (short_rows) {
+        load_short_weights<KSTEPS>(wreg, a.weight, N, static_cast<int>(K), n0 + (lane & 31), lane);
+    } else {
+        load_weight_slice<KSTEPS>(wreg, a.weight, N, K, n0, lane, VEC || K % 4 == 0,
+                                  (kStageHolds ? s_y : s_x[1]) + wave * kWeightScratch);
+    }
     for (int c = tid; c < kGroupColumns; c += kThreads) {
         const int64_t n = cg * kGroupColumns + c;
         s_bias[c] = (a.bias != nullptr && n < N) ? a.bias[n] : 0.0f;
     }
 
-    // One tile of x in flight: 16-byte pieces as loaded (BF16 already without
-    // VEC) and the row's mask byte.  Row flags travel with their x: thread r <
+    // One tile of x in flight: 16-byte pieces as loaded and the row's mask byte.  Row flags travel with their x: thread r <
     // kTileRows reads the byte of row r through a raw buffer over the tile's
     // valid rows (rows past the matrix, and every row when there is no mask,
     // read as zero without an access).
@@ -190,7 +218,8 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
     const uint32_t piece_step = piece_k < K ? 2u * static_cast<uint32_t>(kThreads / kChunksPerRow) *
                                                   static_cast<uint32_t>(a.x_stride) : 0u;
     auto load_chunk = [&](Stage& stage, int64_t t, BufferRsrc buffer, int c) {
-        const int chunk = tid + c * kThreads;
+        // Without VEC, a piece's place is worked out where it is used.
+        const int chunk = VEC ? tid + c * kThreads : opaque_int(tid + c * kThreads);
         const int rr = chunk / kChunksPerRow;
         const int k0 = 8 * (chunk - rr * kChunksPerRow);
         if constexpr (VEC) {
@@ -205,7 +234,11 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
                     buffer, k0 < K ? 2u * static_cast<uint32_t>(rr_c * static_cast<int>(a.x_stride) + k0) : kOutOfRange);
             }
         } else {
-            stage.x[c] = load_x_chunk<XT>(a, t * kTileRows + rr, k0);
+            // Rows past the matrix read its last row: their outputs are not stored.
+            const int64_t row = t * kTileRows + rr < a.rows ? t * kTileRows + rr : a.rows - 1;
+            const uint16_t* at = x + row * a.x_stride;
+            const int cols = static_cast<int>(K);
+            stage.x[c] = short_rows ? load_short_piece(at, k0, cols) : load16_unaligned(at + piece_start<8>(k0, cols));
         }
     };
     auto tile_buffer = [&](int64_t t) {
@@ -226,10 +259,11 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
         load_flags(stage, t);
     };
     auto write_chunk = [&](const Stage& stage, int buf, int c) {
-        const int chunk = tid + c * kThreads;
+        const int chunk = VEC ? tid + c * kThreads : opaque_int(tid + c * kThreads);
         const int rr = chunk / kChunksPerRow;
         const int cc = chunk - rr * kChunksPerRow;
-        *reinterpret_cast<u32x4*>(&s_x[buf][rr * KP + 8 * cc]) = VEC ? to_bf16_piece<XT>(stage.x[c]) : stage.x[c];
+        const u32x4 piece = VEC || short_rows ? stage.x[c] : align_piece16(stage.x[c], 8 * cc, static_cast<int>(K));
+        *reinterpret_cast<u32x4*>(&s_x[buf][rr * KP + 8 * cc]) = to_bf16_piece<XT>(piece);
     };
     auto write_flags = [&](const Stage& stage, int buf) {
         if (tid < kTileRows) {
@@ -244,8 +278,6 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
     // operations complete in issue order as far as the wait counter is
     // concerned and nothing here is conditional, so each wait covers that one
     // stage only: the stage behind it and the y stores stay in flight.
-    // Without VEC, `ahead` is the next tile, loaded before the products and
-    // written after them.
     auto step = [&](int buf, int64_t tile, Stage& stage, int64_t ahead) {
         bool keep[MB];
 #pragma unroll
@@ -282,9 +314,6 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
             }
         };
         const BufferRsrc buffer = tile_buffer(ahead);
-        if constexpr (!VEC) {
-            load_stage(stage, ahead);
-        }
         read_group(0, 0);
 #pragma unroll
         for (int g = 0; g < kGroups; ++g) {
@@ -302,7 +331,7 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
             // This group's share of the next tile's pieces.
 #pragma unroll
             for (int c = 0; c < kChunksPerThread; ++c) {
-                if (VEC && c * kGroups / kChunksPerThread == g) {
+                if (c * kGroups / kChunksPerThread == g) {
                     write_chunk(stage, buf ^ 1, c);
                     load_chunk(stage, ahead, buffer, c);
                 }
@@ -315,16 +344,8 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (VEC) {
-            write_flags(stage, buf ^ 1);
-            load_flags(stage, ahead);
-        } else {
-#pragma unroll
-            for (int c = 0; c < kChunksPerThread; ++c) {
-                write_chunk(stage, buf ^ 1, c);
-            }
-            write_flags(stage, buf ^ 1);
-        }
+        write_flags(stage, buf ^ 1);
+        load_flags(stage, ahead);
         // y^T block: lane holds row m = lane%32 of the 32-row block and
         // features n0 + 8 q + 4 half + r for q, r in 0..3.  The tile is
         // rounded and staged in LDS, then written back row by row so that
@@ -381,18 +402,8 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
                 const int64_t m = tile * kTileRows + mr;
                 const int64_t n = col0 + c8;
                 if (m < a.rows && n < N) {
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(&s_y[mr * YP + c8]);
-                    uint16_t* dst = static_cast<uint16_t*>(a.y) + m * N + n;
-                    if (a.y_vector) {
-                        *reinterpret_cast<u32x4*>(dst) = v;
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 8; ++r) {
-                            if (n + r < N) {
-                                dst[r] = static_cast<uint16_t>(v[r >> 1] >> (16 * (r & 1)));
-                            }
-                        }
-                    }
+                    store_piece(static_cast<uint16_t*>(a.y) + m * N, n, N,
+                                *reinterpret_cast<const u32x4*>(&s_y[mr * YP + c8]));
                 }
             }
         }
@@ -403,9 +414,10 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
     if (tile >= a.tiles) {
         return;
     }
-    // Stages of x in flight: two where the registers hold them beside W.
-    constexpr int kSets = VEC && KSTEPS <= 32 ? 2 : 1;
-    constexpr int kAhead = VEC ? kSets + 1 : 1;
+    // Stages of x in flight: two where the registers hold them beside W and,
+    // without VEC, the pieces' places.
+    constexpr int kSets = KSTEPS == 40 || (!VEC && KSTEPS == 24) ? 1 : 2;
+    constexpr int kAhead = kSets + 1;
     Stage sets[kSets];
     load_stage(sets[0], tile);
     if constexpr (kSets == 2) {
@@ -416,9 +428,7 @@ __global__ __launch_bounds__(kLinearWaves * 64) void linear_kernel(LinearArgs a)
         write_chunk(sets[0], 0, c);
     }
     write_flags(sets[0], 0);
-    if constexpr (VEC) {
-        load_stage(sets[0], tile + kSets * group_count);
-    }
+    load_stage(sets[0], tile + kSets * group_count);
     __syncthreads();
     for (;;) {
         step(0, tile, sets[kSets - 1], tile + kAhead * group_count);
@@ -459,7 +469,8 @@ constexpr int kStreamCols = 128;
 constexpr int kStreamK = 32;
 constexpr int kStreamThreads = 256;
 
-// VEC: whole 16-byte pieces of x, W and y.
+// VEC: whole 16-byte pieces of x, W and y; else pieces aligned to their
+// elements (rows here are longer than a piece).
 template <int XT, int YT, bool VEC>
 __global__ __launch_bounds__(kStreamThreads, VEC && XT == LSSO_HIP_BF16 ? 3 : 2) void linear_stream_kernel(LinearArgs a) {
     constexpr int KP = kStreamK + 8;                 // LDS row pitch (bf16): 16 rows' 16-byte reads cover all banks
@@ -496,7 +507,7 @@ __global__ __launch_bounds__(kStreamThreads, VEC && XT == LSSO_HIP_BF16 ? 3 : 2)
 
     struct Stage {
         u32x4 x[kXPieces];
-        f32x4 w[kWPieces];
+        u32x4 w[kWPieces];
     };
     const uint16_t* x = static_cast<const uint16_t*>(a.x) + m0 * a.x_stride;
     const float* w = a.weight + n0 * K;
@@ -522,41 +533,37 @@ __global__ __launch_bounds__(kStreamThreads, VEC && XT == LSSO_HIP_BF16 ? 3 : 2)
             }
 #pragma unroll
             for (int i = 0; i < kWPieces; ++i) {
-                stage.w[i] = __builtin_bit_cast(f32x4, buffer_load16(wb, wo + i * w_step));
+                stage.w[i] = buffer_load16(wb, wo + i * w_step);
             }
         } else {
+            // Rows past the matrices read their last ones: what they feed is
+            // not stored.
 #pragma unroll
             for (int i = 0; i < kXPieces; ++i) {
-                const int64_t r = x_row + kXRows * i;
-#pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    const int64_t k = k0 + x_k + 2 * p;
-                    const uint32_t lo = (m0 + r < M && k < K) ? x[r * a.x_stride + k] : 0u;
-                    const uint32_t hi = (m0 + r < M && k + 1 < K) ? x[r * a.x_stride + k + 1] : 0u;
-                    stage.x[i][p] = lo | (hi << 16);
-                }
+                const int64_t r = m0 + x_row + kXRows * i < M ? x_row + kXRows * i : M - 1 - m0;
+                stage.x[i] = load16_unaligned(x + r * a.x_stride + piece_start<8>(k0 + x_k, K));
             }
 #pragma unroll
             for (int i = 0; i < kWPieces; ++i) {
-                const int64_t r = w_row + kWRows * i;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int64_t k = k0 + w_k + e;
-                    stage.w[i][e] = (n0 + r < N && k < K) ? w[r * K + k] : 0.0f;
-                }
+                const int64_t r = n0 + w_row + kWRows * i < N ? w_row + kWRows * i : N - 1 - n0;
+                stage.w[i] = load16_unaligned(w + r * K + piece_start<4>(k0 + w_k, K));
             }
         }
     };
-    auto commit = [&](const Stage& stage, int buf) {
+    // The stage at column k0 into buffer `buf`.
+    auto commit = [&](const Stage& stage, int buf, int64_t k0) {
         uint16_t* s_x = s_t + 2 * buf * kOperand;
         uint16_t* s_w = s_x + kOperand;
 #pragma unroll
         for (int i = 0; i < kXPieces; ++i) {
-            *reinterpret_cast<u32x4*>(s_x + (x_row + kXRows * i) * KP + x_k) = to_bf16_piece<XT>(stage.x[i]);
+            const u32x4 piece = VEC ? stage.x[i] : align_piece16(stage.x[i], k0 + x_k, K);
+            *reinterpret_cast<u32x4*>(s_x + (x_row + kXRows * i) * KP + x_k) = to_bf16_piece<XT>(piece);
         }
 #pragma unroll
         for (int i = 0; i < kWPieces; ++i) {
-            const u32x2 packed = {pack_bf16(stage.w[i][0], stage.w[i][1]), pack_bf16(stage.w[i][2], stage.w[i][3])};
+            const u32x4 piece = VEC ? stage.w[i] : align_piece32(stage.w[i], k0 + w_k, K);
+            const f32x4 v = __builtin_bit_cast(f32x4, piece);
+            const u32x2 packed = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
             *reinterpret_cast<u32x2*>(s_w + (w_row + kWRows * i) * KP + w_k) = packed;
         }
     };
@@ -591,7 +598,7 @@ __global__ __launch_bounds__(kStreamThreads, VEC && XT == LSSO_HIP_BF16 ? 3 : 2)
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             if (kk == 1) {
-                commit(stage, buf ^ 1);
+                commit(stage, buf ^ 1, ahead - 2 * kStreamK);
                 load(stage, ahead);
             }
 #pragma unroll
@@ -628,7 +635,7 @@ __global__ __launch_bounds__(kStreamThreads, VEC && XT == LSSO_HIP_BF16 ? 3 : 2)
         const int64_t m = m0 + r;
         s_keep[r] = m < M && (a.row_mask == nullptr || a.row_mask[m] != 0);
     }
-    commit(even, 0);
+    commit(even, 0, 0);
     load(even, 2 * kStreamK);
     __syncthreads();
     // An odd last stage is followed by one of zeros: a second exit from the
@@ -679,16 +686,11 @@ __global__ __launch_bounds__(kStreamThreads, VEC && XT == LSSO_HIP_BF16 ? 3 : 2)
         const int64_t n = n0 + c8;
         if (m < M && n < N) {
             const u32x4 v = *reinterpret_cast<const u32x4*>(&s_y[mr * YP + c8]);
-            uint16_t* dst = static_cast<uint16_t*>(a.y) + m * N + n;
+            uint16_t* row = static_cast<uint16_t*>(a.y) + m * N;
             if (VEC) {
-                *reinterpret_cast<u32x4*>(dst) = v;
+                *reinterpret_cast<u32x4*>(row + n) = v;
             } else {
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    if (n + r < N) {
-                        dst[r] = static_cast<uint16_t>(v[r >> 1] >> (16 * (r & 1)));
-                    }
-                }
+                store_piece(row, n, N, v);
             }
         }
     }
@@ -718,7 +720,7 @@ template <int KSTEPS>
 static hipError_t launch_linear_k(const LinearArgs& a, int x_dtype, int y_dtype, dim3 grid,
                                   hipStream_t stream) {
     // The vector form's 32-bit offsets reach one tile's rows.
-    const bool vec = a.x_vector && a.y_vector && a.x_stride < (1 << 23) && a.out_features < (1 << 23);
+    const bool vec = a.vector && a.x_stride < (1 << 23) && a.out_features < (1 << 23);
     return vec ? launch_linear_kv<KSTEPS, true>(a, x_dtype, y_dtype, grid, stream)
                       : launch_linear_kv<KSTEPS, false>(a, x_dtype, y_dtype, grid, stream);
 }
@@ -732,7 +734,7 @@ hipError_t launch_linear(const LinearArgs& a, int k_steps, int x_dtype, int y_dt
         const dim3 grid(static_cast<unsigned>(rounds * kXcds * a.column_groups));
         const dim3 block(kStreamThreads);
         // The vector form's 32-bit offsets reach one tile's rows.
-        const bool vec = a.x_vector && a.w_vector && a.y_vector && a.x_stride < (1 << 23) && a.in_features < (1 << 22);
+        const bool vec = a.vector && a.x_stride < (1 << 23) && a.in_features < (1 << 22);
         const auto run = [&](auto kernel) { dispatch(kernel, grid, block, stream, a); };
         if (x_dtype == LSSO_HIP_F16) {
             if (y_dtype == LSSO_HIP_F16) {

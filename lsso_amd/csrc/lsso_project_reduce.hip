@@ -193,7 +193,7 @@ __global__ __launch_bounds__(pr_waves<KSTEPS>() * 64) void project_reduce_kernel
         u32x4 wreg[2][KSTEPS];
         // The packed tiles are not written before the first projection.
         static_assert(sizeof(s_y) >= kProj * kWeightScratch * sizeof(uint16_t), "the packed tiles hold the weight scratch");
-        load_weight_rows<2, KSTEPS>(
+        load_weight_rows<true, 2, KSTEPS>(
             wreg, make_buffer(a.weight, 4 * a.width * D),
             [&](int nb, int r) {
                 const int64_t column = packed_column(wave * 64 + nb * 32 + r);

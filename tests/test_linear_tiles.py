@@ -47,3 +47,37 @@ def test_linear_tiles_match_fp64(native, features, rows, pad, masked) -> None:
     start = min(33, rows - 1)
     again = native.linear(x[start:], weight, bias, y_dtype, row_mask=None if mask is None else mask[start:])
     assert torch.equal(again, y[start:])
+
+
+@pytest.mark.parametrize("in_features", (1, 3, 7, 8, 9, 15, 60, 100, 130, 250, 257, 300, 380, 391, 510, 636, 641, 700, 1001))
+@pytest.mark.parametrize(("rows", "out_features", "pad", "offset"), ((1, 1, 0, 0), (63, 7, 1, 0), (130, 9, 3, 1), (2049, 257, 0, 3),
+                                                                     (20000, 321, 2, 1), (77, 264, 8, 1), (300, 100, 0, 0)))
+def test_pieces_aligned_to_their_elements_match_whole_pieces(native, in_features, rows, out_features, pad, offset) -> None:
+    """Rows, strides, bases and outputs that are not whole 16-byte pieces give
+    the bits of the same operands padded with zeros to whole pieces.  What lies
+    between the rows and around the operands is NaN and must not be read into
+    the result."""
+
+    generator = torch.Generator(device="cuda").manual_seed(rows + in_features)
+    x_dtype, y_dtype = ((torch.float16, torch.bfloat16), (torch.bfloat16, torch.float16))[rows % 2]
+    stride = in_features + pad
+    values = torch.randn(rows, in_features, device="cuda", generator=generator).to(x_dtype)
+    storage = torch.full((offset + rows * stride + 16,), float("nan"), device="cuda", dtype=x_dtype)
+    x = storage[offset:offset + rows * stride].view(rows, stride)[:, :in_features]
+    x.copy_(values)
+    weights = torch.randn(out_features, in_features, device="cuda", generator=generator) / math.sqrt(in_features)
+    weight_storage = torch.full((offset + weights.numel() + 8,), float("nan"), device="cuda")
+    weight = weight_storage[offset:offset + weights.numel()].view(out_features, in_features)
+    weight.copy_(weights)
+    bias = torch.randn(out_features, device="cuda", generator=generator)
+    mask = torch.rand(rows, device="cuda", generator=generator) > 0.3 if rows % 3 == 0 else None
+
+    def whole(value: torch.Tensor, *sizes: int) -> torch.Tensor:
+        padded = torch.zeros(*(-(-size // 8) * 8 for size in sizes), device="cuda", dtype=value.dtype)
+        padded[tuple(slice(size) for size in sizes)] = value
+        return padded
+
+    expected = native.linear(whole(values, rows, in_features)[:rows], whole(weights, out_features, in_features),
+                             whole(bias, out_features), y_dtype, row_mask=mask)
+    y = native.linear(x, weight, bias, y_dtype, row_mask=mask)
+    assert torch.equal(y, expected[:, :out_features])
