@@ -152,6 +152,20 @@ __device__ __forceinline__ u32x4 align_piece16(const u32x4& raw, I k, I cols) {
     const u32x4 odd = {(v[0] >> 16) | (v[1] << 16), (v[1] >> 16) | (v[2] << 16), (v[2] >> 16) | (v[3] << 16), v[3] >> 16};
     return (early & 1) != 0 ? odd : v;
 }
+// 16-bit elements k .. k + 7 of a row of `cols` < 8, which holds no whole piece.
+__device__ __forceinline__ u32x4 load_short_piece(const uint16_t* row, int k, int cols) {
+    u32x4 out = {0u, 0u, 0u, 0u};
+    if (k == 0) {
+        for (int i = 0; i < cols; ++i) {
+            const uint32_t bits = static_cast<uint32_t>(row[i]) << (16 * (i & 1));
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                out[p] |= p == i / 2 ? bits : 0u;
+            }
+        }
+    }
+    return out;
+}
 // 32-bit elements k .. k + 3 from the access at piece_start<4>(k, cols).
 template <typename I>
 __device__ __forceinline__ u32x4 align_piece32(const u32x4& raw, I k, I cols) {

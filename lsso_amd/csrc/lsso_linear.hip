@@ -91,20 +91,7 @@ __device__ __forceinline__ u32x4 to_bf16_piece(const u32x4& raw) {
     return out;
 }
 
-// Rows of fewer than 8 elements, which hold no whole piece: element loads.
-__device__ __forceinline__ u32x4 load_short_piece(const uint16_t* row, int k0, int K) {
-    u32x4 out = {0u, 0u, 0u, 0u};
-    if (k0 == 0) {
-        for (int i = 0; i < K; ++i) {
-            const uint32_t bits = static_cast<uint32_t>(row[i]) << (16 * (i & 1));
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                out[p] |= p == i / 2 ? bits : 0u;
-            }
-        }
-    }
-    return out;
-}
+// Weight rows of fewer than 8 elements, element by element.
 template <int KSTEPS>
 __device__ __forceinline__ void load_short_weights(u32x4 (&wreg)[1][KSTEPS], const float* weight, int64_t N, int K,
                                                    int64_t n, int lane) {

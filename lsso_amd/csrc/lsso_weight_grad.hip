@@ -34,6 +34,12 @@
 // 131,072 x (640, 256) and 98 at 8,192 x (1,344, 768); this one 116, 73, 85
 // and 44 (4.6-5.7 TB/s of operands and partials at the first two).
 //
+// Operands that are not whole aligned 16-byte pieces run the same loop and
+// tiles on pieces aligned to their elements; element loads remain for rows of
+// fewer than 8 elements.  Former kernel, this one with element loads, with
+// these pieces (us): 65,537 x (521, 263) 276 / 295 / 74, 65,536 x (228, 100) 54 /
+// 70 / 26, 16,000 x (772, 772) 280 / 226 / 55.
+//
 // A split writes FP32 partials [split][n][k]; column_sum_kernel adds the
 // splits in a fixed order, so the result is deterministic.  The bias sums are
 // taken from the g pieces (in g's own precision, as the reference sums g) by
@@ -101,14 +107,19 @@ __device__ __forceinline__ u32x4 to_bf16_piece(const u32x4& raw) {
     }
 }
 
-// One operand's pieces of a stage: columns c .. c + 7 of rows row_lane +
-// kWgRowLanes * i, zero past the rows (end) and the columns.  VEC: raw-buffer
-// loads whose buffer ends with the split's last row (cols, the row stride and
-// the base multiples of 16 bytes); else element loads under conditions.
-template <typename Tile, bool VEC>
+// How the operands' pieces are loaded.
+constexpr int kWgWhole = 0;      // rows of whole aligned 16-byte pieces
+constexpr int kWgPieces = 1;     // pieces aligned to their elements
+constexpr int kWgElements = 2;   // element loads: rows of fewer than 8 elements
+
+// One operand's pieces of a stage as loaded: columns c .. c + 7 of rows row_lane
+// + kRowLanes * i, zero past the rows (end) and the columns except for
+// kWgPieces, whose pieces finish_piece moves to their columns and zeroes.
+// kWgWhole: raw-buffer loads whose buffer ends with the split's last row.
+template <typename Tile, int FORM>
 __device__ __forceinline__ void load_pieces(u32x4 (&out)[Tile::kPasses], const uint16_t* base, int64_t row,
                                             int64_t end, int64_t stride, int64_t c, int64_t cols, int row_lane) {
-    if constexpr (VEC) {
+    if constexpr (FORM == kWgWhole) {
         const BufferRsrc buffer = make_buffer(base + row * stride, (end - row) * stride * 2);
         const uint32_t offset = c < cols ? static_cast<uint32_t>((row_lane * stride + c) * 2) : kOutOfRange;
         const uint32_t step = c < cols ? static_cast<uint32_t>(Tile::kRowLanes * stride * 2) : 0u;
@@ -116,20 +127,31 @@ __device__ __forceinline__ void load_pieces(u32x4 (&out)[Tile::kPasses], const u
         for (int i = 0; i < Tile::kPasses; ++i) {
             out[i] = buffer_load16(buffer, offset + i * step);
         }
+    } else if constexpr (FORM == kWgPieces) {
+#pragma unroll
+        for (int i = 0; i < Tile::kPasses; ++i) {
+            const int64_t m = row + row_lane + Tile::kRowLanes * i;
+            out[i] = load16_unaligned(base + (m < end ? m : end - 1) * stride + piece_start<8>(c, cols));
+        }
     } else {
 #pragma unroll
         for (int i = 0; i < Tile::kPasses; ++i) {
             const int64_t m = row + row_lane + Tile::kRowLanes * i;
-            u32x4 v;
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
                 const uint32_t lo = (m < end && c + 2 * p < cols) ? base[m * stride + c + 2 * p] : 0u;
                 const uint32_t hi = (m < end && c + 2 * p + 1 < cols) ? base[m * stride + c + 2 * p + 1] : 0u;
-                v[p] = lo | (hi << 16);
+                out[i][p] = lo | (hi << 16);
             }
-            out[i] = v;
         }
     }
+}
+template <int FORM>
+__device__ __forceinline__ u32x4 finish_piece(const u32x4& raw, bool live, int64_t c, int64_t cols) {
+    if constexpr (FORM != kWgPieces) {
+        return raw;
+    }
+    return live ? align_piece16(raw, c, cols) : (u32x4){0u, 0u, 0u, 0u};
 }
 
 template <typename Tile>
@@ -144,7 +166,7 @@ struct WgStage {
 // MASK: a.row_mask is set; SUMS: a.bias_partials is set.  Both are template
 // choices so that a stage is one basic block: the conversions, LDS writes and
 // loads of the next stages are then scheduled between the MFMAs of this one.
-template <typename Tile, int GT, int XT, bool VEC, bool MASK, bool SUMS>
+template <typename Tile, int GT, int XT, int FORM, bool MASK, bool SUMS>
 __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs a) {
     // Row-major stage buffers: s_t[buf][operand][row * Tile::kPitch + column].
     __shared__ __attribute__((aligned(16))) uint16_t s_t[2][2][kWgRows * Tile::kPitch];
@@ -191,8 +213,8 @@ __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs 
         colsum[e] = 0.0f;
     }
     auto load = [&](WgStage<Tile>& stage, int64_t row) {
-        load_pieces<Tile, VEC>(stage.g, g, row, r1, a.g_stride, n0 + 8 * piece, N, row_lane);
-        load_pieces<Tile, VEC>(stage.x, x, row, r1, a.x_stride, k0 + 8 * piece, K, row_lane);
+        load_pieces<Tile, FORM>(stage.g, g, row, r1, a.g_stride, n0 + 8 * piece, N, row_lane);
+        load_pieces<Tile, FORM>(stage.x, x, row, r1, a.x_stride, k0 + 8 * piece, K, row_lane);
         if constexpr (MASK) {
             const BufferRsrc mask = make_buffer(a.row_mask + row, r1 - row);
 #pragma unroll
@@ -201,9 +223,12 @@ __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs 
             }
         }
     };
-    auto commit = [&](WgStage<Tile>& stage, int buf) {
+    auto commit = [&](WgStage<Tile>& stage, int buf, int64_t row) {
 #pragma unroll
         for (int i = 0; i < Tile::kPasses; ++i) {
+            const bool live = row + row_lane + Tile::kRowLanes * i < r1;
+            stage.g[i] = finish_piece<FORM>(stage.g[i], live, n0 + 8 * piece, N);
+            stage.x[i] = finish_piece<FORM>(stage.x[i], live, k0 + 8 * piece, K);
             if constexpr (MASK) {
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
@@ -274,7 +299,7 @@ __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs 
 #pragma unroll
         for (int kk = 0; kk < kWgSteps; ++kk) {
             if (kk == kWgSteps - 1) {
-                commit(stage, buf ^ 1);
+                commit(stage, buf ^ 1, next_row - 2 * kWgRows);
                 load(stage, next_row);
             }
 #pragma unroll
@@ -312,7 +337,7 @@ __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs 
     WgStage<Tile> odd;
     load(even, r0);
     load(odd, r0 + kWgRows);
-    commit(even, 0);
+    commit(even, 0, r0);
     load(even, r0 + 2 * kWgRows);
     __syncthreads();
     for (int64_t row = r0; row < r1; row += 2 * kWgRows) {
@@ -371,7 +396,8 @@ __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs 
 // 39 / 37, 8,192 x (1,344, 768) 48 / 45, 2,048 x (512, 256) 24 / 19: the line
 // lies near 2^33 multiply-adds.
 bool weight_grad_large(int64_t rows, int64_t in_features, int64_t out_features) {
-    return static_cast<double>(rows) * in_features * out_features >= 8.5e9;
+    return in_features >= 8 && out_features >= 8 &&   // whole pieces
+           static_cast<double>(rows) * in_features * out_features >= 8.5e9;
 }
 
 // Row splits.  More splits put more CUs on the product (its time falls as 1 /
@@ -407,26 +433,28 @@ void plan_weight_grad(int64_t rows, int64_t in_features, int64_t out_features, i
     *splits = rows == 0 ? 0 : (rows + *rows_per_split - 1) / *rows_per_split;
 }
 
-template <typename Tile, int GT, int XT, bool VEC>
+template <typename Tile, int GT, int XT, int FORM>
 static void launch_wg(const WeightGradArgs& a, dim3 grid, hipStream_t stream) {
     const auto run = [&](auto kernel) { kernel<<<grid, kWgThreads, 0, stream>>>(a); };
     if (a.row_mask != nullptr) {
-        a.bias_partials != nullptr ? run(weight_grad_kernel<Tile, GT, XT, VEC, true, true>)
-                                   : run(weight_grad_kernel<Tile, GT, XT, VEC, true, false>);
+        a.bias_partials != nullptr ? run(weight_grad_kernel<Tile, GT, XT, FORM, true, true>)
+                                   : run(weight_grad_kernel<Tile, GT, XT, FORM, true, false>);
     } else {
-        a.bias_partials != nullptr ? run(weight_grad_kernel<Tile, GT, XT, VEC, false, true>)
-                                   : run(weight_grad_kernel<Tile, GT, XT, VEC, false, false>);
+        a.bias_partials != nullptr ? run(weight_grad_kernel<Tile, GT, XT, FORM, false, true>)
+                                   : run(weight_grad_kernel<Tile, GT, XT, FORM, false, false>);
     }
 }
 
 template <int GT, int XT>
 static void launch_wg(const WeightGradArgs& a, dim3 grid, hipStream_t stream) {
-    if (!a.vec) {
-        launch_wg<WgSmall, GT, XT, false>(a, grid, stream);
-    } else if (a.large) {
-        launch_wg<WgLarge, GT, XT, true>(a, grid, stream);
+    if (a.vec) {
+        a.large ? launch_wg<WgLarge, GT, XT, kWgWhole>(a, grid, stream)
+                : launch_wg<WgSmall, GT, XT, kWgWhole>(a, grid, stream);
+    } else if (a.in_features >= 8 && a.out_features >= 8) {
+        a.large ? launch_wg<WgLarge, GT, XT, kWgPieces>(a, grid, stream)
+                : launch_wg<WgSmall, GT, XT, kWgPieces>(a, grid, stream);
     } else {
-        launch_wg<WgSmall, GT, XT, true>(a, grid, stream);
+        launch_wg<WgSmall, GT, XT, kWgElements>(a, grid, stream);   // never large
     }
 }
 
@@ -435,11 +463,9 @@ hipError_t launch_weight_grad(const WeightGradArgs& args, int g_dtype, int x_dty
         return hipSuccess;
     }
     WeightGradArgs a = args;
-    // The raw buffers' 32-bit offsets reach one stage's rows.  Element loads
-    // (rows that are not whole 16-byte pieces) take the small tile, whose
-    // registers have room for them; the splits are the plan's either way.
+    // The raw buffers' 32-bit offsets reach one stage's rows.
     a.vec = a.vec && a.g_stride < (1 << 24) && a.x_stride < (1 << 24);
-    a.large = a.vec && weight_grad_large(a.rows, a.in_features, a.out_features);
+    a.large = weight_grad_large(a.rows, a.in_features, a.out_features);
     const int64_t edge = a.large ? WgLarge::kEdge : WgSmall::kEdge;
     a.tiles_n = (a.out_features + edge - 1) / edge;
     a.tiles_k = (a.in_features + edge - 1) / edge;
