@@ -31,7 +31,7 @@
 // The former kernel (128 x 128 tiles of four waves, 8 x 8 blocks transposed in
 // registers with byte permutes, one stage in flight) took, with the column
 // sums, 181 us at 262,144 x (512, 256), 96 at 262,144 x (256, 256), 112 at
-// 131,072 x (640, 256) and 98 at 8,192 x (1,344, 768); this one 116, 73, 85
+// 131,072 x (640, 256) and 98 at 8,192 x (1,344, 768); this one 116, 66, 85
 // and 44 (4.6-5.7 TB/s of operands and partials at the first two).
 //
 // Operands that are not whole aligned 16-byte pieces run the same loop and
@@ -387,17 +387,33 @@ __global__ __launch_bounds__(kWgThreads) void weight_grad_kernel(WeightGradArgs 
     }
 }
 
+template <typename Tile>
+static int64_t wg_tiles(int64_t in_features, int64_t out_features) {
+    return ((out_features + Tile::kEdge - 1) / Tile::kEdge) * ((in_features + Tile::kEdge - 1) / Tile::kEdge);
+}
+
 // The output tile.  The large tile moves half the operand bytes between L2 and
 // the CUs per product but writes four times the partials per workgroup and
-// leaves short row ranges with fewer, longer chains.  Measured with the column
-// sums, large against small (us): 131,072 rows x (640, 256) 79 / 80, x (768,
-// 384) 127 / 144, x (768, 768) 191 / 298, 65,536 x (512, 256) 45 / 46, 16,000 x
-// (768, 768) 46 / 53; but 65,536 x (256, 256) 37 / 31, 16,000 x (768, 384)
-// 39 / 37, 8,192 x (1,344, 768) 48 / 45, 2,048 x (512, 256) 24 / 19: the line
-// lies near 2^33 multiply-adds.
-bool weight_grad_large(int64_t rows, int64_t in_features, int64_t out_features) {
-    return in_features >= 8 && out_features >= 8 &&   // whole pieces
-           static_cast<double>(rows) * in_features * out_features >= 8.5e9;
+// leaves short row ranges with fewer, longer chains, so it takes a long
+// product; a shorter one where the small tiles leave an XCD's workgroups idle
+// (36 tiles at 768 x 768: one split of 64 slots, so little over half) or are too
+// many to be dealt to the XCDs.  Measured with the column sums and without a
+// bias, large over small tile, at 5 / 8.5 / 12 / 20 / 50e9 multiply-adds:
+// outputs of 512 x 512 1.17 / 1.15 / 1.06 / 0.95 / 0.83, 1,344 x 768 1.11 / 1.00
+// / 0.96 / 0.88 / 0.78, 768 x 768 1.05 / 0.90 / 0.83 / 0.71 / 0.61, 640 x 256
+// 1.17 / 1.12 / 1.05 / 0.99 / 0.94.  A single tile per split (256 x 256: 1.19 /
+// 1.24 / 1.13 / 1.17 / 1.01) and outputs that half fill large tiles (384 x 384
+// 1.18 / 1.17 / 1.16 / 1.16 / 1.06, 228 x 100 1.20 throughout, 64 x 64 about 1.9)
+// never gain from it.
+static bool weight_grad_large(int64_t rows, int64_t in_features, int64_t out_features) {
+    const int64_t large = wg_tiles<WgLarge>(in_features, out_features);
+    const int64_t small = wg_tiles<WgSmall>(in_features, out_features);
+    const int64_t slots = WgSmall::kSlotsPerXcd;
+    if (large < 2 || 8 * large >= 3 * small) {   // padded at least 1.5 times as far
+        return false;
+    }
+    const double share = small <= slots ? static_cast<double>(slots / small * small) / slots : 0.75;
+    return static_cast<double>(rows) * in_features * out_features >= 1.2e10 * share;
 }
 
 // Row splits.  More splits put more CUs on the product (its time falls as 1 /
@@ -414,9 +430,9 @@ bool weight_grad_large(int64_t rows, int64_t in_features, int64_t out_features) 
 void plan_weight_grad(int64_t rows, int64_t in_features, int64_t out_features, int64_t* splits,
                       int64_t* rows_per_split) {
     const bool large = weight_grad_large(rows, in_features, out_features);
-    const int64_t edge = large ? WgLarge::kEdge : WgSmall::kEdge;
     const int64_t slots = large ? WgLarge::kSlotsPerXcd : WgSmall::kSlotsPerXcd;
-    const int64_t tiles = ((out_features + edge - 1) / edge) * ((in_features + edge - 1) / edge);
+    const int64_t tiles = large ? wg_tiles<WgLarge>(in_features, out_features)
+                                : wg_tiles<WgSmall>(in_features, out_features);
     const int64_t stages = (rows + kWgRows - 1) / kWgRows;
     int64_t want;
     if (tiles <= slots) {

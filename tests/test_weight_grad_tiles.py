@@ -1,5 +1,5 @@
 """The weight-gradient kernel at the edges of its tiles and plans (GPU): both
-output tiles (256 x 256 from about 2^33 multiply-adds on, else 128 x 128),
+output tiles (256 x 256 for long products that fill such tiles, else 128 x 128),
 column remainders, a last stage of one row, rows that are not whole 16-byte
 pieces or hold none, splits that are not dealt to the XCDs, masks and the
 variants without bias sums, against FP64 of the same BF16 operands.
