@@ -401,6 +401,11 @@ __global__ __launch_bounds__(kMixThreads) void mix_project_kernel(MixProjectArgs
             const int sub = step / (HPW / kTogether);
             const int u0 = step % (HPW / kTogether) * kTogether;
             if constexpr (!kReadFirst) {
+                // Slots one by one: nothing to interleave, so a repeated head
+                // is skipped (wave-uniform).
+                if (u0 > 0 && j + kMixApplyWaves * u0 >= H) {
+                    continue;
+                }
 #pragma unroll
                 for (int u = 0; u < kTogether; ++u) {
                     in[u0 + u][sub] = read(u0 + u, sub);

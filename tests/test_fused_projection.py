@@ -62,6 +62,32 @@ def test_fused_projection_is_bitwise_the_two_step_path(native, batch, rank, head
     assert torch.equal(fused, expected)
 
 
+@pytest.mark.parametrize("rank", (16, 32, 48, 64))
+@pytest.mark.parametrize("masked", (False, True))
+@pytest.mark.parametrize("length", (33, 333))
+def test_five_heads_of_three_feature_blocks(native, rank, masked, length):
+    """More than four heads of more than two feature blocks fill the apply
+    waves' registers, so their two head slots take turns; five heads leave
+    three waves a second slot without a head, 48 features a fourth block
+    without columns."""
+
+    batch, heads, head_dim = 3, 5, 48
+    projected, base, drive, eta_raw, weight, bias = _inputs(batch, rank, heads, head_dim, length, seed=500 + rank)
+    mask = counts = None
+    if masked:
+        lengths = torch.tensor([length, length // 2, 1])
+        mask = (torch.arange(length)[None, :] < lengths[:, None]).cuda()
+        projected = torch.where(mask[:, :, None], projected, torch.zeros_like(projected))
+        counts = lengths.float().cuda()
+    with torch.no_grad():
+        assert native.mix_project_supported(projected, base, drive, eta_raw)
+        fused = native.mix_project(projected, base, drive, eta_raw, None, counts, weight, bias, torch.float16,
+                                   row_mask=mask)
+        expected = _two_step(native, projected, base, drive, eta_raw, None, counts, weight, bias, torch.float16, mask)
+    assert torch.isfinite(fused).all()
+    assert torch.equal(fused, expected)
+
+
 def test_fused_projection_masked_per_sample_positions_and_no_bias(native):
     batch, rank, heads, head_dim, length = 3, 32, 8, 32, 300
     projected, base, drive, eta_raw, weight, _bias = _inputs(batch, rank, heads, head_dim, length, seed=77)

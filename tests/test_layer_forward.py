@@ -278,6 +278,10 @@ def test_project_mix_gradients_equal_the_two_call_path(native):
         (2, 32, 8, 32, 1000, True),
         (1, 64, 6, 64, 300, True),    # C4 geometry: D = 384, apply and projection separate
         (3, 16, 8, 16, 65, False),
+        (2, 16, 5, 48, 97, False),    # five heads of 48: head slots in turn, mixed stored as well
+        (2, 32, 5, 48, 333, True),
+        (1, 48, 5, 48, 65, True),
+        (2, 64, 5, 48, 130, False),
     ],
 )
 def test_layer_train_is_bitwise_the_three_call_path(native, batch, rank, heads, head_dim, length, masked):
