@@ -335,6 +335,35 @@ int run_solve(const MixerPlan& plan, const MixerBuffers& buf, const float* core_
     return error == hipSuccess ? LSSO_HIP_OK : hip_failure(error, "solve_kernel launch");
 }
 
+int compute_units(int* units) {
+    int device = 0;
+    hipError_t error = hipGetDevice(&device);
+    if (error != hipSuccess) {
+        return hip_failure(error, "hipGetDevice");
+    }
+    error = hipDeviceGetAttribute(units, hipDeviceAttributeMultiprocessorCount, device);
+    if (error != hipSuccess) {
+        return hip_failure(error, "hipDeviceGetAttribute");
+    }
+    return LSSO_HIP_OK;
+}
+
+// Heads per workgroup of the staged reduce, 0 where it does not apply.
+int staged_reduce_heads(const MixerPlan& plan, bool vec, int64_t* heads) {
+    *heads = 0;
+    if (plan.cpw != 1) {
+        return LSSO_HIP_OK;
+    }
+    int units = 0;
+    const int status = compute_units(&units);
+    if (status == LSSO_HIP_OK) {
+        *heads = lsso_hip::reduce_staged_group_heads(plan.rank, plan.heads, plan.head_dim, plan.column_groups,
+                                                     plan.batch * plan.reduce_chunks, units,
+                                                     vec && plan.head_dim % 8 == 0);
+    }
+    return status;
+}
+
 // Phase table, L-reductions and the compact solve: everything up to the
 // apply operand records.
 int run_reduce(const MixerPlan& plan, const MixerBuffers& buf, const void* projected,
@@ -378,11 +407,10 @@ int run_reduce(const MixerPlan& plan, const MixerBuffers& buf, const void* proje
     reduce.column_groups = plan.column_groups;
     reduce.partial_stride = plan.partial_stride;
     reduce.total_waves = plan.batch * plan.heads * plan.reduce_chunks * plan.column_groups;
-    reduce.group_heads = plan.cpw == 1 ? lsso_hip::reduce_staged_group_heads(plan.rank, plan.heads, plan.head_dim,
-                                                                              plan.column_groups,
-                                                                              plan.batch * plan.reduce_chunks,
-                                                                              vec && plan.head_dim % 8 == 0)
-                                       : 0;
+    const int status = staged_reduce_heads(plan, vec, &reduce.group_heads);
+    if (status != LSSO_HIP_OK) {
+        return status;
+    }
     const hipError_t error =
         lsso_hip::launch_reduce(static_cast<int>(plan.rank), reduce, plan.cpw, vec, stream);
     return error == hipSuccess ? LSSO_HIP_OK : hip_failure(error, "reduce_kernel launch");
@@ -422,19 +450,6 @@ int run_apply(const MixerPlan& plan, const MixerBuffers& buf, const void* projec
     const hipError_t error =
         lsso_hip::launch_apply(static_cast<int>(plan.rank), apply, plan.nfbw, vec, stream);
     return error == hipSuccess ? LSSO_HIP_OK : hip_failure(error, "apply_kernel launch");
-}
-
-int compute_units(int* units) {
-    int device = 0;
-    hipError_t error = hipGetDevice(&device);
-    if (error != hipSuccess) {
-        return hip_failure(error, "hipGetDevice");
-    }
-    error = hipDeviceGetAttribute(units, hipDeviceAttributeMultiprocessorCount, device);
-    if (error != hipSuccess) {
-        return hip_failure(error, "hipDeviceGetAttribute");
-    }
-    return LSSO_HIP_OK;
 }
 
 // Fused apply + output projection into y (shape inside mix_project_supported).
@@ -917,11 +932,10 @@ int lsso_hip_mixer_backward_ex(const lsso_hip_mixer_shape* shape, const void* gr
     reduce.column_groups = plan.column_groups;
     reduce.partial_stride = plan.partial_stride;
     reduce.total_waves = plan.batch * plan.heads * plan.reduce_chunks * plan.column_groups;
-    reduce.group_heads = plan.cpw == 1 ? lsso_hip::reduce_staged_group_heads(plan.rank, plan.heads, plan.head_dim,
-                                                                              plan.column_groups,
-                                                                              plan.batch * plan.reduce_chunks,
-                                                                              vec && plan.head_dim % 8 == 0)
-                                       : 0;
+    status = staged_reduce_heads(plan, vec, &reduce.group_heads);
+    if (status != LSSO_HIP_OK) {
+        return status;
+    }
     error = lsso_hip::launch_reduce(static_cast<int>(plan.rank), reduce, plan.cpw, vec, stream);
     if (error != hipSuccess) {
         return hip_failure(error, "reduce_kernel launch (backward)");

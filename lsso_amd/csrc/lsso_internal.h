@@ -283,10 +283,10 @@ hipError_t launch_phase(const PhaseArgs& a, hipStream_t stream);
 hipError_t launch_geometry(const GeometryArgs& a, int position_type, hipStream_t stream);
 hipError_t launch_reduce(int rank, const ReduceArgs& a, int cpw, bool vec, hipStream_t stream);
 // Heads per workgroup of the staged reduce for this geometry (items: samples x
-// chunks), or 0 where it
-// does not apply (the one-wave-per-item reduce_kernel runs instead).
+// chunks) on a device of compute_units, or 0 where it does not apply (the
+// one-wave-per-item reduce_kernel runs instead).
 int64_t reduce_staged_group_heads(int64_t rank, int64_t heads, int64_t head_dim, int64_t column_groups,
-                                  int64_t items, bool vec);
+                                  int64_t items, int64_t compute_units, bool vec);
 hipError_t launch_solve(int rank, const SolveArgs& a, int64_t systems, hipStream_t stream);
 hipError_t launch_apply(int rank, const ApplyArgs& a, int nfbw, bool vec, hipStream_t stream);
 // Heads per workgroup of the staged apply for this geometry, or 0 where it

@@ -190,7 +190,6 @@ __global__ __launch_bounds__(256, 2) void reduce_kernel(ReduceArgs a) {
 // k + 1 are in flight during step k's reductions.
 constexpr int kStagedWaves = 8;              // at most, per workgroup
 constexpr int kStagedCols = 512;             // group columns (relation + content) per row, at most
-constexpr int64_t kStagedComputeUnits = 256;
 constexpr int kStagedRelPieces = 3;          // 16-byte pieces per thread and step, at most
 constexpr int kStagedConPieces = 2;
 constexpr int kStagedPhasePieces = 1;
@@ -404,7 +403,7 @@ __global__ __launch_bounds__(kStagedWaves * 64) void reduce_staged_kernel(Reduce
 }
 
 int64_t reduce_staged_group_heads(int64_t rank, int64_t heads, int64_t head_dim, int64_t column_groups,
-                                  int64_t items, bool vec) {
+                                  int64_t items, int64_t compute_units, bool vec) {
     // Rows read as 16-byte pieces: relation and content runs whole pieces.
     if (!vec || rank < 48 || head_dim % 8 != 0 || column_groups < 1 || column_groups > kStagedWaves) {
         return 0;
@@ -430,7 +429,7 @@ int64_t reduce_staged_group_heads(int64_t rank, int64_t heads, int64_t head_dim,
     // the heads over more workgroups as long as each finds a CU of its own (2
     // x 4,096 tokens, 12 heads of 48 + 64: 68 us in 24 workgroups, 50 in 48).
     while (group > 1 && fits((group + 1) / 2) &&
-           items * ((heads + (group + 1) / 2 - 1) / ((group + 1) / 2)) <= kStagedComputeUnits) {
+           items * ((heads + (group + 1) / 2 - 1) / ((group + 1) / 2)) <= compute_units) {
         group = (group + 1) / 2;
     }
     return group;
