@@ -502,9 +502,7 @@ def center_positions(
     takes fewer than 2^32 threads), and ids of another type, shape or device,
     which the tensor path converts or rejects."""
 
-    if device.type != "cuda":
-        raise RuntimeError("device must be a CUDA (ROCm) device")
-    if device.index is None:
+    if device.index is None and device.type == "cuda":
         device = torch.device("cuda", torch.cuda.current_device())
     if valid_mask is not None:
         if valid_mask.dtype != torch.bool or valid_mask.shape != (batch, length):
@@ -517,6 +515,8 @@ def center_positions(
         kind = _ID_TYPES.get(position_ids.dtype, 0)
         if kind == 0 or position_ids.device != device:
             return None
+        if not position_ids.is_cuda:
+            raise RuntimeError("position_ids must be a CUDA (ROCm device) tensor")
         if position_ids.dim() == 1 and position_ids.shape[0] == length:
             token_stride = position_ids.stride(0)
             rows = 1 if valid_mask is None else batch
