@@ -1483,9 +1483,10 @@ namespace {
 // (one reduction wave idle) and each head's reduction, with two pair slots per
 // lane, sets the tile's pace.  Measured on one MI355X with the spill-free
 // rank-48/64 kernels: at B = 64, N = 2048, H = 8, r = 48, d = 32 (the
-// training forward) 146.5 us fused against 75.3 + 53.5 us for the projection
-// and the staged reduce; at B = 32, N = 4096, H = 6, r = 64, D = 384 the stage
-// took 284.7 us fused against 169.6 us.
+// training forward) 152.3 us fused against 66 + 58 us for the projection and
+// the staged reduce; at B = 32, N = 4096, H = 6, r = 64, D = 384 the stage
+// took 282.7 us fused against 160 us.  At rank 32 (B = 64, N = 4096, H = 8, d =
+// 32) it takes 109 us fused against 151.
 //
 // LSSO_HIP_FUSED_PROJECTION overrides the rule for A/B measurements and
 // tests: "1" fuses at every rank the fused kernel supports, "0" never fuses.

@@ -927,7 +927,7 @@ __device__ __forceinline__ void invert32_by_blocks(float* m, float* scratch, int
 
 template <int R>
 // Two workgroups per CU (512 systems on 256 CUs in one round): the register
-// budget is held to 256 per lane, which costs rank 48 a few spills.
+// budget is held to 256 per lane.
 __global__ __launch_bounds__(kSolveThreads, 2) void solve_kernel(SolveArgs a) {
     using SL = SolveLayout<R>;
     using AL = ApplyLayout<R>;
