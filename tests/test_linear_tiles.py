@@ -81,3 +81,19 @@ def test_pieces_aligned_to_their_elements_match_whole_pieces(native, in_features
                              whole(bias, out_features), y_dtype, row_mask=mask)
     y = native.linear(x, weight, bias, y_dtype, row_mask=mask)
     assert torch.equal(y, expected[:, :out_features])
+
+
+@pytest.mark.parametrize(("rows", "in_features", "out_features", "stride"), (
+    (70, 64, 72, (1 << 23) + 8),            # a tile's rows past 32-bit offsets, resident weights
+    (130, 648, 136, (1 << 23) + 8),         # the same, K-streaming
+    (9, (1 << 22) + 8, 8, (1 << 22) + 8),   # weight rows past them
+))
+def test_strides_past_32_bit_tile_offsets(native, rows, in_features, out_features, stride) -> None:
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.empty(rows, stride, device="cuda", dtype=torch.bfloat16)[:, :in_features]
+    x.copy_(torch.randn(rows, in_features, device="cuda", generator=generator))
+    weight = torch.randn(out_features, in_features, device="cuda", generator=generator) / math.sqrt(in_features)
+    y = native.linear(x, weight, None, torch.bfloat16)
+    expected = x.double() @ weight.bfloat16().double().t().contiguous()
+    error = float((y.double() - expected).norm() / expected.norm())
+    assert error <= HALF_ULP[torch.bfloat16] + 2.0 ** -24 * math.sqrt(in_features)

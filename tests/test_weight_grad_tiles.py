@@ -106,6 +106,19 @@ def test_pieces_aligned_to_their_elements_match_whole_pieces(
     assert torch.all((grad_bias.double() - expected_bias[:out_features].double()).abs() <= limit * scale)
 
 
+def test_strides_past_32_bit_stage_offsets(native) -> None:
+    generator = torch.Generator(device="cuda").manual_seed(5)
+    rows, stride = 70, (1 << 24) + 8
+    x = torch.empty(rows, stride, device="cuda", dtype=torch.bfloat16)[:, :72]
+    x.copy_(torch.randn(rows, 72, device="cuda", generator=generator))
+    g = torch.randn(rows, 136, device="cuda", generator=generator).bfloat16()
+    grad_weight, grad_bias = native._weight_gradient(g, x, None, True)
+    expected = g.double().t().contiguous() @ x.double()
+    limit = 2.0 ** -24 * math.sqrt(rows)
+    assert float((grad_weight.double() - expected).norm() / expected.norm()) <= limit
+    assert torch.all((grad_bias.double() - g.double().sum(0)).abs() <= limit * g.double().abs().sum(0))
+
+
 @pytest.mark.parametrize(("splits", "cols"), ((1, 5), (2, 4), (7, 132), (64, 8), (600, 1024), (33, 1003)))
 def test_column_sums_of_few_and_many_splits(native, splits, cols) -> None:
     """The split sums' lane plans (one lane per piece to 32, whole and odd
